@@ -10,13 +10,15 @@
 // rescaled once; v_exp_f32 / v_log_f32 / v_rcp_f32 evaluate it (relative error
 // a few 1e-7, inside the 1e-5 parity bar).
 //
-// Work decomposition (rows of up to 64 vector chunks, C <= 256):
+// Work decomposition.  Rows of more than two 16-byte chunks are cut into slabs
+// of up to 8 chunks, one wave per (segment, slab): see the slab kernels.  Rows
+// of one or two aligned chunks (C = 4, 8) and of C <= 3 run lane groups:
 //   * LC lanes cover one edge row (LC = next power of two >= C / V).
-//   * Short segments (degree <= CAP) belong to G-lane groups (G = 32, or 64
-//     when LC = 64): the group issues all of its segment's loads at once into
-//     RMAX register tiles of PG = G / LC rows, so one memory round trip
-//     brings the whole segment in; max, sum and normalisation run on the
-//     registers and alpha is written once.
+//   * Short segments (degree <= CAP) belong to 32-lane groups: the group
+//     issues all of its segment's loads at once into RMAX register tiles of
+//     PG = 32 / LC rows, so one memory round trip brings the whole segment in;
+//     max, sum and normalisation run on the registers and alpha is written
+//     once.
 //   * Long segments (degree > CAP) belong to a whole 256-thread workgroup:
 //     up to RMAXB tiles of PB = 256 / LC rows are staged in registers (one
 //     read); longer segments stream twice (an online max/sum pass, then the
@@ -28,9 +30,9 @@
 //     segments and skip the long ones, so no workgroup runs a long segment
 //     after its short ones.  This is the degree-binned schedule.  Without a
 //     plan, a workgroup handles its own long segments after its short ones.
+//     The slab kernels need no plan (theirs is empty).
 // All reductions are DPP / ds_swizzle / ds_bpermute butterflies or fixed LDS
 // orders: results are reproducible bit for bit from run to run.
-// Rows wider than 64 chunks use a channel-major kernel (one lane per chunk).
 #include "common.h"
 
 namespace dpa4k {
@@ -143,8 +145,8 @@ __device__ __forceinline__ float span_max(float v) {
   return v;
 }
 
-template <int FROM, int TO>
-__device__ __forceinline__ float span_sum(float v) {
+template <int FROM, int TO, typename T>
+__device__ __forceinline__ T span_sum(T v) {
   if constexpr (FROM <= 1 && TO > 1) v += xor_lane<1>(v);
   if constexpr (FROM <= 2 && TO > 2) v += xor_lane<2>(v);
   if constexpr (FROM <= 4 && TO > 4) v += xor_lane<4>(v);
@@ -961,79 +963,492 @@ __global__ __launch_bounds__(kBlock) void softmax_backward_kernel(BackwardArgs a
 }
 
 // ---------------------------------------------------------------------------
-// rows wider than 64 chunks: one wave per segment, lane per channel
+// rows of more than two chunks: a wave per (segment, slab of columns)
 // ---------------------------------------------------------------------------
+//
+// Columns are independent in the forward, and in the backward until the row
+// sums of grad_env.  So a row is cut into slabs of LS chunks (LS = 2, 4 or 8:
+// 8 chunks are one 128-byte line), and one wave takes one slab of one
+// segment: 64 / LS rows per load, up to R loads, all issued before any
+// arithmetic.  A segment of up to CAP = R * 64 / LS rows is then read once,
+// whatever its width, where a workgroup that stages whole rows in registers
+// holds 16 rows at C = 256 and reads everything longer twice.  R follows the
+// graph's mean degree (slab_rows).  Longer segments are streamed by the same
+// wave: an online max/sum pass, then the write pass.  The sums over the rows
+// are kept in 64 bits: they are few instructions beside the row streams, and
+// alpha and the gradients come out closer to the exact values for it.
+//
+// The forward has no barrier.  In the backward, up to 8 waves of a workgroup
+// take the slabs of one segment and leave each row's partial sum in LDS; after
+// one barrier thread t adds those of row t in slab order and writes grad_env.
+// Rows of more than 8 slabs repeat this, grad_env keeping the raw sum until
+// the last round (thread t reads back only what it wrote itself).
+//
+// Any C >= 4 and any 4-byte alignment: the row's last chunk starts at column
+// C - 4, so it repeats up to three columns of its neighbour, which compute and
+// store the same bits in both lanes and are left out of the row sums (`skip`).
+//
+// Bound by the row streams: C = 256 over 741k edges of 8,192 segments takes
+// 274 us forward (5.6 TB/s) and 380 us backward (6.0), where staging whole rows
+// took 426 and 700 us; C = 128, 991k edges 419 against 707 us for both; C = 64,
+// 182k edges 49 against 61 us; C = 16, 1.48M edges 88 against 109 us.  Scattered
+// rows (through an order): C = 128 545 against 819 us, C = 16 unchanged
+// (208 us, bound by the 64-byte gathers).  A streamed round takes its maximum
+// first: an online update per value kept a wave of 512 rows busy for 53 us,
+// this form for 25 us.  Errors against 64 bits (C = 16 to 256, degree 70 with
+// hubs): alpha 1.1e-7 -> 7e-8, grad_logit 2.8-3.3e-7 -> 1.1e-7.
 
-template <bool kOrdered>
-__global__ __launch_bounds__(kBlock) void softmax_forward_wide_kernel(ForwardArgs a) {
-  const int64_t segment = block_index() * kWaves + (threadIdx.x >> 6);
-  if (segment >= a.n_nodes) return;
-  const int lane = threadIdx.x & 63;
-  const int64_t channels = a.channels;
-  int64_t begin, end;
-  segment_bounds(a.offsets, segment, a.n_edges, begin, end);
-  for (int64_t c = lane; c < channels; c += 64) {
-    float peak = -INFINITY, sum = 0.0f, carry = 0.0f;
-    for (int64_t slot = begin; slot < end; ++slot) {
-      const int64_t e = edge_of<kOrdered>(a.order, slot, a.n_edges);
-      if (e >= 0) online_add(peak, sum, carry, log2_weight(a.logit[e * channels + c], a.env[e]));
+constexpr int kSlabWaves = 8;  // most slabs of one segment side by side in a backward workgroup
+
+// A float4 at 4-byte alignment (one dwordx4 access).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ fvec<4> load_chunk(const float* __restrict__ p) {
+  const f32x4u raw = *reinterpret_cast<const f32x4u*>(p);
+  return fvec<4>{{raw.x, raw.y, raw.z, raw.w}};
+}
+__device__ __forceinline__ fvec<4> load_chunk_stream(const float* __restrict__ p) {
+  const f32x4u raw = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(p));
+  return fvec<4>{{raw.x, raw.y, raw.z, raw.w}};
+}
+__device__ __forceinline__ void store_chunk(float* __restrict__ p, const fvec<4>& value) {
+  const f32x4u raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
+  *reinterpret_cast<f32x4u*>(p) = raw;
+}
+__device__ __forceinline__ void store_chunk_stream(float* __restrict__ p, const fvec<4>& value) {
+  const f32x4u raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
+  __builtin_nontemporal_store(raw, reinterpret_cast<f32x4u*>(p));
+}
+
+// How a wave finds its rows: natural order through buffer views, or edge ids
+// (from `order`, or the slot itself) and 64-bit addresses, the ids kept in 32
+// bits where they fit.  Rows are read and written once and go non-temporally,
+// except (SharedViews) where slabs of 128 bytes do not fall on cache lines, so
+// that two waves share most lines: there the default policy keeps a line until
+// its other half comes (C = 191, 991k edges: 1,364 -> 961 us; C = 256 the
+// other way round: 659 against 726 us).
+struct Views {};
+struct SharedViews {};
+template <typename Id>
+constexpr bool kUsesViews = __is_same(Id, Views) || __is_same(Id, SharedViews);
+template <typename Id>
+constexpr int kRowPolicy = __is_same(Id, SharedViews) ? 0 : kNonTemporal;
+
+template <int kPolicy>
+__device__ __forceinline__ void buffer_store_chunk(BufferView view, uint32_t offset, const fvec<4>& value) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const f32x4 raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, raw), view, static_cast<int>(offset), 0, kPolicy);
+}
+
+// Rows [first, first + CAP) of a segment that ends at `end`, as R tiles of PR
+// rows; lane (p, k) holds row i * PR + p, columns [column, column + 4).  The
+// views end with the rows, so a tile's offset is the lane's own plus a
+// multiple of i, with no test per tile; a lane without a column starts past
+// the end (2^31) and stays there (CAP rows are under 2^30 bytes).
+template <int LOG_LS, int R, typename Id>
+struct SlabRows {
+  static constexpr int LS = 1 << LOG_LS;
+  static constexpr int PR = 64 >> LOG_LS;
+  static constexpr int CAP = R * PR;
+  int64_t first;   // wave-uniform
+  int rows, p;     // rows below `end`, at most CAP
+  bool live;
+  uint32_t row_bytes, lane_at;
+  Id id[kUsesViews<Id> ? 1 : R];
+
+  __device__ __forceinline__ SlabRows(int64_t first_, int64_t end, bool live_, int64_t column, int64_t channels)
+      : first(first_), live(live_) {
+    const int64_t left = end - first_;
+    rows = static_cast<int>(left < CAP ? left : CAP);
+    p = static_cast<int>(threadIdx.x & 63) >> LOG_LS;
+    row_bytes = static_cast<uint32_t>(channels) * 4u;
+    lane_at = live ? static_cast<uint32_t>(p) * row_bytes + static_cast<uint32_t>(column) * 4u : kNoRow;
+  }
+  __device__ __forceinline__ bool row(int i) const { return live & (i * PR + p < rows); }
+  __device__ __forceinline__ uint32_t at(int i) const { return lane_at + static_cast<uint32_t>(i * PR) * row_bytes; }
+  __device__ __forceinline__ uint32_t scalar_at(int i) const { return static_cast<uint32_t>(p + i * PR) * 4u; }
+  // These rows of a row-major [n_edges, channels] array.
+  __device__ __forceinline__ BufferView view(const float* base, int64_t channels) const {
+    return buffer_view(base + first * channels, static_cast<int64_t>(rows) * channels * 4);
+  }
+  // Ids of every tile; a lane without a row (or with an order entry out of
+  // range) keeps kNone and reads edge `first` instead.
+  static constexpr uint64_t kNone = ~uint64_t(0);
+  __device__ __forceinline__ void find(const int64_t* __restrict__ order, int64_t n_edges) {
+    if constexpr (!kUsesViews<Id>) {
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int64_t slot = first + (row(i) ? i * PR + p : 0);
+        const int64_t e = order != nullptr ? order[slot] : slot;
+        id[i] = row(i) && static_cast<uint64_t>(e) < static_cast<uint64_t>(n_edges) ? static_cast<Id>(e)
+                                                                                     : static_cast<Id>(kNone);
+      }
     }
-    float null_value = -INFINITY;
-    if (a.null_logit != nullptr) {
-      null_value = a.null_logit[segment * channels + c] * kLog2e;
-      online_add(peak, sum, carry, null_value);
+  }
+  __device__ __forceinline__ bool has(int i) const {
+    if constexpr (kUsesViews<Id>) return row(i);
+    else return id[i] != static_cast<Id>(kNone);
+  }
+  __device__ __forceinline__ int64_t edge(int i) const {  // a valid edge also where there is no row
+    if constexpr (kUsesViews<Id>) return first + i * PR + p;
+    else return has(i) ? static_cast<int64_t>(id[i]) : first;
+  }
+};
+
+// The logit chunks and envelopes of every tile, all loads issued before any use.
+template <int LOG_LS, int R, typename Id>
+__device__ __forceinline__ void slab_forward_loads(const ForwardArgs& a, SlabRows<LOG_LS, R, Id>& t, int64_t column,
+                                                   float (&value)[R][4], float (&envelope)[R]) {
+  t.find(a.order, a.n_edges);
+  if constexpr (kUsesViews<Id>) {
+    const BufferView logit = t.view(a.logit, a.channels);
+    const BufferView env = t.view(a.env, 1);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const fvec<4> x = buffer_load_vec<4, kRowPolicy<Id>>(logit, t.at(i));
+      envelope[i] = buffer_load_f32(env, t.scalar_at(i));
+#pragma unroll
+      for (int v = 0; v < 4; ++v) value[i][v] = x.v[v];
     }
-    const float inverse = inverse_total(sum + carry);
-    for (int64_t slot = begin; slot < end; ++slot) {
-      const int64_t e = edge_of<kOrdered>(a.order, slot, a.n_edges);
-      if (e < 0) continue;
-      a.alpha[e * channels + c] = weight_of(log2_weight(a.logit[e * channels + c], a.env[e]), peak) * inverse;
+  } else {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int64_t e = t.edge(i);
+      const fvec<4> x = load_chunk_stream(a.logit + e * a.channels + column);
+      envelope[i] = a.env[e];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) value[i][v] = x.v[v];
     }
-    if (a.null_logit != nullptr) a.null_alpha[segment * channels + c] = weight_of(null_value, peak) * inverse;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (!kUsesViews<Id>)
+#pragma unroll
+    for (int i = 0; i < R; ++i) envelope[i] = t.has(i) ? envelope[i] : 0.0f;
+}
+
+// 1 / D rounded once (a Newton step on v_rcp_f32 in 64 bits), with D = 1 for a
+// segment without mass.
+__device__ __forceinline__ float inverse_of(double total) {
+  const double d = total > 0.0 ? total : 1.0;
+  const double r = static_cast<double>(__builtin_amdgcn_rcpf(static_cast<float>(d)));
+  return static_cast<float>(__builtin_fma(r, __builtin_fma(-d, r, 1.0), r));
+}
+
+template <int LOG_LS, int R, typename Id>
+__device__ __forceinline__ void slab_forward_stores(const ForwardArgs& a, const SlabRows<LOG_LS, R, Id>& t,
+                                                    int64_t column, const float (&alpha)[R][4], int tiles) {
+  const BufferView out = t.view(a.alpha, a.channels);
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (i >= tiles) continue;
+    const fvec<4> row{{alpha[i][0], alpha[i][1], alpha[i][2], alpha[i][3]}};
+    if constexpr (kUsesViews<Id>) buffer_store_chunk<kRowPolicy<Id>>(out, t.at(i), row);
+    else if (t.has(i)) store_chunk_stream(a.alpha + t.edge(i) * a.channels + column, row);
   }
 }
 
-template <bool kOrdered>
-__global__ __launch_bounds__(kBlock) void softmax_backward_wide_kernel(BackwardArgs a) {
-  const int64_t segment = block_index() * kWaves + (threadIdx.x >> 6);
+template <int LOG_LS, int R, typename Id>
+__global__ __launch_bounds__(kBlock) void softmax_forward_slab_kernel(ForwardArgs a, int64_t slabs) {
+  using T = SlabRows<LOG_LS, R, Id>;
+  constexpr int LS = T::LS, PR = T::PR, CAP = T::CAP;
+  const int64_t unit = uniform_i64(block_index() * kWaves + (threadIdx.x >> 6));
+  const int64_t segment = unit / slabs;
   if (segment >= a.n_nodes) return;
+  const int64_t slab = unit - segment * slabs;
   const int lane = threadIdx.x & 63;
-  const int64_t channels = a.channels;
+  const int64_t chunk = slab * LS + (lane & (LS - 1));
+  const bool live = chunk * 4 < a.channels;
+  const int64_t column = live ? (chunk * 4 + 4 <= a.channels ? chunk * 4 : a.channels - 4) : 0;
+  const bool has_null = a.null_logit != nullptr;
   int64_t begin, end;
   segment_bounds(a.offsets, segment, a.n_edges, begin, end);
-  const bool has_null = a.null_alpha != nullptr;
-  // Channel windows of 64 lanes; grad_env keeps the raw channel sum until the
-  // last window, which applies the 2 / env factor.
-  for (int64_t base = 0; base < channels; base += 64) {
-    const int64_t c = base + lane;
-    const bool live = c < channels;
-    const bool last = base + 64 >= channels;
-    float expect = 0.0f, carry = 0.0f;
-    if (live)
-      for (int64_t slot = begin; slot < end; ++slot) {
-        const int64_t e = edge_of<kOrdered>(a.order, slot, a.n_edges);
-        if (e >= 0) compensated_add(expect, carry, a.alpha[e * channels + c] * a.grad_alpha[e * channels + c]);
+  float nv[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) nv[v] = -INFINITY;
+  if (has_null) {
+    const fvec<4> n0 = load_chunk(a.null_logit + segment * a.channels + column);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) nv[v] = n0.v[v] * kLog2e;
+  }
+  float total[4], nw[4];
+  if (end - begin <= CAP) {
+    T t(begin, end, live, column, a.channels);
+    float value[R][4], envelope[R];
+    if (begin < end) slab_forward_loads(a, t, column, value, envelope);
+    const int tiles = (t.rows + PR - 1) / PR;
+    float peak[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) peak[v] = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+      if (i < tiles) {
+        const float term = row_term(envelope[i]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          value[i][v] = log2_weight_of_row(value[i][v], term);
+          peak[v] = fmaxf(peak[v], value[i][v]);
+        }
       }
-    if (has_null && live)
-      compensated_add(expect, carry, a.null_alpha[segment * channels + c] * a.grad_null_alpha[segment * channels + c]);
-    expect = expect + carry;
-    for (int64_t slot = begin; slot < end; ++slot) {
-      const int64_t e = edge_of<kOrdered>(a.order, slot, a.n_edges);
-      if (e < 0) continue;
-      float out = 0.0f;
-      if (live) {
-        out = a.alpha[e * channels + c] * (a.grad_alpha[e * channels + c] - expect);
-        a.grad_logit[e * channels + c] = out;
+    float shift[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      peak[v] = fmaxf(span_max<LS, 64>(peak[v]), nv[v]);
+      shift[v] = shift_of(peak[v]);
+    }
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+      if (i < tiles)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          value[i][v] = exp2_of(value[i][v] - shift[v]);
+          sum[v] += static_cast<double>(value[i][v]);
+        }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      nw[v] = exp2_of(nv[v] - shift[v]);
+      total[v] = inverse_of(span_sum<LS, 64>(sum[v]) + static_cast<double>(nw[v]));
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+      if (i < tiles)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) value[i][v] *= total[v];
+    if (begin < end) slab_forward_stores(a, t, column, value, tiles);
+  } else {
+    float peak[4];
+    double sum[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int v = 0; v < 4; ++v) peak[v] = -INFINITY;
+    for (int64_t base = begin; base < end; base += CAP) {
+      T t(base, end, live, column, a.channels);
+      float value[R][4], envelope[R];
+      slab_forward_loads(a, t, column, value, envelope);
+      // a round's maximum first, then one rescale and the round's terms
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const float term = row_term(envelope[i]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) value[i][v] = log2_weight_of_row(value[i][v], term);
       }
-      float row = group_sum<64>(out);
-      if (lane == 0) {
-        if (base > 0) row = a.grad_env[e] + row;
-        a.grad_env[e] = last ? env_gradient(row, a.env[e]) : row;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        float top = peak[v];
+#pragma unroll
+        for (int i = 0; i < R; ++i) top = fmaxf(top, value[i][v]);
+        const float shift = shift_of(top);
+        sum[v] *= static_cast<double>(exp2_of(peak[v] - shift));  // by 0 while the column has no mass
+#pragma unroll
+        for (int i = 0; i < R; ++i) sum[v] += static_cast<double>(exp2_of(value[i][v] - shift));
+        peak[v] = top;
       }
     }
-    if (has_null && live)
-      a.grad_null_logit[segment * channels + c] =
-          a.null_alpha[segment * channels + c] * (a.grad_null_alpha[segment * channels + c] - expect);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const float top = fmaxf(span_max<LS, 64>(peak[v]), nv[v]);
+      const float shift = shift_of(top);
+      const double part = sum[v] * static_cast<double>(exp2_of(peak[v] - shift));
+      peak[v] = shift;
+      nw[v] = exp2_of(nv[v] - shift);
+      total[v] = inverse_of(span_sum<LS, 64>(part) + static_cast<double>(nw[v]));
+    }
+    for (int64_t base = begin; base < end; base += CAP) {
+      T t(base, end, live, column, a.channels);
+      float value[R][4], envelope[R];
+      slab_forward_loads(a, t, column, value, envelope);
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const float term = row_term(envelope[i]);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          value[i][v] = exp2_of(log2_weight_of_row(value[i][v], term) - peak[v]) * total[v];
+      }
+      slab_forward_stores(a, t, column, value, R);
+    }
+  }
+  if (has_null && live && lane < LS)
+    store_chunk(a.null_alpha + segment * a.channels + column,
+                fvec<4>{{nw[0] * total[0], nw[1] * total[1], nw[2] * total[2], nw[3] * total[3]}});
+}
+
+// alpha and grad_alpha chunks of every tile (zeros without a row).
+template <int LOG_LS, int R, typename Id>
+__device__ __forceinline__ void slab_backward_loads(const BackwardArgs& a, SlabRows<LOG_LS, R, Id>& t,
+                                                    int64_t column, float (&x)[R][4], float (&g)[R][4]) {
+  t.find(a.order, a.n_edges);
+  if constexpr (kUsesViews<Id>) {
+    const BufferView alpha = t.view(a.alpha, a.channels);
+    const BufferView grad = t.view(a.grad_alpha, a.channels);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const fvec<4> xv = buffer_load_vec<4, kRowPolicy<Id>>(alpha, t.at(i));
+      const fvec<4> gv = buffer_load_vec<4, kRowPolicy<Id>>(grad, t.at(i));
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        x[i][v] = xv.v[v];
+        g[i][v] = gv.v[v];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  } else {
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int64_t e = t.edge(i);
+      const fvec<4> xv = load_chunk_stream(a.alpha + e * a.channels + column);
+      const fvec<4> gv = load_chunk_stream(a.grad_alpha + e * a.channels + column);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        x[i][v] = xv.v[v];
+        g[i][v] = gv.v[v];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        x[i][v] = t.has(i) ? x[i][v] : 0.0f;
+        g[i][v] = t.has(i) ? g[i][v] : 0.0f;
+      }
+  }
+}
+
+// SW waves share a segment (SW > 1), or every wave has a segment of its own
+// (SW = 1, rows of one slab).
+template <int LOG_LS, int R, int SW, typename Id>
+__global__ __launch_bounds__(SW == 1 ? kBlock : SW * 64) void softmax_backward_slab_kernel(BackwardArgs a,
+                                                                                         int64_t slabs) {
+  using T = SlabRows<LOG_LS, R, Id>;
+  constexpr int LS = T::LS, PR = T::PR, CAP = T::CAP;
+  constexpr int kSegments = SW == 1 ? kWaves : 1;  // segments per workgroup
+  __shared__ float row_sum[kSegments][CAP][SW];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int64_t segment = block_index() * kSegments + (SW == 1 ? wave : 0);
+  if (segment >= a.n_nodes) return;  // the whole workgroup, or a wave that shares nothing
+  auto& sums = row_sum[SW == 1 ? wave : 0];
+  const int part = SW == 1 ? 0 : wave;
+  const int lane = threadIdx.x & 63;
+  const int member = SW == 1 ? lane : static_cast<int>(threadIdx.x);  // among the SW * 64 threads of the segment
+  const bool has_null = a.null_alpha != nullptr;
+  int64_t begin, end;
+  segment_bounds(a.offsets, segment, a.n_edges, begin, end);
+
+  for (int64_t round = 0; round < slabs; round += SW) {
+    const int64_t chunk = (round + part) * LS + (lane & (LS - 1));
+    const bool live = chunk * 4 < a.channels;
+    const int64_t column = live ? (chunk * 4 + 4 <= a.channels ? chunk * 4 : a.channels - 4) : 0;
+    const int skip = live ? static_cast<int>(chunk * 4 - column) : 4;  // columns a neighbour accounts for
+    const bool last = round + SW >= slabs;
+    float a0[4], g0[4], expect[4], rest[4];  // S = expect + rest
+    double dot[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int v = 0; v < 4; ++v) a0[v] = g0[v] = 0.0f;
+    // S of each column from the lanes' partial dot products
+    const auto split = [&]() {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const double total = __builtin_fma(static_cast<double>(a0[v]), static_cast<double>(g0[v]),
+                                           span_sum<LS, 64>(dot[v]));
+        expect[v] = static_cast<float>(total);
+        rest[v] = static_cast<float>(total - static_cast<double>(expect[v]));
+      }
+    };
+    const auto add_products = [&](const float(&xs)[R][4], const float(&gs)[R][4], int tiles) {
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+        if (i < tiles)
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            dot[v] = __builtin_fma(static_cast<double>(xs[i][v]), static_cast<double>(gs[i][v]), dot[v]);
+    };
+    if (has_null) {
+      const fvec<4> xv = load_chunk(a.null_alpha + segment * a.channels + column);
+      const fvec<4> gv = load_chunk(a.grad_null_alpha + segment * a.channels + column);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        a0[v] = xv.v[v];
+        g0[v] = gv.v[v];
+      }
+    }
+    float x[R][4], g[R][4];
+    // edge and envelope of the rows this thread finishes, loaded ahead of the rows
+    constexpr int kOwn = (CAP + SW * 64 - 1) / (SW * 64);
+    int64_t own_edge[kOwn];
+    float own_env[kOwn];
+    const auto own_rows = [&](const T& t) {
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q) {
+        const int r = member + q * SW * 64;
+        const int64_t slot = t.first + (r < t.rows ? r : 0);
+        const int64_t e = a.order != nullptr ? a.order[slot] : slot;
+        const bool ok = r < t.rows && static_cast<uint64_t>(e) < static_cast<uint64_t>(a.n_edges);
+        own_edge[q] = ok ? e : -1;
+        own_env[q] = a.env[ok ? e : t.first];
+      }
+    };
+    const auto finish = [&](const T& t) {
+      const BufferView out_view = t.view(a.grad_logit, a.channels);
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        if (i * PR >= t.rows) continue;  // wave-uniform
+        fvec<4> out;
+        float row = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          out.v[v] = x[i][v] * ((g[i][v] - expect[v]) - rest[v]);
+          row += v >= skip ? out.v[v] : 0.0f;
+        }
+        row = span_sum<1, LS>(row);
+        if constexpr (kUsesViews<Id>) buffer_store_chunk<kRowPolicy<Id>>(out_view, t.at(i), out);
+        else if (t.has(i) && live) store_chunk_stream(a.grad_logit + t.edge(i) * a.channels + column, out);
+        if ((lane & (LS - 1)) == 0) sums[i * PR + t.p][part] = row;
+      }
+      if constexpr (SW > 1) __syncthreads();
+      else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int q = 0; q < kOwn; ++q) {
+        if (own_edge[q] < 0) continue;
+        float sum = round > 0 ? a.grad_env[own_edge[q]] : 0.0f;
+#pragma unroll
+        for (int w = 0; w < SW; ++w) sum += sums[member + q * SW * 64][w];
+        a.grad_env[own_edge[q]] = last ? env_gradient(sum, own_env[q]) : sum;
+      }
+    };
+    if (end - begin <= CAP) {
+      if (begin < end) {
+        T t(begin, end, live, column, a.channels);
+        own_rows(t);
+        slab_backward_loads(a, t, column, x, g);
+        add_products(x, g, (t.rows + PR - 1) / PR);
+        split();
+        finish(t);
+      } else {
+        split();
+      }
+    } else {
+      for (int64_t base = begin; base < end; base += CAP) {
+        T t(base, end, live, column, a.channels);
+        slab_backward_loads(a, t, column, x, g);
+        add_products(x, g, R);
+      }
+      split();
+      for (int64_t base = begin; base < end; base += CAP) {
+        T t(base, end, live, column, a.channels);
+        own_rows(t);
+        slab_backward_loads(a, t, column, x, g);
+        finish(t);
+        if constexpr (SW > 1) __syncthreads();  // the row sums are read before the next rows overwrite them
+        else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
+    }
+    if (has_null && live && lane < LS)
+      store_chunk(a.grad_null_logit + segment * a.channels + column,
+                  fvec<4>{{a0[0] * ((g0[0] - expect[0]) - rest[0]), a0[1] * ((g0[1] - expect[1]) - rest[1]),
+                           a0[2] * ((g0[2] - expect[2]) - rest[2]), a0[3] * ((g0[3] - expect[3]) - rest[3])}});
+    if constexpr (SW > 1) {
+      if (!last) __syncthreads();
+    }
   }
 }
 
@@ -1139,12 +1554,15 @@ int lanes_log_for(int64_t chunks) {
   return log;
 }
 
-// Short-path capacity of the kernel that runs `channels` with (vec4) or
-// without 128-bit rows; 0 for the channel-major kernel (no plan use).
+// Rows of at most two aligned chunks (C = 4, 8) and of fewer than four
+// columns run the lane-group kernels, everything else the slab kernels.
+bool uses_slabs(int64_t channels, bool vec4) { return channels > 4 && !(channels == 8 && vec4); }
+
+// Short-path capacity of the lane-group kernel that runs `channels` with
+// (vec4) or without 128-bit rows; 0 for the slab kernels (no plan use).
 int64_t capacity_for(int64_t channels, bool vec4) {
-  const int64_t chunks = vec4 ? channels / 4 : channels;
-  if (chunks > 64) return 0;
-  return short_capacity(vec4 ? 4 : 1, 1 << lanes_log_for(chunks));
+  if (uses_slabs(channels, vec4)) return 0;
+  return short_capacity(vec4 ? 4 : 1, 1 << lanes_log_for(vec4 ? channels / 4 : channels));
 }
 
 int64_t short_blocks(int64_t n_nodes, int v, int log_lc, bool backward) {
@@ -1186,31 +1604,90 @@ int launch_backward(const BackwardArgs& a, const int64_t* plan, int64_t n_long, 
   return launched("softmax_backward_kernel");
 }
 
-template <int V, typename Args>
-int dispatch_forward(int log_lc, const Args& a, const int64_t* list, int64_t n_long, hipStream_t stream) {
-  switch (log_lc) {
-    case 0: return launch_forward<V, 0>(a, list, n_long, stream);
-    case 1: return launch_forward<V, 1>(a, list, n_long, stream);
-    case 2: return launch_forward<V, 2>(a, list, n_long, stream);
-    case 3: return launch_forward<V, 3>(a, list, n_long, stream);
-    case 4: return launch_forward<V, 4>(a, list, n_long, stream);
-    case 5: return launch_forward<V, 5>(a, list, n_long, stream);
-    default: return launch_forward<V, 6>(a, list, n_long, stream);
+// Rows a slab wave holds in registers: the mean degree and 3.5 of its standard
+// deviations (Poisson), so that only outliers are streamed; 64, 96 or 128.
+int slab_rows(int64_t n_edges, int64_t n_nodes) {
+  const double mean = static_cast<double>(n_edges) / static_cast<double>(n_nodes);
+  const double rows = mean + 3.5 * sqrt(mean);
+  return rows <= 64.0 ? 64 : (rows <= 96.0 ? 96 : 128);
+}
+
+// Natural order through 32-bit view offsets, edge ids in 32 bits, or in 64.
+enum class RowIds { kViews, kSharedViews, kNarrow, kWide };
+RowIds row_ids(const int64_t* order, int64_t n_edges, int64_t channels) {
+  if (channels > (int64_t(1) << 20)) return RowIds::kWide;  // 128 rows stay within 2^30 bytes
+  if (order == nullptr) return channels % 32 == 0 || channels < 32 ? RowIds::kViews : RowIds::kSharedViews;
+  return n_edges < 0xffffffffLL ? RowIds::kNarrow : RowIds::kWide;
+}
+
+int slab_lanes_log(int64_t channels) { return channels <= 8 ? 1 : (channels <= 16 ? 2 : 3); }
+
+template <int LOG_LS, typename Id>
+int launch_forward_slabs(const ForwardArgs& a, int rows, int64_t slabs, hipStream_t stream) {
+  constexpr int PR = 64 >> LOG_LS;
+  const dim3 grid = launch_grid((a.n_nodes * slabs + kWaves - 1) / kWaves, kBlock);
+  if constexpr (!__is_same(Id, int64_t)) {
+    if (rows == 64) softmax_forward_slab_kernel<LOG_LS, 64 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs);
+    if (rows == 96) softmax_forward_slab_kernel<LOG_LS, 96 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs);
+    if (rows != 128) return launched("softmax_forward_slab_kernel");
+  }
+  softmax_forward_slab_kernel<LOG_LS, 128 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs);
+  return launched("softmax_forward_slab_kernel");
+}
+
+template <int LOG_LS, int SW, typename Id>
+int launch_backward_slabs_of(const BackwardArgs& a, int rows, int64_t slabs, hipStream_t stream) {
+  constexpr int PR = 64 >> LOG_LS;
+  constexpr int kThreads = SW == 1 ? kBlock : SW * 64;
+  const dim3 grid = launch_grid(SW == 1 ? (a.n_nodes + kWaves - 1) / kWaves : a.n_nodes, kThreads);
+  if constexpr (!__is_same(Id, int64_t)) {
+    if (rows == 64) softmax_backward_slab_kernel<LOG_LS, 64 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs);
+    if (rows == 96) softmax_backward_slab_kernel<LOG_LS, 96 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs);
+    if (rows != 128) return launched("softmax_backward_slab_kernel");
+  }
+  softmax_backward_slab_kernel<LOG_LS, 128 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs);
+  return launched("softmax_backward_slab_kernel");
+}
+
+template <int LOG_LS, typename Id>
+int launch_backward_slabs(const BackwardArgs& a, int rows, int64_t slabs, hipStream_t stream) {
+  if constexpr (LOG_LS == 3) {
+    if (slabs > 4) return launch_backward_slabs_of<LOG_LS, kSlabWaves, Id>(a, rows, slabs, stream);
+    if (slabs > 2) return launch_backward_slabs_of<LOG_LS, 4, Id>(a, rows, slabs, stream);
+    if (slabs > 1) return launch_backward_slabs_of<LOG_LS, 2, Id>(a, rows, slabs, stream);
+  }
+  return launch_backward_slabs_of<LOG_LS, 1, Id>(a, rows, slabs, stream);
+}
+
+#define DPA4K_SLABS(LAUNCH, ID)                                                         \
+  (log_ls == 1 ? LAUNCH<1, ID>(a, rows, slabs, stream)                                   \
+               : (log_ls == 2 ? LAUNCH<2, ID>(a, rows, slabs, stream) : LAUNCH<3, ID>(a, rows, slabs, stream)))
+
+int forward_slabs(const ForwardArgs& a, hipStream_t stream) {
+  const int log_ls = slab_lanes_log(a.channels);
+  const int64_t slabs = ((a.channels + 3) / 4 + (1 << log_ls) - 1) >> log_ls;
+  const int rows = slab_rows(a.n_edges, a.n_nodes);
+  if (!grid_fits(a.n_nodes * slabs, kBlock)) return fail(DPA4K_EINVAL, "segment softmax: grid too large");
+  switch (row_ids(a.order, a.n_edges, a.channels)) {
+    case RowIds::kViews: return DPA4K_SLABS(launch_forward_slabs, Views);
+    case RowIds::kSharedViews: return launch_forward_slabs<3, SharedViews>(a, rows, slabs, stream);
+    case RowIds::kNarrow: return DPA4K_SLABS(launch_forward_slabs, uint32_t);
+    default: return DPA4K_SLABS(launch_forward_slabs, int64_t);
   }
 }
 
-template <int V, typename Args>
-int dispatch_backward(int log_lc, const Args& a, const int64_t* list, int64_t n_long, hipStream_t stream) {
-  switch (log_lc) {
-    case 0: return launch_backward<V, 0>(a, list, n_long, stream);
-    case 1: return launch_backward<V, 1>(a, list, n_long, stream);
-    case 2: return launch_backward<V, 2>(a, list, n_long, stream);
-    case 3: return launch_backward<V, 3>(a, list, n_long, stream);
-    case 4: return launch_backward<V, 4>(a, list, n_long, stream);
-    case 5: return launch_backward<V, 5>(a, list, n_long, stream);
-    default: return launch_backward<V, 6>(a, list, n_long, stream);
+int backward_slabs(const BackwardArgs& a, hipStream_t stream) {
+  const int log_ls = slab_lanes_log(a.channels);
+  const int64_t slabs = ((a.channels + 3) / 4 + (1 << log_ls) - 1) >> log_ls;
+  const int rows = slab_rows(a.n_edges, a.n_nodes);
+  switch (row_ids(a.order, a.n_edges, a.channels)) {
+    case RowIds::kViews: return DPA4K_SLABS(launch_backward_slabs, Views);
+    case RowIds::kSharedViews: return launch_backward_slabs<3, SharedViews>(a, rows, slabs, stream);
+    case RowIds::kNarrow: return DPA4K_SLABS(launch_backward_slabs, uint32_t);
+    default: return DPA4K_SLABS(launch_backward_slabs, int64_t);
   }
 }
+#undef DPA4K_SLABS
 
 int check_common(int64_t n_edges, int64_t n_nodes, int64_t channels, const char* what) {
   if (n_edges < 0 || n_nodes < 0) return fail(DPA4K_EINVAL, "%s: negative sizes", what);
@@ -1234,20 +1711,16 @@ int softmax_forward(const float* logit, const float* env, const int64_t* offsets
   hipStream_t stream = as_stream(stream_handle);
   const bool vec4 = channels % 4 == 0 && aligned16(logit) && aligned16(alpha) &&
                     (null_logit == nullptr || (aligned16(null_logit) && aligned16(null_alpha)));
-  const int64_t chunks = vec4 ? channels / 4 : channels;
   const ForwardArgs a{logit, env, offsets, null_logit, order, alpha, null_alpha, n_edges, n_nodes, channels};
-  if (chunks > 64) {
-    const dim3 grid = launch_grid((n_nodes + kWaves - 1) / kWaves, kBlock);
-    if (order != nullptr) softmax_forward_wide_kernel<true><<<grid, kBlock, 0, stream>>>(a);
-    else softmax_forward_wide_kernel<false><<<grid, kBlock, 0, stream>>>(a);
-    return launched("softmax_forward_wide_kernel");
-  }
+  if (uses_slabs(channels, vec4)) return forward_slabs(a, stream);
   // a plan applies only to the geometry it was built for; otherwise run unplanned
   const bool use_plan = plan != nullptr && plan_capacity == capacity_for(channels, vec4);
   const int64_t* words = use_plan ? static_cast<const int64_t*>(plan) : nullptr;
-  const int log_lc = lanes_log_for(chunks);
-  return vec4 ? dispatch_forward<4>(log_lc, a, words, use_plan ? n_long : 0, stream)
-              : dispatch_forward<1>(log_lc, a, words, use_plan ? n_long : 0, stream);
+  const int64_t listed = use_plan ? n_long : 0;
+  if (vec4) return channels == 4 ? launch_forward<4, 0>(a, words, listed, stream) : launch_forward<4, 1>(a, words, listed, stream);
+  if (channels == 1) return launch_forward<1, 0>(a, words, listed, stream);
+  if (channels == 2) return launch_forward<1, 1>(a, words, listed, stream);
+  return launch_forward<1, 2>(a, words, listed, stream);
 }
 
 int softmax_backward(const float* alpha, const float* grad_alpha, const float* env, const int64_t* offsets,
@@ -1270,20 +1743,17 @@ int softmax_backward(const float* alpha, const float* grad_alpha, const float* e
   const bool vec4 = channels % 4 == 0 && aligned16(alpha) && aligned16(grad_alpha) && aligned16(grad_logit) &&
                     (!has_null || (aligned16(null_alpha) && aligned16(grad_null_alpha) &&
                                    aligned16(grad_null_logit)));
-  const int64_t chunks = vec4 ? channels / 4 : channels;
   const BackwardArgs a{alpha, grad_alpha, env, offsets, null_alpha, grad_null_alpha, order,
                        grad_logit, grad_null_logit, grad_env, n_edges, n_nodes, channels};
-  if (chunks > 64) {
-    const dim3 grid = launch_grid((n_nodes + kWaves - 1) / kWaves, kBlock);
-    if (order != nullptr) softmax_backward_wide_kernel<true><<<grid, kBlock, 0, stream>>>(a);
-    else softmax_backward_wide_kernel<false><<<grid, kBlock, 0, stream>>>(a);
-    return launched("softmax_backward_wide_kernel");
-  }
+  if (uses_slabs(channels, vec4)) return backward_slabs(a, stream);
+  // a plan applies only to the geometry it was built for; otherwise run unplanned
   const bool use_plan = plan != nullptr && plan_capacity == capacity_for(channels, vec4);
   const int64_t* words = use_plan ? static_cast<const int64_t*>(plan) : nullptr;
-  const int log_lc = lanes_log_for(chunks);
-  return vec4 ? dispatch_backward<4>(log_lc, a, words, use_plan ? n_long : 0, stream)
-              : dispatch_backward<1>(log_lc, a, words, use_plan ? n_long : 0, stream);
+  const int64_t listed = use_plan ? n_long : 0;
+  if (vec4) return channels == 4 ? launch_backward<4, 0>(a, words, listed, stream) : launch_backward<4, 1>(a, words, listed, stream);
+  if (channels == 1) return launch_backward<1, 0>(a, words, listed, stream);
+  if (channels == 2) return launch_backward<1, 1>(a, words, listed, stream);
+  return launch_backward<1, 2>(a, words, listed, stream);
 }
 
 }  // namespace
@@ -1331,7 +1801,8 @@ extern "C" int dpa4k_segment_softmax_plan(const int64_t* offsets, int64_t n_edge
   // torch's allocator are 16-byte aligned), for the scalar one otherwise.
   const int64_t capacity = capacity_for(channels, channels % 4 == 0);
   int64_t* words = static_cast<int64_t*>(plan);
-  const int64_t tiles = plan_tiles(n_nodes);
+  // The slab kernels need no plan: an empty one, and no host synchronisation.
+  const int64_t tiles = capacity > 0 ? plan_tiles(n_nodes) : 0;
   int64_t* counts = words + kPlanHeader + n_nodes;
   if (tiles > 0) {
     plan_count_kernel<<<launch_grid(tiles, kPlanThreads), kPlanThreads, 0, stream>>>(offsets, n_nodes, n_edges,
@@ -1340,6 +1811,11 @@ extern "C" int dpa4k_segment_softmax_plan(const int64_t* offsets, int64_t n_edge
   }
   plan_scan_kernel<<<1, kPlanThreads, 0, stream>>>(counts, tiles, capacity, words);
   if (int s = launched("plan_scan_kernel")) return s;
+  if (capacity == 0) {
+    *n_long = 0;
+    *plan_capacity = 0;
+    return DPA4K_OK;
+  }
   if (tiles > 0) {
     plan_write_kernel<<<launch_grid(tiles, kPlanThreads), kPlanThreads, 0, stream>>>(
         offsets, n_nodes, n_edges, capacity, counts, words + kPlanHeader);

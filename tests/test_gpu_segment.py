@@ -546,6 +546,52 @@ def test_segment_softmax_planned_and_unplanned_paths(channels, use_order):
     assert_gradient(g1[2], e_ge, t_ge, "grad_env")
 
 
+@pytest.mark.parametrize("channels", [5, 8, 13, 31, 33, 68, 100, 257, 300])
+@pytest.mark.parametrize("filler", [20, 60, 90])
+@pytest.mark.parametrize("use_order", [False, True])
+def test_segment_softmax_slab_edges(channels, filler, use_order):
+    """Rows cut into slabs of columns: widths that end inside a slab or a 16-byte chunk, bases 4 bytes
+    off 16-byte alignment (C = 8 included, which runs the lane groups when aligned), degrees around each
+    register capacity (the mean degree picks 64, 96 or 128 rows), streamed segments and, past 256
+    channels, several rounds of slabs.  Same rule against the float32 oracle and float64 as above."""
+    announce("softmax slabs", channels, filler, use_order)
+    degrees = np.array([0, 1, 7, 8, 9, 63, 64, 65, 95, 96, 97, 127, 128, 129, 191, 193, 257, 400]
+                       + [filler] * 60, dtype=np.int64)
+    n = degrees.size
+    dst_sorted = torch.from_numpy(workloads.dst_from_degrees(degrees))
+    if use_order:
+        dst, order, offsets = _shuffled(dst_sorted, seed=channels)
+    else:
+        dst, order, offsets = dst_sorted, None, ref.segment_offsets(dst_sorted, n)
+    gen = torch.Generator().manual_seed(channels + filler)
+    edges = dst.numel()
+    logit = torch.randn(edges, channels, generator=gen) * 2.0
+    logit.view(-1)[::101] = 40.0
+    env = torch.rand(edges, generator=gen) + 0.1
+    env[::11] = -1.0
+    null_logit = torch.randn(n, channels, generator=gen)
+    up = torch.randn(edges, channels, generator=gen)
+    up_null = torch.randn(n, channels, generator=gen)
+
+    def off_by_one(tensor):  # the same values at a base 4 bytes past 16-byte alignment
+        buffer = torch.empty(tensor.numel() + 1, device=DEV)
+        return buffer[1:].copy_(tensor.reshape(-1)).view(tensor.shape)
+
+    leaves = [off_by_one(t).requires_grad_(True) for t in (logit, null_logit)]
+    env_dev = env.to(DEV).requires_grad_(True)
+    result = kernels.segment_softmax(leaves[0], env_dev, offsets.to(DEV), leaves[1],
+                                     order=None if order is None else order.to(DEV))
+    grads = torch.autograd.grad(result, (leaves[0], env_dev, leaves[1]), (off_by_one(up), off_by_one(up_null)))
+    e_alpha, e_null = ref.segment_softmax_reference(logit, env, dst, offsets, null_logit)
+    assert_close_scaled(result[0], e_alpha, what="alpha")
+    assert_close_scaled(result[1], e_null, what="null_alpha")
+    e_gl, e_ge, e_gn = ref.segment_softmax_backward_reference(up, logit, env, dst, offsets, null_logit, up_null)
+    t_gl, t_ge, t_gn = segment_softmax_backward_f64(up, logit, env, dst, n, null_logit, up_null)
+    assert_gradient(grads[0], e_gl, t_gl, "grad_logit")
+    assert_gradient(grads[1], e_ge, t_ge, "grad_env")
+    assert_gradient(grads[2], e_gn, t_gn, "grad_null")
+
+
 def test_segment_softmax_plan_lists_the_long_segments():
     from bysj_amd.kernels import _C
 
