@@ -303,6 +303,28 @@ __device__ __forceinline__ void store_vec_stream(float* __restrict__ p, const fv
   }
 }
 
+// Four floats at 4-byte alignment: one dwordx4 access, like the aligned ones.
+// Rows of any width of at least 4 are read in such chunks, the last one
+// starting at width - 4 and repeating up to three of its neighbour's columns.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ fvec<4> load_chunk(const float* __restrict__ p) {
+  const f32x4u raw = *reinterpret_cast<const f32x4u*>(p);
+  return fvec<4>{{raw.x, raw.y, raw.z, raw.w}};
+}
+__device__ __forceinline__ fvec<4> load_chunk_stream(const float* __restrict__ p) {
+  const f32x4u raw = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(p));
+  return fvec<4>{{raw.x, raw.y, raw.z, raw.w}};
+}
+__device__ __forceinline__ void store_chunk(float* __restrict__ p, const fvec<4>& value) {
+  const f32x4u raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
+  *reinterpret_cast<f32x4u*>(p) = raw;
+}
+__device__ __forceinline__ void store_chunk_stream(float* __restrict__ p, const fvec<4>& value) {
+  const f32x4u raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
+  __builtin_nontemporal_store(raw, reinterpret_cast<f32x4u*>(p));
+}
+
 // ---------------------------------------------------------------------------
 // Device: buffer views
 // ---------------------------------------------------------------------------
@@ -387,6 +409,13 @@ __device__ __forceinline__ void buffer_store_vec_stream(BufferView view, uint32_
                                             static_cast<int>(offset == kNoRow ? kNoRow : offset + 4u * i), 0,
                                             kNonTemporal);
   }
+}
+
+template <int kPolicy>
+__device__ __forceinline__ void buffer_store_chunk(BufferView view, uint32_t offset, const fvec<4>& value) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const f32x4 raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, raw), view, static_cast<int>(offset), 0, kPolicy);
 }
 
 __device__ __forceinline__ void buffer_store_f32(BufferView view, uint32_t offset, float value) {

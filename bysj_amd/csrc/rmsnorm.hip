@@ -4,15 +4,15 @@
 //   u = grad * scale,  grad_x = inv * u - (x * inv^3) * mean(x * u)
 //   grad_scale[w] = sum_rows grad * (x * inv)
 //
-// One wave per row.  Rows of up to 64 * 16 float4 chunks (W <= 4096) stay in
-// registers between the sum of squares and the scaled store, so x is read
-// once; the row sum is a DPP / swizzle / bpermute butterfly.  Wider rows take
-// a two-pass streaming kernel.  The reference accumulates grad_scale with one
-// float atomic per (row, column); here each wave keeps per-column partials
-// for its fixed set of rows (two rows loaded per round), the four waves of a
-// workgroup add theirs in LDS, the workgroup partials go to the workspace and
-// a workgroup per 64 columns sums them (its waves split the rows, each load
-// reading 256 contiguous bytes) -- every order fixed.
+// A wave, or 16 or 32 of its lanes, per row.  Rows of up to 64 * 16 float4
+// chunks (W <= 4096) stay in registers between the sum of squares and the
+// scaled store, so x is read once; the row sum is a DPP / swizzle / bpermute
+// butterfly.  Wider rows take a two-pass streaming kernel.  The reference
+// accumulates grad_scale with one float atomic per (row, column); here each
+// lane group keeps per-column partials for its fixed set of rows, the groups
+// of a workgroup add theirs in LDS, the workgroup partials go to the workspace
+// and a workgroup per 64 columns sums them (its waves split the rows, each
+// load reading 256 contiguous bytes) -- every order fixed.
 #include <mutex>
 #include <vector>
 
@@ -35,174 +35,235 @@ constexpr int64_t kRegisterMaxWidth = 64 * 16 * 4;  // widest row the register k
 // scratch_for_stream() obtains from hipGetSymbolAddress.
 static_assert(int64_t(kPartialWaves / kWaves) * kRegisterMaxWidth * 4 == DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES,
               "the header's scratch size must match the partial matrix bound");
-__device__ __align__(256) float scratch[DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES / 4];
+constexpr int64_t kScratchFloats = DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES / 4;
+__device__ __align__(256) float scratch[kScratchFloats];
 
 __device__ __forceinline__ float inverse_rms_of(float sum_squares, int64_t width, float eps) {
   return 1.0f / sqrtf(sum_squares / static_cast<float>(width) + eps);
 }
 
-template <int V, int CPL>
+// A row's chunks over a group of LG lanes: chunk j of lane l is V columns of
+// the row, from byte at(j).  With V = 4 the row's last chunk starts at width -
+// 4, whatever the width and the alignment; where the width is no multiple of 4
+// (kTail) its first `skip` columns are the neighbour's, equal in both lanes, and
+// count in no sum.  A chunk past the row lies past every view: past the row's
+// own view where a wave has one row (LG = 64), else at kNoRow.
+template <int V, int LG, int CPL, bool kTail>
+struct RowChunks {
+  static constexpr bool kOwnView = LG == 64 && !kTail;
+  uint32_t first, start[kOwnView ? 1 : CPL];
+  int skip[kTail ? CPL : 1];
+  __device__ __forceinline__ RowChunks(int lane, int64_t width) {
+    first = static_cast<uint32_t>(lane) * (V * 4u);
+    if constexpr (!kOwnView)
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) {
+        const int64_t begin = static_cast<int64_t>(lane + LG * j) * V;
+        const int64_t column = !kTail || begin + V <= width ? begin : width - V;
+        const bool live = begin < width;
+        start[j] = live ? static_cast<uint32_t>(column) * 4u : kNoRow;
+        if constexpr (kTail) skip[j] = live ? static_cast<int>(begin - column) : V;
+      }
+  }
+  __device__ __forceinline__ uint32_t at(int j) const {
+    if constexpr (kOwnView) return first + static_cast<uint32_t>(j * LG * V * 4);
+    else return start[j];
+  }
+  __device__ __forceinline__ bool counts(int j, int i) const {
+    if constexpr (kTail) return i >= skip[j];
+    else return true;
+  }
+};
+
+// The GPW rows from `first` of a row-major [rows, width] array (none past its end).
+template <int GPW>
+__device__ __forceinline__ BufferView group_view(const float* p, int64_t first, int64_t rows, int64_t width) {
+  const int64_t left = rows - first;
+  const int64_t count = left < GPW ? (left < 0 ? 0 : left) : GPW;
+  return buffer_view(p + (count > 0 ? first : 0) * width, count * width * 4);
+}
+
+// One group of LG lanes per row (LG = 16, 32 or 64: the row's chunks, CPL per
+// lane past 64), NR rows per group in flight, so a wave covers 64 / LG * NR
+// consecutive rows.  Bound by the two row streams.  A wave per row with one
+// chunk a lane left most lanes without a column and little in flight at narrow
+// widths: 262,144 rows of 64 took 61 us (2.2 TB/s), now 24 us (5.6); rows of 1,024
+// are unchanged (33 us for 24,576 rows, 6.1 TB/s).  Rows whose width is not a
+// multiple of 4 were read one float a lane, twice past 1,024 columns: 24,576
+// rows of 2,777 took 175 us, now 102 us.
+template <int V, int LG, int CPL, int NR, bool kTail>
 __global__ __launch_bounds__(kBlock) void rmsnorm_forward_kernel(
+    const float* __restrict__ x, const float* __restrict__ scale, float* __restrict__ y,
+    float* __restrict__ inverse_rms, int64_t rows, int64_t width, float eps) {
+  constexpr int GPW = 64 / LG;
+  const int64_t base = uniform_i64((block_index() * kWaves + (threadIdx.x >> 6)) * (GPW * NR));
+  if (base >= rows) return;
+  const int lane = threadIdx.x & (LG - 1);
+  const int group = (threadIdx.x & 63) / LG;
+  const uint32_t group_at = static_cast<uint32_t>(group) * (static_cast<uint32_t>(width) * 4u);
+  const RowChunks<V, LG, CPL, kTail> chunks(lane, width);
+  // The rows and the scale are loaded before the reduction, through views
+  // (zeros past the rows), so that no load sits in a branch: a load in a
+  // divergent branch is waited for before the branch closes, and the chunk
+  // loads would follow one another instead of overlapping.
+  const BufferView row_s = buffer_view(scale, scale != nullptr ? width * 4 : 0);
+  fvec<V> value[NR][CPL], s[CPL];
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const BufferView rows_x = group_view<GPW>(x, base + r * GPW, rows, width);
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) value[r][j] = buffer_load_vec<V>(rows_x, group_at + chunks.at(j));
+  }
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) s[j] = buffer_load_vec<V>(row_s, chunks.at(j));
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < CPL; ++j)
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+        sum = sum + (chunks.counts(j, i) ? value[r][j].v[i] * value[r][j].v[i] : 0.0f);
+    sum = group_sum<LG>(sum);
+    const float inv = inverse_rms_of(sum, width, eps);
+    const BufferView rows_y = group_view<GPW>(y, base + r * GPW, rows, width);
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) {
+      fvec<V> out;
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        out.v[i] = value[r][j].v[i] * inv;
+        if (scale != nullptr) out.v[i] = out.v[i] * s[j].v[i];
+      }
+      buffer_store_vec_stream<V>(rows_y, group_at + chunks.at(j), out);
+    }
+    if (lane == 0 && base + r * GPW + group < rows) inverse_rms[base + r * GPW + group] = inv;
+  }
+}
+
+// Rows wider than the register kernels hold: a wave per row, two passes.
+__global__ __launch_bounds__(kBlock) void rmsnorm_forward_wide_kernel(
     const float* __restrict__ x, const float* __restrict__ scale, float* __restrict__ y,
     float* __restrict__ inverse_rms, int64_t rows, int64_t width, float eps) {
   const int64_t row = block_index() * kWaves + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int lane = threadIdx.x & 63;
-  const int64_t chunks = width / V;
   const float* xr = x + row * width;
   float* yr = y + row * width;
-  if constexpr (CPL > 0) {
-    // The row and the scale chunks are loaded before the reduction, through
-    // views (zeros past the row), so that no load sits in a branch: a load in
-    // a divergent branch is waited for before the branch closes, and the
-    // chunk loads would follow one another instead of overlapping.
-    const BufferView row_x = buffer_view(x + uniform_i64(row) * width, width * 4);
-    const BufferView row_s = buffer_view(scale, scale != nullptr ? width * 4 : 0);
-    fvec<V> value[CPL], s[CPL];
-    float sum = 0.0f;
+  float sum = 0.0f;
+  for (int64_t c = lane * 4; c < width; c += 256) {
+    const int64_t column = c + 4 <= width ? c : width - 4;
+    const fvec<4> value = load_chunk(xr + column);
 #pragma unroll
-    for (int j = 0; j < CPL; ++j) {
-      const uint32_t offset = static_cast<uint32_t>(lane + 64 * j) * (V * 4u);
-      value[j] = buffer_load_vec<V>(row_x, offset);
-      s[j] = buffer_load_vec<V>(row_s, offset);
-    }
-#pragma unroll
-    for (int j = 0; j < CPL; ++j)
-#pragma unroll
-      for (int i = 0; i < V; ++i) sum = sum + value[j].v[i] * value[j].v[i];
-    sum = group_sum<64>(sum);
-    const float inv = inverse_rms_of(sum, width, eps);
-#pragma unroll
-    for (int j = 0; j < CPL; ++j) {
-      const int64_t q = lane + 64 * j;
-      if (q >= chunks) continue;
-      fvec<V> out;
-#pragma unroll
-      for (int i = 0; i < V; ++i) {
-        out.v[i] = value[j].v[i] * inv;
-        if (scale != nullptr) out.v[i] = out.v[i] * s[j].v[i];
-      }
-      store_vec_stream<V>(yr + q * V, out);
-    }
-    if (lane == 0) inverse_rms[row] = inv;
-  } else {
-    float sum = 0.0f;
-    for (int64_t q = lane; q < chunks; q += 64) {
-      const fvec<V> value = load_vec<V>(xr + q * V);
-#pragma unroll
-      for (int i = 0; i < V; ++i) sum = sum + value.v[i] * value.v[i];
-    }
-    sum = group_sum<64>(sum);
-    const float inv = inverse_rms_of(sum, width, eps);
-    for (int64_t q = lane; q < chunks; q += 64) {
-      const fvec<V> value = load_vec<V>(xr + q * V);
-      fvec<V> out;
-      fvec<V> s;
-      if (scale != nullptr) s = load_vec<V>(scale + q * V);
-#pragma unroll
-      for (int i = 0; i < V; ++i) {
-        out.v[i] = value.v[i] * inv;
-        if (scale != nullptr) out.v[i] = out.v[i] * s.v[i];
-      }
-      store_vec<V>(yr + q * V, out);
-    }
-    if (lane == 0) inverse_rms[row] = inv;
+    for (int i = 0; i < 4; ++i) sum = sum + (column + i >= c ? value.v[i] * value.v[i] : 0.0f);
   }
+  sum = group_sum<64>(sum);
+  const float inv = inverse_rms_of(sum, width, eps);
+  for (int64_t c = lane * 4; c < width; c += 256) {
+    const int64_t column = c + 4 <= width ? c : width - 4;
+    const fvec<4> value = load_chunk(xr + column);
+    fvec<4> out, s;
+    if (scale != nullptr) s = load_chunk(scale + column);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      out.v[i] = value.v[i] * inv;
+      if (scale != nullptr) out.v[i] = out.v[i] * s.v[i];
+    }
+    store_chunk(yr + column, out);
+  }
+  if (lane == 0) inverse_rms[row] = inv;
 }
 
-// Register path (CPL > 0): wave w handles rows w, w + waves, ... (two per round); with
-// `partial` non-null it also stores its per-column sum of grad * (x * inv)
-// as row w of the [waves, W] partial matrix.
-template <int V, int CPL>
+// Register path: wave w handles the GPW = 64 / LG rows from w * GPW, then those
+// `waves` * GPW further on, and so on, NR of these row sets per round (far
+// apart, so that a small grid still spreads over every wave); with `partial`
+// non-null the workgroup also stores its per-column sum of grad * (x * inv) as
+// its row of the [workgroups, W] partial matrix.  All rows of a round are loaded
+// before any is reduced, non-temporally: they are read once (114,688 rows of
+// 1,024: 261 -> 247 us).  Bound by the three row streams; against a wave per
+// row, 262,144 rows of 64 went from 62 to 33 us; rows of 2,777 from 269 us and 11 ms for
+// the scale gradient, a thread per column over all rows, to 130 us with it.
+template <int V, int LG, int CPL, int NR, bool kTail>
 __global__ __launch_bounds__(kBlock) void rmsnorm_backward_kernel(
     const float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ scale,
     const float* __restrict__ inverse_rms, float* __restrict__ grad_x, float* __restrict__ partial,
     int64_t rows, int64_t width) {
+  constexpr int GPW = 64 / LG;
   const int64_t wave_id = static_cast<int64_t>(blockIdx.x) * kWaves + (threadIdx.x >> 6);
-  const int64_t waves = static_cast<int64_t>(gridDim.x) * kWaves;
-  const int lane = threadIdx.x & 63;
-  const int64_t chunks = width / V;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kWaves * GPW;
+  const int lane = threadIdx.x & (LG - 1);
+  const int group = (threadIdx.x & 63) / LG;
+  const uint32_t group_at = static_cast<uint32_t>(group) * (static_cast<uint32_t>(width) * 4u);
+  const RowChunks<V, LG, CPL, kTail> chunks(lane, width);
+  const BufferView row_s = buffer_view(scale, scale != nullptr ? width * 4 : 0);
 
   fvec<V> s[CPL], column[CPL];
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
-    const int64_t q = lane + 64 * j;
+    s[j] = buffer_load_vec<V>(row_s, chunks.at(j));
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-      s[j].v[i] = 1.0f;
-      column[j].v[i] = 0.0f;
-    }
-    if (scale != nullptr && q < chunks) s[j] = load_vec<V>(scale + q * V);
+    for (int i = 0; i < V; ++i) column[j].v[i] = 0.0f;
   }
 
-  // Rows wave_id, wave_id + waves, ... two per round: both rows' loads are
-  // issued before either is reduced.  The rows are read once and loaded
-  // non-temporally (config 3R: 261 -> 247 us).
-  for (int64_t first = wave_id; first < rows; first += 2 * waves) {
-    fvec<V> g[2][CPL], xv[2][CPL];
-    float inv[2];
+  for (int64_t base = uniform_i64(wave_id * GPW); base < rows; base += stride * NR) {
+    fvec<V> g[NR][CPL], xv[NR][CPL];
+    float inv[NR];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int64_t row = first + r * waves;
-      const bool ok = row < rows;
-      inv[r] = ok ? inverse_rms[row] : 0.0f;
+    for (int r = 0; r < NR; ++r) {
+      const int64_t first = base + r * stride;
+      const BufferView rows_g = group_view<GPW>(grad, first, rows, width);
+      const BufferView rows_x = group_view<GPW>(x, first, rows, width);
+      inv[r] = buffer_load_f32(group_view<GPW>(inverse_rms, first, rows, 1), static_cast<uint32_t>(group) * 4u);
 #pragma unroll
       for (int j = 0; j < CPL; ++j) {
-        const int64_t q = lane + 64 * j;
-        if (ok && q < chunks) {
-          g[r][j] = load_vec_stream<V>(grad + row * width + q * V);
-          xv[r][j] = load_vec_stream<V>(x + row * width + q * V);
-        } else {
-#pragma unroll
-          for (int i = 0; i < V; ++i) g[r][j].v[i] = xv[r][j].v[i] = 0.0f;
-        }
+        g[r][j] = buffer_load_vec<V, kNonTemporal>(rows_g, group_at + chunks.at(j));
+        xv[r][j] = buffer_load_vec<V, kNonTemporal>(rows_x, group_at + chunks.at(j));
       }
     }
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int64_t row = first + r * waves;
-      fvec<V> u[CPL];
+    for (int r = 0; r < NR; ++r) {
       float dot = 0.0f;
 #pragma unroll
       for (int j = 0; j < CPL; ++j)
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-          u[j].v[i] = scale != nullptr ? g[r][j].v[i] * s[j].v[i] : g[r][j].v[i];
-          dot = dot + xv[r][j].v[i] * u[j].v[i];
+          const float u = scale != nullptr ? g[r][j].v[i] * s[j].v[i] : g[r][j].v[i];
+          dot = dot + (chunks.counts(j, i) ? xv[r][j].v[i] * u : 0.0f);
         }
-      dot = group_sum<64>(dot);
-      if (row >= rows) continue;
+      dot = group_sum<LG>(dot);
       const float mean_dot = dot / static_cast<float>(width);
       const float inv3 = inv[r] * inv[r] * inv[r];
+      const BufferView rows_o = group_view<GPW>(grad_x, base + r * stride, rows, width);
 #pragma unroll
       for (int j = 0; j < CPL; ++j) {
-        const int64_t q = lane + 64 * j;
-        if (q >= chunks) continue;
         fvec<V> out;
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-          out.v[i] = inv[r] * u[j].v[i] - xv[r][j].v[i] * inv3 * mean_dot;
+          const float u = scale != nullptr ? g[r][j].v[i] * s[j].v[i] : g[r][j].v[i];
+          out.v[i] = inv[r] * u - xv[r][j].v[i] * inv3 * mean_dot;
           if (partial != nullptr) column[j].v[i] = column[j].v[i] + g[r][j].v[i] * (xv[r][j].v[i] * inv[r]);
         }
-        store_vec_stream<V>(grad_x + row * width + q * V, out);
+        buffer_store_vec_stream<V>(rows_o, group_at + chunks.at(j), out);
       }
     }
   }
   if (partial != nullptr) {
-    // the four waves' column sums meet in LDS and are added in wave order;
-    // the workgroup writes one row of the [workgroups, W] partial matrix
-    extern __shared__ float columns[];  // [kWaves][CPL * 64 * V]
-    constexpr int kSpan = CPL * 64 * V;
-    const int wave = threadIdx.x >> 6;
+    // the groups' column sums meet in LDS and are added in group order; the
+    // workgroup writes one row of the [workgroups, W] partial matrix (a column
+    // that two lanes hold is written twice with the same value)
+    extern __shared__ float columns[];  // [kWaves * GPW][CPL * LG * V]
+    constexpr int kSpan = CPL * LG * V;
+    const int member = (threadIdx.x >> 6) * GPW + group;
 #pragma unroll
     for (int j = 0; j < CPL; ++j)
+      if (chunks.at(j) < kSpan * 4u)
 #pragma unroll
-      for (int i = 0; i < V; ++i) columns[wave * kSpan + (lane + 64 * j) * V + i] = column[j].v[i];
+        for (int i = 0; i < V; ++i) columns[member * kSpan + chunks.at(j) / 4 + i] = column[j].v[i];
     __syncthreads();
     for (int64_t c = threadIdx.x; c < width; c += kBlock) {
       float sum = columns[c];
 #pragma unroll
-      for (int w = 1; w < kWaves; ++w) sum = sum + columns[w * kSpan + c];
+      for (int w = 1; w < kWaves * GPW; ++w) sum = sum + columns[w * kSpan + c];
       partial[static_cast<int64_t>(blockIdx.x) * width + c] = sum;
     }
   }
@@ -250,7 +311,6 @@ __global__ __launch_bounds__(kColumnWaves * 64) void partial_columns_kernel(cons
 }
 
 // Streaming grad_x for wide rows: two passes over the row.
-template <int V>
 __global__ __launch_bounds__(kBlock) void rmsnorm_backward_wide_kernel(
     const float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ scale,
     const float* __restrict__ inverse_rms, float* __restrict__ grad_x, int64_t rows,
@@ -258,97 +318,147 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_backward_wide_kernel(
   const int64_t row = block_index() * kWaves + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int lane = threadIdx.x & 63;
-  const int64_t chunks = width / V;
   const float* gr = grad + row * width;
   const float* xr = x + row * width;
   float dot = 0.0f;
-  for (int64_t q = lane; q < chunks; q += 64) {
-    const fvec<V> g = load_vec<V>(gr + q * V);
-    const fvec<V> xv = load_vec<V>(xr + q * V);
-    fvec<V> s;
-    if (scale != nullptr) s = load_vec<V>(scale + q * V);
+  for (int64_t c = lane * 4; c < width; c += 256) {
+    const int64_t column = c + 4 <= width ? c : width - 4;
+    const fvec<4> g = load_chunk(gr + column);
+    const fvec<4> xv = load_chunk(xr + column);
+    fvec<4> s;
+    if (scale != nullptr) s = load_chunk(scale + column);
 #pragma unroll
-    for (int i = 0; i < V; ++i) dot = dot + xv.v[i] * (scale != nullptr ? g.v[i] * s.v[i] : g.v[i]);
+    for (int i = 0; i < 4; ++i)
+      dot = dot + (column + i >= c ? xv.v[i] * (scale != nullptr ? g.v[i] * s.v[i] : g.v[i]) : 0.0f);
   }
   dot = group_sum<64>(dot);
   const float mean_dot = dot / static_cast<float>(width);
   const float inv = inverse_rms[row];
   const float inv3 = inv * inv * inv;
-  for (int64_t q = lane; q < chunks; q += 64) {
-    const fvec<V> g = load_vec<V>(gr + q * V);
-    const fvec<V> xv = load_vec<V>(xr + q * V);
-    fvec<V> s;
-    if (scale != nullptr) s = load_vec<V>(scale + q * V);
-    fvec<V> out;
+  for (int64_t c = lane * 4; c < width; c += 256) {
+    const int64_t column = c + 4 <= width ? c : width - 4;
+    const fvec<4> g = load_chunk(gr + column);
+    const fvec<4> xv = load_chunk(xr + column);
+    fvec<4> s;
+    if (scale != nullptr) s = load_chunk(scale + column);
+    fvec<4> out;
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
+    for (int i = 0; i < 4; ++i) {
       const float u = scale != nullptr ? g.v[i] * s.v[i] : g.v[i];
       out.v[i] = inv * u - xv.v[i] * inv3 * mean_dot;
     }
-    store_vec<V>(grad_x + row * width + q * V, out);
+    store_chunk(grad_x + row * width + column, out);
   }
 }
 
-// grad_scale for wide rows: thread per column, rows summed in order.
+// grad_scale of wide rows: a thread per column and share of the rows (shares
+// along y), its rows summed in order, one row of the partial matrix per share.
 __global__ __launch_bounds__(kBlock) void rmsnorm_scale_columns_kernel(
     const float* __restrict__ grad, const float* __restrict__ x,
-    const float* __restrict__ inverse_rms, float* __restrict__ grad_scale, int64_t rows,
+    const float* __restrict__ inverse_rms, float* __restrict__ partial, int64_t rows, int64_t per_share,
     int64_t width) {
   const int64_t col = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   if (col >= width) return;
+  const int64_t first = blockIdx.y * per_share;
+  const int64_t last = first + per_share < rows ? first + per_share : rows;
   float sum = 0.0f;
-  for (int64_t row = 0; row < rows; ++row)
+  for (int64_t row = first; row < last; ++row)
     sum = sum + grad[row * width + col] * (x[row * width + col] * inverse_rms[row]);
-  grad_scale[col] = sum;
+  partial[blockIdx.y * width + col] = sum;
 }
 
-int per_lane_for(int64_t chunks) {
+// The register kernels' shape for a row of `width` floats: chunks of V floats
+// over LG lanes, CPL per lane.  LG lanes cover rows of up to 256 columns with
+// one chunk each; wider rows take 64 lanes and CPL chunks.
+struct RowShape {
+  int v, lanes, per_lane;
+};
+bool fits_registers(int64_t width) { return width <= kRegisterMaxWidth; }
+RowShape shape_for(int64_t width) {
+  if (width < 4) return {1, 16, 1};
+  const int64_t chunks = (width + 3) / 4;
+  if (chunks <= 16) return {4, 16, 1};
+  if (chunks <= 32) return {4, 32, 1};
   int cpl = 1;
-  while (cpl < 16 && 64 * cpl < chunks) cpl <<= 1;
-  return 64 * cpl >= chunks ? cpl : 0;
+  while (64 * cpl < chunks) cpl <<= 1;
+  return {4, 64, cpl};
 }
 
-template <int V>
-int launch_forward(int cpl, const float* x, const float* scale, float* y, float* inverse_rms,
+// Row sets in flight per wave: forward 4 for the lane groups below a wave where
+// the grid fills the chip (16 waves on each CU) all the same, else 1 (rows of
+// 512 took 25.3 us with two against 23.4 us with one, 32,768 rows); backward 4
+// and 2, and 1 where a row alone takes 128 registers (2,048 columns on: 139 us
+// with two, spilling past the wave's own registers, 120 us with one).
+constexpr int forward_rows(int lanes) { return lanes < 64 ? 4 : 1; }
+constexpr int backward_rows(int lanes, int cpl) { return cpl >= 16 ? 1 : (lanes < 64 ? 4 : 2); }
+constexpr int64_t kFullGrid = 4096;  // waves
+
+// Calls LAUNCH(V, LG, CPL) for a row shape.
+#define DPA4K_ROW_SHAPES(shape, LAUNCH)                   \
+  if (shape.v == 1) LAUNCH(1, 16, 1);                     \
+  else if (shape.lanes == 16) LAUNCH(4, 16, 1);           \
+  else if (shape.lanes == 32) LAUNCH(4, 32, 1);           \
+  else if (shape.per_lane == 1) LAUNCH(4, 64, 1);         \
+  else if (shape.per_lane == 2) LAUNCH(4, 64, 2);         \
+  else if (shape.per_lane == 4) LAUNCH(4, 64, 4);         \
+  else if (shape.per_lane == 8) LAUNCH(4, 64, 8);         \
+  else LAUNCH(4, 64, 16);
+
+// Workgroups whose waves take `sets` row sets each.
+int64_t row_blocks(const RowShape& shape, int sets, int64_t rows) {
+  const int64_t per_block = static_cast<int64_t>(kWaves) * (64 / shape.lanes) * sets;
+  return (rows + per_block - 1) / per_block;
+}
+
+template <int V, int LG, int CPL, int NR>
+void launch_forward_rows(const RowShape& shape, const float* x, const float* scale, float* y, float* inverse_rms,
+                         int64_t rows, int64_t width, float eps, hipStream_t stream) {
+  const dim3 grid = launch_grid(row_blocks(shape, NR, rows), kBlock);
+  if (V == 4 && width % 4 != 0)
+    rmsnorm_forward_kernel<V, LG, CPL, NR, V == 4><<<grid, kBlock, 0, stream>>>(x, scale, y, inverse_rms, rows,
+                                                                                width, eps);
+  else
+    rmsnorm_forward_kernel<V, LG, CPL, NR, false><<<grid, kBlock, 0, stream>>>(x, scale, y, inverse_rms, rows, width,
+                                                                               eps);
+}
+
+int launch_forward(const float* x, const float* scale, float* y, float* inverse_rms,
                    int64_t rows, int64_t width, float eps, hipStream_t stream) {
-  const dim3 grid = launch_grid((rows + kWaves - 1) / kWaves, kBlock);
-#define DPA4K_RMS_FWD(C)                                                                  \
-  rmsnorm_forward_kernel<V, C><<<grid, kBlock, 0, stream>>>(x, scale, y, inverse_rms, rows, \
-                                                            width, eps)
-  switch (cpl) {
-    case 1: DPA4K_RMS_FWD(1); break;
-    case 2: DPA4K_RMS_FWD(2); break;
-    case 4: DPA4K_RMS_FWD(4); break;
-    case 8: DPA4K_RMS_FWD(8); break;
-    case 16: DPA4K_RMS_FWD(16); break;
-    default: DPA4K_RMS_FWD(0); break;
-  }
+  const RowShape shape = shape_for(width);
+  const bool full = row_blocks(shape, forward_rows(shape.lanes), rows) * kWaves >= kFullGrid;
+#define DPA4K_RMS_FWD(V, LG, CPL)                                                                               \
+  (full ? launch_forward_rows<V, LG, CPL, forward_rows(LG)> : launch_forward_rows<V, LG, CPL, 1>)(             \
+      shape, x, scale, y, inverse_rms, rows, width, eps, stream)
+  DPA4K_ROW_SHAPES(shape, DPA4K_RMS_FWD)
 #undef DPA4K_RMS_FWD
   return launched("rmsnorm_forward_kernel");
 }
 
-template <int V>
-int launch_backward(int cpl, unsigned int grid, const float* grad, const float* x,
+int launch_backward(unsigned int grid, const float* grad, const float* x,
                     const float* scale, const float* inverse_rms, float* grad_x, float* partial,
                     int64_t rows, int64_t width, hipStream_t stream) {
-#define DPA4K_RMS_BWD(C)                                                                              \
-  rmsnorm_backward_kernel<V, C><<<grid, kBlock, partial != nullptr ? kWaves * C * 64 * V * sizeof(float) : 0, \
-                                  stream>>>(grad, x, scale, inverse_rms, grad_x, partial, rows, width)
-  switch (cpl) {
-    case 1: DPA4K_RMS_BWD(1); break;
-    case 2: DPA4K_RMS_BWD(2); break;
-    case 4: DPA4K_RMS_BWD(4); break;
-    case 8: DPA4K_RMS_BWD(8); break;
-    default: DPA4K_RMS_BWD(16); break;
-  }
+  const RowShape shape = shape_for(width);
+#define DPA4K_RMS_BWD(V, LG, CPL)                                                                              \
+  ((V == 4 && width % 4 != 0 ? rmsnorm_backward_kernel<V, LG, CPL, backward_rows(LG, CPL), V == 4>                  \
+                             : rmsnorm_backward_kernel<V, LG, CPL, backward_rows(LG, CPL), false>))                 \
+      <<<grid, kBlock, partial != nullptr ? kWaves * CPL * 64 * V * sizeof(float) : 0, stream>>>(               \
+          grad, x, scale, inverse_rms, grad_x, partial, rows, width)
+  DPA4K_ROW_SHAPES(shape, DPA4K_RMS_BWD)
 #undef DPA4K_RMS_BWD
   return launched("rmsnorm_backward_kernel");
 }
 
-unsigned int partial_blocks(int64_t rows) {
-  const int64_t wanted = (rows + kWaves - 1) / kWaves;
-  const int64_t cap = kPartialWaves / kWaves;
-  return static_cast<unsigned int>(wanted < 1 ? 1 : (wanted > cap ? cap : wanted));
+// Rows of the partial matrix that the scale gradient takes: the backward's
+// workgroups, or the shares of wide rows (at least 64 rows each, and no more
+// than `scratch` holds, so that both entry points add in the same order).
+unsigned int partial_blocks(int64_t rows, int64_t width) {
+  const RowShape shape = shape_for(width);
+  int64_t cap = kPartialWaves / kWaves;
+  int64_t wanted = (rows + 63) / 64;
+  if (fits_registers(width)) wanted = row_blocks(shape, 1, rows);
+  else cap = cap < kScratchFloats / width ? cap : kScratchFloats / width;
+  wanted = wanted > cap ? cap : wanted;
+  return static_cast<unsigned int>(wanted < 1 ? 1 : wanted);
 }
 
 // Device address of `scratch` on the device that runs `stream`, looked up once
@@ -390,7 +500,7 @@ int scratch_for_stream(hipStream_t stream, float*& out) {
 
 size_t backward_workspace_bytes(int64_t rows, int64_t width) {
   if (rows <= 0 || width <= 0) return 0;
-  return round_up_256(static_cast<size_t>(partial_blocks(rows)) * static_cast<size_t>(width) * 4);
+  return round_up_256(static_cast<size_t>(partial_blocks(rows, width)) * static_cast<size_t>(width) * 4);
 }
 
 // The backward with its column partials in `workspace` (checked against the size the
@@ -412,60 +522,52 @@ int rmsnorm_backward(const float* grad, const float* x, const float* scale, cons
   }
   if (grad == nullptr || x == nullptr || inverse_rms == nullptr || grad_x == nullptr)
     return fail(DPA4K_EINVAL, "RMSNorm backward: null pointer");
-  const bool vec4 = width % 4 == 0 && aligned16(grad) && aligned16(x) && aligned16(grad_x) &&
-                    (scale == nullptr || aligned16(scale));
-  const int64_t chunks = vec4 ? width / 4 : width;
-  const int cpl = per_lane_for(chunks);
-  if (cpl == 0) {
+  const bool wide = !fits_registers(width);
+  if (wide) {
     const dim3 grid = launch_grid((rows + kWaves - 1) / kWaves, kBlock);
-    if (vec4)
-      rmsnorm_backward_wide_kernel<4><<<grid, kBlock, 0, stream>>>(grad, x, scale, inverse_rms,
-                                                                    grad_x, rows, width);
-    else
-      rmsnorm_backward_wide_kernel<1><<<grid, kBlock, 0, stream>>>(grad, x, scale, inverse_rms,
-                                                                    grad_x, rows, width);
+    rmsnorm_backward_wide_kernel<<<grid, kBlock, 0, stream>>>(grad, x, scale, inverse_rms, grad_x, rows, width);
     if (int s = launched("rmsnorm_backward_wide_kernel")) return s;
-    if (grad_scale != nullptr) {
-      rmsnorm_scale_columns_kernel<<<blocks_for(width, kBlock), kBlock, 0, stream>>>(
-          grad, x, inverse_rms, grad_scale, rows, width);
-      return launched("rmsnorm_scale_columns_kernel");
-    }
-    return DPA4K_OK;
-  }
-  if (grad_scale == nullptr) {
+    if (grad_scale == nullptr) return DPA4K_OK;
+  } else if (grad_scale == nullptr) {
     // the register kernel strides over rows: one row of blocks covers any count
-    const int64_t wanted = (rows + kWaves - 1) / kWaves;
+    const RowShape shape = shape_for(width);
+    const int64_t wanted = row_blocks(shape, 1, rows);
     const int64_t limit = row_block_limit(kBlock);
     const unsigned int grid = static_cast<unsigned int>(wanted < limit ? wanted : limit);
-    return vec4 ? launch_backward<4>(cpl, grid, grad, x, scale, inverse_rms, grad_x, nullptr, rows,
-                                     width, stream)
-                : launch_backward<1>(cpl, grid, grad, x, scale, inverse_rms, grad_x, nullptr, rows,
-                                     width, stream);
+    return launch_backward(grid, grad, x, scale, inverse_rms, grad_x, nullptr, rows, width, stream);
   }
+  unsigned int parts = partial_blocks(rows, width);
   const size_t needed = backward_workspace_bytes(rows, width);
-  if (static_scratch) {
-    // every row of partials the register kernels write fits (width <= kRegisterMaxWidth here)
-    if (needed > static_cast<size_t>(DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES))
+  if (static_scratch && !(wide && parts == 1)) {
+    if (needed > static_cast<size_t>(DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES) + 256)
       return fail(DPA4K_EINVAL,
                   "RMSNorm backward (no allocation): %zu bytes of column partials exceed the %d-byte scratch",
                   needed, DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES);
     float* address = nullptr;
     if (int s = scratch_for_stream(stream, address)) return s;
     workspace = address;
-    workspace_bytes = DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES;
+    workspace_bytes = needed;  // the partials fit; only their size's rounding may not
   }
-  if (workspace == nullptr || workspace_bytes < needed)
-    return fail(DPA4K_EWORKSPACE, "RMSNorm backward: workspace of %zu bytes is smaller than %zu",
-                workspace_bytes, needed);
-  const unsigned int grid = partial_blocks(rows);
+  if (workspace == nullptr || workspace_bytes < needed) {
+    if (!wide)
+      return fail(DPA4K_EWORKSPACE, "RMSNorm backward: workspace of %zu bytes is smaller than %zu",
+                  workspace_bytes, needed);
+    parts = 1;  // wide rows also run without a workspace, a thread per column over all rows
+  }
   float* partial = static_cast<float*>(workspace);
-  int s = vec4 ? launch_backward<4>(cpl, grid, grad, x, scale, inverse_rms, grad_x, partial, rows,
-                                    width, stream)
-               : launch_backward<1>(cpl, grid, grad, x, scale, inverse_rms, grad_x, partial, rows,
-                                    width, stream);
-  if (s) return s;
+  if (wide) {
+    const int64_t per_share = (rows + parts - 1) / parts;
+    float* target = parts > 1 ? partial : grad_scale;
+    rmsnorm_scale_columns_kernel<<<dim3(blocks_for(width, kBlock), parts), kBlock, 0, stream>>>(
+        grad, x, inverse_rms, target, rows, per_share, width);
+    if (int s = launched("rmsnorm_scale_columns_kernel")) return s;
+    if (parts == 1) return DPA4K_OK;
+  } else {
+    const int s = launch_backward(parts, grad, x, scale, inverse_rms, grad_x, partial, rows, width, stream);
+    if (s) return s;
+  }
   partial_columns_kernel<<<static_cast<unsigned int>((width + 63) / 64), kColumnWaves * 64, 0, stream>>>(
-      partial, grid, width, grad_scale);
+      partial, parts, width, grad_scale);
   return launched("partial_columns_kernel");
 }
 
@@ -488,12 +590,10 @@ extern "C" int dpa4k_rmsnorm_forward(const float* x, const float* scale, float* 
   if (x == nullptr || y == nullptr || inverse_rms == nullptr)
     return fail(DPA4K_EINVAL, "RMSNorm: null pointer");
   hipStream_t stream = as_stream(stream_handle);
-  const bool vec4 = width % 4 == 0 && aligned16(x) && aligned16(y) &&
-                    (scale == nullptr || aligned16(scale));
-  const int64_t chunks = vec4 ? width / 4 : width;
-  const int cpl = per_lane_for(chunks);
-  return vec4 ? launch_forward<4>(cpl, x, scale, y, inverse_rms, rows, width, eps, stream)
-              : launch_forward<1>(cpl, x, scale, y, inverse_rms, rows, width, eps, stream);
+  if (fits_registers(width)) return launch_forward(x, scale, y, inverse_rms, rows, width, eps, stream);
+  rmsnorm_forward_wide_kernel<<<launch_grid((rows + kWaves - 1) / kWaves, kBlock), kBlock, 0, stream>>>(
+      x, scale, y, inverse_rms, rows, width, eps);
+  return launched("rmsnorm_forward_wide_kernel");
 }
 
 extern "C" size_t dpa4k_rmsnorm_backward_workspace_size(int64_t rows, int64_t width) {

@@ -1000,26 +1000,6 @@ __global__ __launch_bounds__(kBlock) void softmax_backward_kernel(BackwardArgs a
 
 constexpr int kSlabWaves = 8;  // most slabs of one segment side by side in a backward workgroup
 
-// A float4 at 4-byte alignment (one dwordx4 access).
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-
-__device__ __forceinline__ fvec<4> load_chunk(const float* __restrict__ p) {
-  const f32x4u raw = *reinterpret_cast<const f32x4u*>(p);
-  return fvec<4>{{raw.x, raw.y, raw.z, raw.w}};
-}
-__device__ __forceinline__ fvec<4> load_chunk_stream(const float* __restrict__ p) {
-  const f32x4u raw = __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(p));
-  return fvec<4>{{raw.x, raw.y, raw.z, raw.w}};
-}
-__device__ __forceinline__ void store_chunk(float* __restrict__ p, const fvec<4>& value) {
-  const f32x4u raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
-  *reinterpret_cast<f32x4u*>(p) = raw;
-}
-__device__ __forceinline__ void store_chunk_stream(float* __restrict__ p, const fvec<4>& value) {
-  const f32x4u raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
-  __builtin_nontemporal_store(raw, reinterpret_cast<f32x4u*>(p));
-}
-
 // How a wave finds its rows: natural order through buffer views, or edge ids
 // (from `order`, or the slot itself) and 64-bit addresses, the ids kept in 32
 // bits where they fit.  Rows are read and written once and go non-temporally,
@@ -1033,13 +1013,6 @@ template <typename Id>
 constexpr bool kUsesViews = __is_same(Id, Views) || __is_same(Id, SharedViews);
 template <typename Id>
 constexpr int kRowPolicy = __is_same(Id, SharedViews) ? 0 : kNonTemporal;
-
-template <int kPolicy>
-__device__ __forceinline__ void buffer_store_chunk(BufferView view, uint32_t offset, const fvec<4>& value) {
-  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-  const f32x4 raw = {value.v[0], value.v[1], value.v[2], value.v[3]};
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, raw), view, static_cast<int>(offset), 0, kPolicy);
-}
 
 // Rows [first, first + CAP) of a segment that ends at `end`, as R tiles of PR
 // rows; lane (p, k) holds row i * PR + p, columns [column, column + 4).  The

@@ -149,6 +149,36 @@ def test_rmsnorm_forward_tail_widths(shape):
         assert_close_scaled(out, loops.rmsnorm_loop(x, scale, 1e-5), what="vs fp64 truth")
 
 
+@pytest.mark.parametrize("rows,width", [(9, 2), (300, 3), (1, 4), (70001, 5), (17, 63), (70001, 64), (33, 65), (66000, 100),
+                                        (7, 129), (2049, 255), (131, 257), (13, 510), (4500, 513), (40, 1023), (3, 1025),
+                                        (3300, 2047), (5, 2777), (6, 4094), (3, 4097), (200, 5003)])
+def test_rmsnorm_row_shapes(rows, width):
+    """Lane groups of 16, 32 and 64 lanes at their edges, widths whose last chunk repeats columns, grids
+    below and above the one that takes several row sets per wave, the streaming rows, and operands 4
+    bytes off 16-byte alignment: forward and gradients against float64 and bit for bit aligned."""
+    announce("rmsnorm shapes", rows, width)
+    gen = torch.Generator().manual_seed(rows + width)
+    x, up = torch.randn(rows, width, generator=gen), torch.randn(rows, width, generator=gen)
+    scale = torch.randn(width, generator=gen)
+
+    def run(offset):
+        def place(t):
+            return torch.empty(t.numel() + offset, device=DEV)[offset:].copy_(t.reshape(-1)).view(t.shape)
+
+        xd, sd = place(x).requires_grad_(True), place(scale).requires_grad_(True)
+        out = kernels.rmsnorm(xd, sd, eps=1e-5)
+        return (out.detach(), *torch.autograd.grad(out, (xd, sd), place(up)))
+
+    out, grad_x, grad_scale = run(0)
+    wide = x.double()
+    assert_close_scaled(out, wide * torch.rsqrt(wide.square().mean(1, keepdim=True) + 1e-5) * scale.double(), what="out")
+    t_x, t_s = rmsnorm_backward_f64(up, x, scale, eps=1e-5)
+    assert_close_scaled(grad_x, t_x, what="grad_x vs fp64")
+    assert_close_scaled(grad_scale, t_s, what="grad_scale vs fp64")
+    for got, want, name in zip(run(1), (out, grad_x, grad_scale), ("out", "grad_x", "grad_scale")):
+        assert_bitwise(got, want, f"{name} off alignment")
+
+
 @pytest.mark.parametrize("shape", [(5, 3, 127), (64, 1024), (9, 5000)])
 def test_rmsnorm_gradients(shape):
     announce("rmsnorm bwd", shape)

@@ -74,6 +74,18 @@ def test_noalloc_backward_matches_the_workspace_entry_point():
             assert_close_scaled(got_scale, truth_scale, what="grad_scale vs fp64 closed form")
 
 
+@pytest.mark.parametrize("rows,width", [(700, 5003), (64, 4100), (65, 4100)])
+def test_noalloc_backward_of_streamed_rows(rows, width):
+    """Rows past the register kernels split the scale gradient's rows too, in as many shares for either entry point."""
+    library = _lib.load()
+    announce("rmsnorm backward noalloc, streamed rows", rows, width)
+    grad, x, scale, inverse_rms = _inputs(rows, width, seed=rows + width, offset=0)
+    want_x, want_scale = _with_workspace(library, grad, x, scale, inverse_rms)
+    got_x, got_scale = _without_allocation(library, grad, x, scale, inverse_rms)
+    assert_bitwise(got_x, want_x, "grad_x")
+    assert_bitwise(got_scale, want_scale, "grad_scale")
+
+
 def test_noalloc_backward_without_scale_gradient_and_empty_rows():
     library = _lib.load()
     announce("rmsnorm backward noalloc: no scale gradient, zero rows")
