@@ -2,7 +2,7 @@
 // csrc/segment_sum.cpp:214-317 of the reference).
 //
 // Layout: a lane group of G lanes owns one destination segment; lane l of
-// the group owns the float4 (or float) channel chunks l, l + G, ... of the
+// the group owns the 16-byte (C < 4: float) channel chunks l, l + G, ... of the
 // row.  The group walks the segment's CSR slots in order, so every output
 // element is accumulated sequentially in slot order with the product rounded
 // before the add -- the same arithmetic as `index_add_` on the CPU, hence a
@@ -10,15 +10,16 @@
 // -ffp-contract=off).  256-thread blocks hold 256 / G segments; rows of
 // C = 128 floats give G = 32 (two segments per wave, one 512-byte row per
 // half wave per load), C >= 256 gives one segment per wave with several
-// chunks per lane.
+// chunks per lane, or, on grids too small to fill the chip, one wave per
+// window of 64 chunks (512 segments of 1,024 floats: 58 -> 34 us).
 //
-// Backward is segment-parallel too: a workgroup (rows of 64 to 256 floats)
+// Backward is segment-parallel too: a workgroup (rows of 61 to 2,048 floats)
 // or a lane group loads grad_out[n] once, writes grad_src for every edge of
 // the segment, and reduces the per-edge channel dot product (grad_edge_scale,
-// and summed over the segment grad_node_scale) with a fixed butterfly.  The reference's edge-parallel grad_src kernel
-// needs `dst`; here the CSR names each edge's segment, which the grouping
-// contract makes identical.  Grids too small to fill the chip (few segments)
-// keep up to 32 rows per lane in flight.
+// and summed over the segment grad_node_scale) with a fixed butterfly.  The
+// reference's edge-parallel grad_src kernel needs `dst`; here the CSR names
+// each edge's segment, which the grouping contract makes identical.  Grids too
+// small to fill the chip (few segments) keep up to 32 rows per lane in flight.
 #include "common.h"
 
 namespace dpa4k {
@@ -26,26 +27,51 @@ namespace {
 
 constexpr int kBlock = 256;
 
-template <int V, int G, int CPL, int U, bool kScaleEdge, bool kOrdered>
+// Column of chunk `chunk` of a row of `channels` floats: with V = 4 the last
+// chunk starts at channels - 4 whatever the width, so up to three columns are
+// held by two lanes, which compute and store the same bits (columns are
+// independent; a dot product counts them once, see `skip`).
+template <int V>
+__device__ __forceinline__ int64_t chunk_column(int64_t chunk, int64_t channels, bool& live) {
+  const int64_t column = chunk * V;
+  live = column < channels;
+  return live ? (column + V <= channels ? column : channels - V) : 0;
+}
+
+// A chunk at 4-byte alignment; kStream for rows read or written once.
+template <int V, bool kStream>
+__device__ __forceinline__ fvec<V> load_row_chunk(const float* __restrict__ p) {
+  if constexpr (V == 4) return kStream ? load_chunk_stream(p) : load_chunk(p);
+  else return kStream ? load_vec_stream<V>(p) : load_vec<V>(p);
+}
+template <int V, bool kStream>
+__device__ __forceinline__ void store_row_chunk(float* __restrict__ p, const fvec<V>& value) {
+  if constexpr (V == 4) {
+    if constexpr (kStream) store_chunk_stream(p, value);
+    else store_chunk(p, value);
+  } else {
+    if constexpr (kStream) store_vec_stream<V>(p, value);
+    else store_vec<V>(p, value);
+  }
+}
+
+template <int V, int G, int CPL, int U, bool kScaleEdge, bool kOrdered, bool kStream>
 __global__ __launch_bounds__(kBlock) void segment_sum_forward_kernel(
     const float* __restrict__ src, const int64_t* __restrict__ offsets,
     const float* __restrict__ edge_scale, const float* __restrict__ node_scale,
     const int64_t* __restrict__ order, float* __restrict__ out, int64_t n_edges, int64_t n_nodes,
-    int64_t channels, int64_t chunk_base) {
+    int64_t channels, int64_t windows) {
   constexpr int kSegments = kBlock / G;
-  const int64_t segment = block_index() * kSegments + threadIdx.x / G;
+  const int64_t unit = block_index() * kSegments + threadIdx.x / G;
+  const int64_t segment = windows == 1 ? unit : unit / windows;
   if (segment >= n_nodes) return;
   const int lane = threadIdx.x % G;
-  const int64_t chunks = channels / V;
+  const int64_t chunk_base = (unit - segment * windows) * (G * CPL);
 
   int64_t column[CPL];
   bool live[CPL];
 #pragma unroll
-  for (int j = 0; j < CPL; ++j) {
-    const int64_t chunk = chunk_base + lane + static_cast<int64_t>(G) * j;
-    live[j] = chunk < chunks;
-    column[j] = chunk * V;
-  }
+  for (int j = 0; j < CPL; ++j) column[j] = chunk_column<V>(chunk_base + lane + static_cast<int64_t>(G) * j, channels, live[j]);
 
   int64_t begin, end;
   segment_bounds(offsets, segment, n_edges, begin, end);
@@ -74,7 +100,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_forward_kernel(
 #pragma unroll
       for (int j = 0; j < CPL; ++j) {
         if (live[j] && ok) {
-          x[u][j] = load_vec_stream<V>(src + edge[u] * channels + column[j]);
+          x[u][j] = load_row_chunk<V, kStream>(src + edge[u] * channels + column[j]);
         } else {
 #pragma unroll
           for (int i = 0; i < V; ++i) x[u][j].v[i] = 0.0f;
@@ -100,7 +126,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_forward_kernel(
     fvec<V> result;
 #pragma unroll
     for (int i = 0; i < V; ++i) result.v[i] = scaled ? acc[j].v[i] * scale : acc[j].v[i];
-    store_vec<V>(out + segment * channels + column[j], result);
+    store_row_chunk<V, false>(out + segment * channels + column[j], result);
   }
 }
 
@@ -114,6 +140,12 @@ __global__ __launch_bounds__(kBlock) void segment_sum_forward_kernel(
 // is read once; U edges per round are loaded before any arithmetic.
 // `accumulate` adds the partial dots of this channel window to the values
 // written by the previous window (channels wider than one window).
+//
+// Any width of at least 4 runs in 16-byte chunks, whatever its alignment; one
+// float a lane took 463 us at C = 77 (1.98M edges; now 263 us by the workgroup
+// kernel) and 166 us at C = 13 (now 85).  Natural-order rows of up to 16 floats
+// share lines with the next slots' rows, and their gradients are stored with
+// the default policy, which merges them (C = 8: 99 -> 60 us, C = 16 even).
 template <int V, int G, int CPL, int U, bool kOrdered>
 __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
     const float* __restrict__ grad_out, const float* __restrict__ src,
@@ -126,7 +158,6 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
   const int64_t segment = block_index() * kSegments + threadIdx.x / G;
   if (segment >= n_nodes) return;
   const int lane = threadIdx.x % G;
-  const int64_t chunks = channels / V;
   const bool want_edge = grad_edge_scale != nullptr;
   const bool want_node = grad_node_scale != nullptr;
   const bool need_dot = want_edge || want_node;
@@ -134,11 +165,12 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
 
   int64_t column[CPL];
   bool live[CPL];
+  int skip[CPL];
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
     const int64_t chunk = chunk_base + lane + static_cast<int64_t>(G) * j;
-    live[j] = chunk < chunks;
-    column[j] = chunk * V;
+    column[j] = chunk_column<V>(chunk, channels, live[j]);
+    skip[j] = live[j] ? static_cast<int>(chunk * V - column[j]) : 0;
   }
 
   const float scale = node_scale != nullptr ? node_scale[segment] : 1.0f;
@@ -146,7 +178,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
     if (live[j]) {
-      g[j] = load_vec<V>(grad_out + segment * channels + column[j]);
+      g[j] = load_row_chunk<V, false>(grad_out + segment * channels + column[j]);
     } else {
 #pragma unroll
       for (int i = 0; i < V; ++i) g[j].v[i] = 0.0f;
@@ -171,7 +203,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
 #pragma unroll
       for (int j = 0; j < CPL; ++j) {
         if (need_dot && live[j] && edge[u] >= 0) {
-          x[u][j] = load_vec<V>(src + edge[u] * channels + column[j]);
+          x[u][j] = load_row_chunk<V, false>(src + edge[u] * channels + column[j]);
         } else {
 #pragma unroll
           for (int i = 0; i < V; ++i) x[u][j].v[i] = 0.0f;
@@ -187,7 +219,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
         fvec<V> out;
 #pragma unroll
         for (int i = 0; i < V; ++i) out.v[i] = has_edge_scale ? gs[j].v[i] * weight[u] : gs[j].v[i];
-        store_vec_stream<V>(grad_src + edge[u] * channels + column[j], out);
+        store_row_chunk<V, (kOrdered || G * CPL * V > 16)>(grad_src + edge[u] * channels + column[j], out);
       }
     }
     if (need_dot) {
@@ -197,7 +229,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
 #pragma unroll
         for (int j = 0; j < CPL; ++j)
 #pragma unroll
-          for (int i = 0; i < V; ++i) d = d + g[j].v[i] * x[u][j].v[i];
+          for (int i = 0; i < V; ++i) d = d + (V == 1 || i >= skip[j] ? g[j].v[i] * x[u][j].v[i] : 0.0f);
         dot[u] = group_sum<G>(d);
       }
 #pragma unroll
@@ -264,7 +296,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_staged_kernel(
       const int row = item / chunks;
       const int64_t e = item < items ? edge_of<kOrdered>(order, first + row, n_edges) : -1;
       if (e >= 0) {  // rows are read once: non-temporal (config 1: 7.6 -> 7.25 us)
-        x[k] = load_vec_stream<4>(src + e * channels + static_cast<int64_t>(item - row * chunks) * 4);
+        x[k] = load_chunk_stream(src + e * channels + static_cast<int64_t>(item - row * chunks) * 4);
       } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i) x[k].v[i] = 0.0f;
@@ -304,12 +336,15 @@ __global__ __launch_bounds__(kBlock) void segment_sum_staged_kernel(
   if (t < width) out[segment * channels + t] = node_scale != nullptr ? acc * node_scale[segment] : acc;
 }
 
-// Backward: SG = 256 / G lane groups of G lanes (G >= chunks) take the
-// segment's rows round-robin, U rows per group per round with every load of
-// a round issued first.  grad_edge_scale is per edge; the groups' partial
-// grad_node_scale sums meet in LDS in group order.  Rows of at most 64 chunks.
-// kStreamRows loads the rows non-temporally (small grids, see the launcher).
-template <int G, int U, bool kOrdered, bool kStreamRows>
+// Backward: SG = 256 / G lane groups of G lanes (CPL chunks of a row per lane)
+// take the segment's rows round-robin, U rows per group per round with every
+// load of a round issued first.  grad_edge_scale is per edge; the groups'
+// partial grad_node_scale sums meet in LDS in group order.  kStreamRows loads
+// the rows non-temporally (small grids, see the launcher).  Bound by the
+// streams of src and grad_src.  Rows of several chunks per lane used to run a
+// wave per segment, 2 rows in flight: 3,000 segments of 90 rows of 1,024
+// floats took 483 us, here 452; 512 such segments 139 us, here 84.
+template <int G, int CPL, int U, bool kOrdered, bool kStreamRows, bool kStreamGrads>
 __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
     const float* __restrict__ grad_out, const float* __restrict__ src,
     const int64_t* __restrict__ offsets, const float* __restrict__ edge_scale,
@@ -322,24 +357,33 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
   if (segment >= n_nodes) return;
   const int lane = threadIdx.x % G;
   const int group = threadIdx.x / G;
-  const int chunks = static_cast<int>(channels / 4);
-  const bool live = lane < chunks;
-  const int64_t column = static_cast<int64_t>(live ? lane : 0) * 4;
+  int64_t column[CPL];
+  bool live[CPL];
+  int skip[CPL];
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) {
+    const int64_t chunk = lane + static_cast<int64_t>(G) * j;
+    column[j] = chunk_column<4>(chunk, channels, live[j]);
+    skip[j] = live[j] ? static_cast<int>(chunk * 4 - column[j]) : 0;
+  }
   const bool want_edge = grad_edge_scale != nullptr;
   const bool want_node = grad_node_scale != nullptr;
   const bool need_dot = want_edge || want_node;
   const bool has_edge_scale = edge_scale != nullptr;
 
   const float scale = node_scale != nullptr ? node_scale[segment] : 1.0f;
-  fvec<4> g, gs;
-  if (live) {
-    g = load_vec<4>(grad_out + segment * channels + column);
-  } else {
+  fvec<4> g[CPL], gs[CPL];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) g.v[i] = 0.0f;
+  for (int j = 0; j < CPL; ++j) {
+    if (live[j]) {
+      g[j] = load_chunk(grad_out + segment * channels + column[j]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) g[j].v[i] = 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) gs[j].v[i] = node_scale != nullptr ? g[j].v[i] * scale : g[j].v[i];
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) gs.v[i] = node_scale != nullptr ? g.v[i] * scale : g.v[i];
 
   int64_t begin, end;
   segment_bounds(offsets, segment, n_edges, begin, end);
@@ -347,7 +391,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
   for (int64_t base = begin + group; base < end; base += static_cast<int64_t>(SG) * U) {
     int64_t edge[U];
     float weight[U];
-    fvec<4> x[U];
+    fvec<4> x[U][CPL];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t slot = base + static_cast<int64_t>(u) * SG;
@@ -356,28 +400,36 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       weight[u] = has_edge_scale && edge[u] >= 0 ? edge_scale[edge[u]] : 1.0f;
-      if (need_dot && live && edge[u] >= 0) {
-        x[u] = kStreamRows ? load_vec_stream<4>(src + edge[u] * channels + column)
-                           : load_vec<4>(src + edge[u] * channels + column);
-      } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x[u].v[i] = 0.0f;
+      for (int j = 0; j < CPL; ++j) {
+        if (need_dot && live[j] && edge[u] >= 0) {
+          x[u][j] = load_row_chunk<4, kStreamRows>(src + edge[u] * channels + column[j]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[u][j].v[i] = 0.0f;
+        }
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      if (edge[u] < 0 || !live) continue;
-      fvec<4> o;
+      if (edge[u] < 0) continue;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) o.v[i] = has_edge_scale ? gs.v[i] * weight[u] : gs.v[i];
-      store_vec_stream<4>(grad_src + edge[u] * channels + column, o);
+      for (int j = 0; j < CPL; ++j) {
+        if (!live[j]) continue;
+        fvec<4> o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o.v[i] = has_edge_scale ? gs[j].v[i] * weight[u] : gs[j].v[i];
+        store_row_chunk<4, kStreamGrads>(grad_src + edge[u] * channels + column[j], o);
+      }
     }
     if (need_dot) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         float d = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) d = d + g.v[i] * x[u].v[i];
+        for (int j = 0; j < CPL; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) d = d + (i >= skip[j] ? g[j].v[i] * x[u][j].v[i] : 0.0f);
         d = group_sum<G>(d);
         if (edge[u] < 0) continue;
         if (want_edge && lane == 0) grad_edge_scale[edge[u]] = scale * d;
@@ -412,24 +464,33 @@ int launch_staged_forward(const float* src, const int64_t* offsets, const float*
   return launched("segment_sum_staged_kernel");
 }
 
-template <int G>
+template <int G, int CPL>
 int launch_wide_backward_g(const float* grad_out, const float* src, const int64_t* offsets,
                            const float* edge_scale, const float* node_scale, const int64_t* order,
                            float* grad_src, float* grad_edge_scale, float* grad_node_scale, int64_t n_edges,
                            int64_t n_nodes, int64_t channels, hipStream_t stream) {
-  constexpr int U = 8;
+  constexpr int U = CPL >= 8 ? 1 : 8 / CPL;  // 8 chunks of a row set in flight per lane
   const dim3 grid = launch_grid(n_nodes, kBlock);
-  // Non-temporal row loads pay on small grids (config 1: 11.4 -> 10.6-10.9 us) and not on large ones
-  // (config 1R: 1,846 -> 1,886-1,903 us), measured on one box.
+  // Gradient rows are stored non-temporally, and on small grids the rows loaded so (config 1: 11.4 ->
+  // 10.6-10.9 us; on large ones it does not pay, config 1R: 1,846 -> 1,886-1,903 us), except rows of several
+  // chunks per lane that do not end on cache lines (C = 331: 419 -> 390 us forward and backward; C = 77, one
+  // chunk per lane, the other way round: 402 against 424 us).
   const bool stream_rows = n_nodes < 4096;
-#define DPA4K_SUM_BWD_WIDE(ORD, NT)                                                                    \
-  segment_sum_backward_wide_kernel<G, U, ORD, NT><<<grid, kBlock, 0, stream>>>(                         \
+  const bool shared_lines = CPL > 1 && channels % 32 != 0;
+#define DPA4K_SUM_BWD_WIDE(ORD, NT, NTG)                                                                \
+  segment_sum_backward_wide_kernel<G, CPL, U, ORD, NT, NTG><<<grid, kBlock, 0, stream>>>(                \
       grad_out, src, offsets, edge_scale, node_scale, order, grad_src, grad_edge_scale, grad_node_scale, \
       n_edges, n_nodes, channels)
+  if constexpr (CPL > 1) {
+    if (shared_lines) {
+      if (order != nullptr) DPA4K_SUM_BWD_WIDE(true, false, false); else DPA4K_SUM_BWD_WIDE(false, false, false);
+      return launched("segment_sum_backward_wide_kernel");
+    }
+  }
   if (order != nullptr) {
-    if (stream_rows) DPA4K_SUM_BWD_WIDE(true, true); else DPA4K_SUM_BWD_WIDE(true, false);
+    if (stream_rows) DPA4K_SUM_BWD_WIDE(true, true, true); else DPA4K_SUM_BWD_WIDE(true, false, true);
   } else {
-    if (stream_rows) DPA4K_SUM_BWD_WIDE(false, true); else DPA4K_SUM_BWD_WIDE(false, false);
+    if (stream_rows) DPA4K_SUM_BWD_WIDE(false, true, true); else DPA4K_SUM_BWD_WIDE(false, false, true);
   }
 #undef DPA4K_SUM_BWD_WIDE
   return launched("segment_sum_backward_wide_kernel");
@@ -439,27 +500,30 @@ int launch_wide_backward(const float* grad_out, const float* src, const int64_t*
                          const float* node_scale, const int64_t* order, float* grad_src, float* grad_edge_scale,
                          float* grad_node_scale, int64_t n_edges, int64_t n_nodes, int64_t channels,
                          hipStream_t stream) {
-  const int64_t chunks = channels / 4;
-  if (chunks <= 16)
-    return launch_wide_backward_g<16>(grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
-                                      grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, stream);
-  if (chunks <= 32)
-    return launch_wide_backward_g<32>(grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
-                                      grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, stream);
-  return launch_wide_backward_g<64>(grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
-                                    grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, stream);
+#define DPA4K_SUM_BWD_G(G, CPL)                                                                         \
+  return launch_wide_backward_g<G, CPL>(grad_out, src, offsets, edge_scale, node_scale, order, grad_src, \
+                                        grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, stream)
+  const int64_t chunks = (channels + 3) / 4;
+  if (chunks <= 16) DPA4K_SUM_BWD_G(16, 1);
+  if (chunks <= 32) DPA4K_SUM_BWD_G(32, 1);
+  if (chunks <= 64) DPA4K_SUM_BWD_G(64, 1);
+  if (chunks <= 128) DPA4K_SUM_BWD_G(64, 2);
+  if (chunks <= 256) DPA4K_SUM_BWD_G(64, 4);
+  DPA4K_SUM_BWD_G(64, 8);
+#undef DPA4K_SUM_BWD_G
 }
 
-// The workgroup-per-segment kernels take float4 rows of 16 to 64 chunks (64
-// to 256 channels).  The forward uses its staged kernel on grids of fewer
-// than kWideSegments segments; on larger grids the lane-group kernel's
-// several rows in flight per lane stream faster (config 1R: 1.03 ms against
-// 1.07-1.17 ms).  The backward uses its workgroup kernel on every grid
-// (config 1R: 1.75 ms against 2.15 ms for the lane-group kernel).
+// The workgroup-per-segment kernels.  The forward uses its staged kernel for
+// rows of 16 to 64 whole chunks (64 to 256 channels) on grids of fewer than
+// kWideSegments segments; on larger grids the lane-group kernel's several rows
+// in flight per lane stream faster (config 1R: 1.03 ms against 1.07-1.17 ms).
+// The backward uses its workgroup kernel on every grid for rows of 16 to 512
+// chunks (config 1R: 1.75 ms against 2.15 ms for the lane-group kernel).
 constexpr int64_t kWideSegments = 4096;
-bool wide_rows(int64_t chunks) { return chunks >= 16 && chunks <= 64; }
-bool use_wide_forward(int64_t n_nodes, int64_t chunks) { return n_nodes < kWideSegments && wide_rows(chunks); }
-bool use_wide_backward(int64_t chunks) { return wide_rows(chunks); }
+bool use_wide_forward(int64_t n_nodes, int64_t channels) {
+  return n_nodes < kWideSegments && channels % 4 == 0 && channels >= 64 && channels <= 256;
+}
+bool use_wide_backward(int64_t channels) { return channels > 60 && channels <= 2048; }
 
 // Lane-group geometry for a row of `chunks` vector chunks.
 struct Geometry {
@@ -477,6 +541,7 @@ Geometry geometry_for(int64_t chunks) {
   }
   return g;
 }
+int64_t chunks_for(int64_t channels) { return channels < 4 ? channels : (channels + 3) / 4; }
 
 // Slots per round: about 32 loaded floats per lane, or 128 when the grid is
 // too small to fill the chip (then each lane must keep more bytes in flight).
@@ -488,16 +553,29 @@ constexpr int unroll_for(bool small_grid) {
 template <int V, int G, int CPL, int U>
 int launch_forward_u(const float* src, const int64_t* offsets, const float* edge_scale,
                      const float* node_scale, const int64_t* order, float* out, int64_t n_edges,
-                     int64_t n_nodes, int64_t channels, int64_t chunk_base, hipStream_t stream) {
-  const dim3 grid = launch_grid((n_nodes + kBlock / G - 1) / (kBlock / G), kBlock);
-#define DPA4K_SUM_FWD(SCALE, ORD)                                                                     \
-  segment_sum_forward_kernel<V, G, CPL, U, SCALE, ORD><<<grid, kBlock, 0, stream>>>(                \
-      src, offsets, edge_scale, node_scale, order, out, n_edges, n_nodes, channels, chunk_base)
-  if (edge_scale != nullptr) {
-    if (order != nullptr) DPA4K_SUM_FWD(true, true); else DPA4K_SUM_FWD(true, false);
-  } else {
-    if (order != nullptr) DPA4K_SUM_FWD(false, true); else DPA4K_SUM_FWD(false, false);
+                     int64_t n_nodes, int64_t channels, hipStream_t stream) {
+  // windows of G * CPL chunks are further units of the grid
+  const int64_t windows = (chunks_for(channels) + G * CPL - 1) / (G * CPL);
+  const dim3 grid = launch_grid((n_nodes * windows + kBlock / G - 1) / (kBlock / G), kBlock);
+#define DPA4K_SUM_FWD(SCALE, ORD, NT)                                                                 \
+  segment_sum_forward_kernel<V, G, CPL, U, SCALE, ORD, NT><<<grid, kBlock, 0, stream>>>(             \
+      src, offsets, edge_scale, node_scale, order, out, n_edges, n_nodes, channels, windows)
+#define DPA4K_SUM_FWD_ANY(NT)                                                                         \
+  if (edge_scale != nullptr) {                                                                        \
+    if (order != nullptr) DPA4K_SUM_FWD(true, true, NT); else DPA4K_SUM_FWD(true, false, NT);         \
+  } else {                                                                                            \
+    if (order != nullptr) DPA4K_SUM_FWD(false, true, NT); else DPA4K_SUM_FWD(false, false, NT);       \
   }
+  // Rows under 64 bytes share most of their lines with the next slots' rows: the default policy keeps those
+  // (C = 13, 1.98M edges: 48 -> 41 us).
+  if constexpr (G * CPL * V <= 16) {
+    if (channels < 16 && order == nullptr) {
+      DPA4K_SUM_FWD_ANY(false)
+      return launched("segment_sum_forward_kernel");
+    }
+  }
+  DPA4K_SUM_FWD_ANY(true)
+#undef DPA4K_SUM_FWD_ANY
 #undef DPA4K_SUM_FWD
   return launched("segment_sum_forward_kernel");
 }
@@ -528,17 +606,18 @@ constexpr int ordered_unroll_for() {
 template <int V, int G, int CPL>
 int launch_forward(const float* src, const int64_t* offsets, const float* edge_scale,
                    const float* node_scale, const int64_t* order, float* out, int64_t n_edges,
-                   int64_t n_nodes, int64_t channels, int64_t chunk_base, hipStream_t stream) {
-  if (small_grid(n_nodes, G))
-    return launch_forward_u<V, G, CPL, unroll_for<V, CPL>(true)>(src, offsets, edge_scale, node_scale, order,
-                                                                 out, n_edges, n_nodes, channels, chunk_base,
-                                                                 stream);
+                   int64_t n_nodes, int64_t channels, hipStream_t stream) {
+  if constexpr (CPL == 1) {
+    if (small_grid(n_nodes, G))
+      return launch_forward_u<V, G, CPL, unroll_for<V, CPL>(true)>(src, offsets, edge_scale, node_scale, order, out,
+                                                                   n_edges, n_nodes, channels, stream);
+  }
   if (order == nullptr)
     return launch_forward_u<V, G, CPL, contiguous_unroll_for<V, CPL>()>(src, offsets, edge_scale, node_scale,
                                                                         order, out, n_edges, n_nodes, channels,
-                                                                        chunk_base, stream);
+                                                                        stream);
   return launch_forward_u<V, G, CPL, ordered_unroll_for<V, CPL>()>(src, offsets, edge_scale, node_scale, order, out,
-                                                                   n_edges, n_nodes, channels, chunk_base, stream);
+                                                                   n_edges, n_nodes, channels, stream);
 }
 
 template <int V, int G, int CPL, int U>
@@ -630,23 +709,16 @@ extern "C" int dpa4k_segment_sum_forward(const float* src, const int64_t* offset
   if (offsets == nullptr || out == nullptr || (n_edges > 0 && src == nullptr))
     return fail(DPA4K_EINVAL, "segment sum: null pointer");
   hipStream_t stream = as_stream(stream_handle);
-  const bool vec4 = channels % 4 == 0 && aligned16(src) && aligned16(out);
-  const int64_t chunks = vec4 ? channels / 4 : channels;
-  if (vec4 && use_wide_forward(n_nodes, chunks))
+  if (use_wide_forward(n_nodes, channels))
     return launch_staged_forward(src, offsets, edge_scale, node_scale, order, out, n_edges, n_nodes, channels,
                                  stream);
-  const Geometry geo = geometry_for(chunks);
-  for (int64_t base = 0; base < chunks; base += geo.window()) {
-    const int status =
-        vec4 ? dispatch_geometry<4, ForwardLauncher>(geo, src, offsets, edge_scale, node_scale,
-                                                     order, out, n_edges, n_nodes, channels, base,
-                                                     stream)
-             : dispatch_geometry<1, ForwardLauncher>(geo, src, offsets, edge_scale, node_scale,
-                                                     order, out, n_edges, n_nodes, channels, base,
-                                                     stream);
-    if (status) return status;
-  }
-  return DPA4K_OK;
+  Geometry geo = geometry_for(chunks_for(channels));
+  // a grid too small to fill the chip takes one chunk per lane, and a wave per window of the row
+  if (small_grid(n_nodes, geo.group)) geo.per_lane = 1;
+  return channels >= 4 ? dispatch_geometry<4, ForwardLauncher>(geo, src, offsets, edge_scale, node_scale, order, out,
+                                                               n_edges, n_nodes, channels, stream)
+                       : dispatch_geometry<1, ForwardLauncher>(geo, src, offsets, edge_scale, node_scale, order, out,
+                                                               n_edges, n_nodes, channels, stream);
 }
 
 extern "C" int dpa4k_segment_sum_backward(const float* grad_out, const float* src,
@@ -667,24 +739,20 @@ extern "C" int dpa4k_segment_sum_backward(const float* grad_out, const float* sr
   if (grad_node_scale != nullptr && node_scale == nullptr)
     return fail(DPA4K_EINVAL, "segment sum backward: grad_node_scale needs node_scale");
   hipStream_t stream = as_stream(stream_handle);
-  const bool vec4 = channels % 4 == 0 && aligned16(grad_out) && aligned16(grad_src) &&
-                    (src == nullptr || aligned16(src));
-  const int64_t chunks = vec4 ? channels / 4 : channels;
-  if (vec4 && use_wide_backward(chunks))
+  if (use_wide_backward(channels))
     return launch_wide_backward(grad_out, src, offsets, edge_scale, node_scale, order, grad_src, grad_edge_scale,
                                 grad_node_scale, n_edges, n_nodes, channels, stream);
+  const int64_t chunks = chunks_for(channels);
   const Geometry geo = geometry_for(chunks);
   int accumulate = 0;
   for (int64_t base = 0; base < chunks; base += geo.window()) {
     const int status =
-        vec4 ? dispatch_geometry<4, BackwardLauncher>(
-                   geo, grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
-                   grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, base, accumulate,
-                   stream)
-             : dispatch_geometry<1, BackwardLauncher>(
-                   geo, grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
-                   grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, base, accumulate,
-                   stream);
+        channels >= 4 ? dispatch_geometry<4, BackwardLauncher>(geo, grad_out, src, offsets, edge_scale, node_scale,
+                                                               order, grad_src, grad_edge_scale, grad_node_scale,
+                                                               n_edges, n_nodes, channels, base, accumulate, stream)
+                      : dispatch_geometry<1, BackwardLauncher>(geo, grad_out, src, offsets, edge_scale, node_scale,
+                                                               order, grad_src, grad_edge_scale, grad_node_scale,
+                                                               n_edges, n_nodes, channels, base, accumulate, stream);
     if (status) return status;
     accumulate = 1;
   }

@@ -399,6 +399,49 @@ def test_segment_sum_backward_matches_autograd(channels, use_order):
     assert_gradient(grads[2], e_s, t_s, "grad_node_scale")
 
 
+@pytest.mark.parametrize("channels", [2, 4, 5, 7, 13, 15, 17, 33, 59, 61, 77, 127, 255, 257, 331, 510, 800, 1023, 1025, 2049])
+@pytest.mark.parametrize("use_order", [False, True])
+@pytest.mark.parametrize("nodes", [40, 4500])
+def test_segment_sum_any_width(channels, use_order, nodes):
+    """Widths whose last 16-byte chunk repeats columns, on both sides of the lane-group, workgroup and
+    window limits, on grids below and above those that fill the chip; at 16-byte alignment and 4 bytes
+    off it (the same bits).  grad_edge_scale counts every column once."""
+    announce("segment_sum widths", channels, use_order, nodes)
+    if nodes > 40 and channels > 512:
+        nodes = 2200  # more than 2,048 waves all the same
+    degrees = np.random.default_rng(channels).poisson(3.0, nodes).astype(np.int64)
+    degrees[:8] = [0, 1, 31, 32, 33, 64, 65, 9]
+    degrees[-1] = 2
+    dst_sorted = torch.from_numpy(workloads.dst_from_degrees(degrees))
+    if use_order:
+        dst, order, offsets = _shuffled(dst_sorted, seed=3)
+    else:
+        dst, order, offsets = dst_sorted, None, ref.segment_offsets(dst_sorted, nodes)
+    gen = torch.Generator().manual_seed(channels + 1)
+    src = torch.randn(dst.numel(), channels, generator=gen)
+    w = torch.rand(dst.numel(), generator=gen) + 0.5
+    s = torch.rand(nodes, generator=gen) + 0.5
+    g = torch.randn(nodes, channels, generator=gen)
+
+    def run(offset):
+        def place(t):
+            return torch.empty(t.numel() + offset, device=DEV)[offset:].copy_(t.reshape(-1)).view(t.shape)
+
+        x, wd, sd = place(src).requires_grad_(True), w.to(DEV).requires_grad_(True), s.to(DEV).requires_grad_(True)
+        out = kernels.segment_sum(x, dst.to(DEV), offsets.to(DEV), wd, sd, order=None if order is None else order.to(DEV))
+        return (out.detach(), *torch.autograd.grad(out, (x, wd, sd), place(g)))
+
+    out, grad_src, grad_w, grad_s = run(0)
+    assert_bitwise(out, ref.segment_sum_reference(src, dst, offsets, w, s), "forward vs sequential oracle")
+    e_src, e_w, e_s = ref.segment_sum_backward_reference(g, src, dst, offsets, w, s)
+    _, t_w, t_s = segment_sum_backward_f64(g, src, dst, nodes, w, s)
+    assert_bitwise(grad_src, e_src, "grad_src")
+    assert_gradient(grad_w, e_w, t_w, "grad_edge_scale")
+    assert_gradient(grad_s, e_s, t_s, "grad_node_scale")
+    for got, want, name in zip(run(1), (out, grad_src, grad_w, grad_s), ("out", "grad_src", "grad_w", "grad_s")):
+        assert_bitwise(got, want, f"{name} off alignment")
+
+
 def test_segment_sum_node_scale_shape_and_empty_edges_backward():
     announce("segment_sum bwd shapes")
     dst, offsets = _graph([2, 1, 3])
