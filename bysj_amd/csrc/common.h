@@ -366,6 +366,14 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t value) {
   return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+// `value` of lane `lane` (wave-uniform), as a wave-uniform (scalar) value.
+__device__ __forceinline__ int64_t uniform_lane_i64(int64_t value, int lane) {
+  const uint64_t bits = static_cast<uint64_t>(value);
+  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(bits), lane);
+  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(bits >> 32), lane);
+  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
 // Cache policy of buffer loads and stores: 0 the default, kNonTemporal for
 // data read or written once.
 constexpr int kNonTemporal = 2;

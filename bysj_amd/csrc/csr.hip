@@ -67,7 +67,7 @@ constexpr int kLocalItems = 16;
 constexpr int kLocalChunk = kThreads * kLocalItems;    // 8192 elements per bucket-local round
 constexpr int64_t kShortGap = 64;                      // offsets a thread fills alone
 
-enum : int32_t { kFlagOutOfRange = 1, kFlagUnsorted = 2, kFlagSlotRange = 4, kFlagSlotShared = 8 };
+enum : int32_t { kFlagOutOfRange = 1, kFlagUnsorted = 2, kFlagSlotRange = 4, kFlagSlotShared = 8, kFlagSlotDegrees = 16 };
 constexpr int kSlotRowsShift = 16;  // bits 16..23: most rows reading one radial slot (GIE grouping)
 enum Gate : int { kAlways = 0, kIfSorted = 1, kIfUnsorted = 2 };
 
@@ -1614,17 +1614,25 @@ __global__ __launch_bounds__(kThreads) void widen_kernel(const uint32_t* __restr
 
 // Range and sharing checks of the GIE radial slots (one block of 64).  Also
 // ORs the largest number of rows that read one slot, capped at 255, into
-// bits 16..23 of the status word (kSlotRowsShift).
+// bits 16..23 of the status word (kSlotRowsShift), and whether the map is one
+// slot per degree: rows (l + 1)^2 - 1 - (2 l + 1) up to (l + 1)^2 - 2 read slot
+// l - 1, for l = 1 to n_radial.
 __global__ __launch_bounds__(64) void slot_check_kernel(const int64_t* __restrict__ radial_slot, int64_t n_rows,
                                                         int64_t n_radial, int32_t* __restrict__ status) {
   __shared__ int most;
-  if (threadIdx.x == 0) most = 0;
+  __shared__ int strays;
+  if (threadIdx.x == 0) {
+    most = 0;
+    strays = n_radial <= 255 && n_rows == (n_radial + 1) * (n_radial + 1) - 1 ? 0 : 1;
+  }
   __syncthreads();
   int32_t local = 0;
   int rows_of_slot = 0;
   for (int64_t r = threadIdx.x; r < n_rows; r += blockDim.x) {
     const int64_t slot = radial_slot[r];
     if (static_cast<uint64_t>(slot) >= static_cast<uint64_t>(n_radial)) local |= kFlagSlotRange;
+    const bool of_degree = slot >= 0 && slot < 255 && r >= (slot + 1) * (slot + 1) - 1 && r < (slot + 2) * (slot + 2) - 1;
+    if (!of_degree) atomicOr(&strays, 1);
     int64_t readers = 0;
     for (int64_t other = 0; other < n_rows; ++other) readers += radial_slot[other] == slot ? 1 : 0;
     if (readers > 1) local |= kFlagSlotShared;
@@ -1633,7 +1641,7 @@ __global__ __launch_bounds__(64) void slot_check_kernel(const int64_t* __restric
   }
   atomicMax(&most, rows_of_slot);
   __syncthreads();
-  if (threadIdx.x == 0) local |= most << kSlotRowsShift;
+  if (threadIdx.x == 0) local |= (most << kSlotRowsShift) | (strays == 0 ? kFlagSlotDegrees : 0);
   if (local != 0) atomicOr(status, local);
 }
 
@@ -2017,6 +2025,7 @@ extern "C" int dpa4k_gie_group(const int64_t* dst, const int64_t* radial_slot, i
   if (flags & kFlagSlotRange) return fail(DPA4K_EINVAL, "GIE radial_slot values must be within the radial range");
   const bool sorted = !(flags & kFlagUnsorted);
   if (host_info != nullptr)
-    *host_info = (sorted ? 1 : 0) | ((flags & kFlagSlotShared) ? 0 : 2) | (flags & (0xff << kSlotRowsShift));
+    *host_info = (sorted ? 1 : 0) | ((flags & kFlagSlotShared) ? 0 : 2) | ((flags & kFlagSlotDegrees) ? 4 : 0) |
+                 (flags & (0xff << kSlotRowsShift));
   return DPA4K_OK;
 }

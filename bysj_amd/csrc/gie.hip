@@ -332,6 +332,269 @@ __global__ __launch_bounds__(kBlock) void gie_forward_shared_kernel(
       for (int64_t c = lane; c < row_chunks; c += 64) store_vec<4>(node_out + (r + 1) * channels + c * 4, zero);
 }
 
+__device__ __forceinline__ float fused_inverse_rms(float sum_squares, int64_t width, float eps) {
+  return 1.0f / sqrtf(sum_squares / static_cast<float>(width) + eps);
+}
+
+// ---------------------------------------------------------------------------
+// One radial slot per degree (DeepMD's map), forward and fused RMSNorm
+// ---------------------------------------------------------------------------
+//
+// Degree l has 2 l + 1 rows that read slot l - 1, so with LMAX known at compile
+// time every row, its slot and its accumulator are fixed registers.  A lane
+// owns F channels of a node (C = 64 F / NPW: 64 lanes of one or two channels,
+// or two nodes of 32 lanes) and all R = (LMAX + 1)^2 - 1 rows of them: per edge
+// it loads its F channels of each slot once and does the R F products and sums,
+// the least the sequential rounding allows (product rounded, then added, edges
+// in CSR order: gie_forward_kernel's output bit for bit).  Each 16-lane row of
+// the wave loads the edge's zonal values, and the multiplications take them
+// through a DPP row broadcast.
+//
+// The lane layout of gie_forward_shared_kernel (four groups of 16 lanes, four
+// channels a lane, rows dealt to the groups) ran 5 row iterations of 17
+// instructions per edge for 15 rows at C = 64, bound by their issue; here it is
+// 30 VALU operations and 4 loads, and the kernel is bound by the L1's misses in
+// flight (104 of them per CU, 1,270 cycles each): lanes of 2 or 4 channels, 4 to
+// 24 edges a round, half the waves and zonal values through scalar loads all
+// take 355-385 us where this takes 358.  Measured (us, before -> now): lmax 3,
+// 2.22M edges, C = 64 402 -> 358, C = 32 285 -> 190, C = 128 (half the edges)
+// 420 -> 349; lmax 1, C = 64 166 -> 120; lmax 4, C = 64, 741k edges (9 rows on one
+// slot, which was loaded once per row) 323 -> 166; fused with RMSNorm, which
+// loaded each slot once per row, lmax 3 566 -> 347, lmax 4 346 -> 164.
+//
+// With kNorm the finished row goes through LDS into rmsnorm_forward_kernel's
+// chunk layout (each wave its own tile), so that y, x and inverse_rms equal
+// the two kernels run back to back, bit for bit.
+
+template <int K>
+__device__ __forceinline__ float zonal_broadcast_of(float value) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(value), 0x150 + K, 0xf, 0xf, true));
+}
+
+// k < 16, a constant once the caller's loop is unrolled.
+__device__ __forceinline__ float zonal_broadcast(float value, int k) {
+  switch (k) {
+    case 0: return zonal_broadcast_of<0>(value);
+    case 1: return zonal_broadcast_of<1>(value);
+    case 2: return zonal_broadcast_of<2>(value);
+    case 3: return zonal_broadcast_of<3>(value);
+    case 4: return zonal_broadcast_of<4>(value);
+    case 5: return zonal_broadcast_of<5>(value);
+    case 6: return zonal_broadcast_of<6>(value);
+    case 7: return zonal_broadcast_of<7>(value);
+    case 8: return zonal_broadcast_of<8>(value);
+    case 9: return zonal_broadcast_of<9>(value);
+    case 10: return zonal_broadcast_of<10>(value);
+    case 11: return zonal_broadcast_of<11>(value);
+    case 12: return zonal_broadcast_of<12>(value);
+    case 13: return zonal_broadcast_of<13>(value);
+    case 14: return zonal_broadcast_of<14>(value);
+    default: return zonal_broadcast_of<15>(value);
+  }
+}
+
+template <int F>
+__device__ __forceinline__ void load_channels_stream(const float* __restrict__ p, float (&out)[F]) {
+  if constexpr (F == 2) {
+    typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+    const f32x2u raw = __builtin_nontemporal_load(reinterpret_cast<const f32x2u*>(p));
+    out[0] = raw.x;
+    out[1] = raw.y;
+  } else {
+    out[0] = __builtin_nontemporal_load(p);
+  }
+}
+
+template <int F>
+__device__ __forceinline__ void store_channels(float* __restrict__ p, const float (&value)[F]) {
+  if constexpr (F == 2) {
+    typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+    const f32x2u raw = {value[0], value[1]};
+    *reinterpret_cast<f32x2u*>(p) = raw;
+  } else {
+    *p = value[0];
+  }
+}
+
+struct DegreeArgs {
+  const float* zonal;
+  const float* radial;
+  const int64_t* offsets;
+  const int64_t* order;
+  const float* inv;
+  float* out;  // the rows, or with kNorm the pre-norm rows when wanted
+  int64_t n_edges, n_nodes;
+  // kNorm
+  const float* scale;
+  float* y;
+  float* inverse_rms;
+  float eps;
+};
+
+template <int LMAX, int F, int NPW, bool kOrdered, bool kNorm>
+__global__ __launch_bounds__(kBlock) void gie_forward_degrees_kernel(DegreeArgs a) {
+  constexpr int R = (LMAX + 1) * (LMAX + 1) - 1;
+  constexpr int C = 64 * F / NPW;
+  constexpr int ZR = (R + 15) / 16;                       // zonal values a lane loads per edge
+  constexpr int U = 64 / (LMAX * F + ZR) < 16 ? 64 / (LMAX * F + ZR) : 16;  // edges whose loads go out together
+  constexpr int W = (R + 1) * C;
+  __shared__ float tile[kNorm ? kWaves * NPW * W : 1];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
+  const int half = lane / (64 / NPW);  // which of the wave's nodes
+  const int64_t first_node = (block_index() * kWaves + wave) * NPW;
+  if (first_node >= a.n_nodes) return;
+  const int64_t node = first_node + half;
+  const bool live = NPW == 1 || node < a.n_nodes;
+  const int channel = (lane & (64 / NPW - 1)) * F;
+
+  int64_t begin = 0, end = 0;
+  if (live) segment_bounds(a.offsets, node, a.n_edges, begin, end);
+  int64_t steps = end - begin;
+  if constexpr (NPW > 1) {
+    int64_t most = 0;
+#pragma unroll
+    for (int h = 0; h < NPW; ++h) {
+      const int64_t of_node = uniform_lane_i64(steps, h * (64 / NPW));
+      most = of_node > most ? of_node : most;
+    }
+    steps = most;
+  }
+  const float* zonal_lane[ZR];
+#pragma unroll
+  for (int j = 0; j < ZR; ++j) {
+    const int r = (lane & 15) + 16 * j;
+    zonal_lane[j] = a.zonal + (r < R ? r : R - 1);
+  }
+  const float* radial_lane = a.radial + channel;
+
+  float acc[R][F];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int f = 0; f < F; ++f) acc[r][f] = 0.0f;
+
+  for (int64_t t = 0; t < steps; t += U) {
+    float z[U][ZR], x[U][LMAX][F];
+    bool use[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t slot = begin + t + u;
+      const int64_t e = slot < end ? edge_of<kOrdered>(a.order, slot, a.n_edges) : -1;
+      use[u] = e >= 0;
+      const int64_t edge = e >= 0 ? e : 0;  // a valid edge to load from when this one is absent
+#pragma unroll
+      for (int j = 0; j < ZR; ++j) z[u][j] = zonal_lane[j][edge * R];
+#pragma unroll
+      for (int l = 0; l < LMAX; ++l) load_channels_stream<F>(radial_lane + (edge * LMAX + l) * C, x[u][l]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (!use[u]) continue;  // uniform over each node's lanes
+#pragma unroll
+      for (int l = 0; l < LMAX; ++l)
+#pragma unroll
+        for (int r = (l + 1) * (l + 1) - 1; r < (l + 2) * (l + 2) - 1; ++r) {
+          const float zr = zonal_broadcast(z[u][r / 16], r % 16);
+#pragma unroll
+          for (int f = 0; f < F; ++f) acc[r][f] = acc[r][f] + zr * x[u][l][f];
+        }
+    }
+  }
+
+  const float degree_scale = live ? a.inv[node] : 0.0f;
+  float value[F];
+  if constexpr (!kNorm) {
+    if (!live) return;
+    float* rows = a.out + node * W + channel;
+#pragma unroll
+    for (int f = 0; f < F; ++f) value[f] = 0.0f * degree_scale;
+    store_channels<F>(rows, value);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+      for (int f = 0; f < F; ++f) value[f] = acc[r][f] * degree_scale;
+      store_channels<F>(rows + (r + 1) * C, value);
+    }
+  } else {
+    float* rows = tile + (wave * NPW + half) * W + channel;
+#pragma unroll
+    for (int f = 0; f < F; ++f) rows[f] = 0.0f * degree_scale;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int f = 0; f < F; ++f) rows[(r + 1) * C + f] = acc[r][f] * degree_scale;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave reads back only its own tile
+    constexpr int CPL = (W / 4 + 63) / 64;
+#pragma unroll
+    for (int h = 0; h < NPW; ++h) {
+      if (first_node + h >= a.n_nodes) break;
+      const float* row = tile + (wave * NPW + h) * W;
+      float* y_row = a.y + (first_node + h) * W;
+      fvec<4> v[CPL];
+      float sum = 0.0f;
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) {
+        const int q = lane + 64 * j;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j].v[i] = q * 4 < W ? row[q * 4 + i] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sum = sum + v[j].v[i] * v[j].v[i];
+      }
+      sum = group_sum<64>(sum);
+      const float inv_rms = fused_inverse_rms(sum, W, a.eps);
+#pragma unroll
+      for (int j = 0; j < CPL; ++j) {
+        const int q = lane + 64 * j;
+        if (q * 4 >= W) continue;
+        fvec<4> s, out;
+        if (a.scale != nullptr) s = load_vec<4>(a.scale + q * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          out.v[i] = v[j].v[i] * inv_rms;
+          if (a.scale != nullptr) out.v[i] = out.v[i] * s.v[i];
+        }
+        store_vec_stream<4>(y_row + q * 4, out);
+        if (a.out != nullptr) store_vec<4>(a.out + (first_node + h) * W + q * 4, v[j]);
+      }
+      if (lane == 0) a.inverse_rms[first_node + h] = inv_rms;
+    }
+  }
+}
+
+// Whether the kernels above take this shape (slot_info bit 4, see
+// dpa4k_gie_group).
+bool takes_degrees(int32_t slot_info, int64_t n_rows, int64_t n_radial, int64_t channels) {
+  return (slot_info & 4) && n_radial >= 1 && n_radial <= 4 && n_rows == (n_radial + 1) * (n_radial + 1) - 1 &&
+         (channels == 32 || channels == 64 || channels == 128);
+}
+
+template <int LMAX, int F, int NPW, bool kNorm>
+void launch_degrees_of(const DegreeArgs& a, hipStream_t stream) {
+  const dim3 grid = launch_grid((a.n_nodes + kWaves * NPW - 1) / (kWaves * NPW), kBlock);
+  if (a.order != nullptr) gie_forward_degrees_kernel<LMAX, F, NPW, true, kNorm><<<grid, kBlock, 0, stream>>>(a);
+  else gie_forward_degrees_kernel<LMAX, F, NPW, false, kNorm><<<grid, kBlock, 0, stream>>>(a);
+}
+
+template <int LMAX, bool kNorm>
+void launch_degrees_channels(const DegreeArgs& a, int64_t channels, hipStream_t stream) {
+  if (channels == 32) launch_degrees_of<LMAX, 1, 2, kNorm>(a, stream);
+  else if (channels == 64) launch_degrees_of<LMAX, 1, 1, kNorm>(a, stream);
+  else if constexpr (!kNorm || LMAX < 4) launch_degrees_of<LMAX, 2, 1, kNorm>(a, stream);  // rows of 2,048 floats
+}
+
+template <bool kNorm>
+int launch_degrees(const DegreeArgs& a, int64_t lmax, int64_t channels, hipStream_t stream) {
+  switch (lmax) {
+    case 1: launch_degrees_channels<1, kNorm>(a, channels, stream); break;
+    case 2: launch_degrees_channels<2, kNorm>(a, channels, stream); break;
+    case 3: launch_degrees_channels<3, kNorm>(a, channels, stream); break;
+    default: launch_degrees_channels<4, kNorm>(a, channels, stream); break;
+  }
+  return launched("gie_forward_degrees_kernel");
+}
+
 // Fused GIE -> RMSNorm over each node's flattened row of W = (R + 1) * C
 // floats (no reference counterpart; the reference runs the two operators
 // back to back).  One wave per node, float4 chunks.  Lane l owns the chunks
@@ -342,10 +605,6 @@ __global__ __launch_bounds__(kBlock) void gie_forward_shared_kernel(
 // 1 / sqrt(mean + eps) and the scaled output then follow the RMSNorm kernel
 // step for step, so y, the pre-norm row x (written only when x_out is
 // given) and inverse_rms equal the two kernels run back to back, bit for bit.
-__device__ __forceinline__ float fused_inverse_rms(float sum_squares, int64_t width, float eps) {
-  return 1.0f / sqrtf(sum_squares / static_cast<float>(width) + eps);
-}
-
 template <int CPL, bool kOrdered>
 __global__ __launch_bounds__(kBlock) void gie_rmsnorm_forward_kernel(
     const float* __restrict__ zonal, const float* __restrict__ radial,
@@ -1205,6 +1464,10 @@ extern "C" int dpa4k_gie_zonal_scatter_forward_csr(
   hipStream_t stream = as_stream(stream_handle);
   const bool vec4 = channels % 4 == 0 && aligned16(radial) && aligned16(out);
   const int64_t row_chunks = vec4 ? channels / 4 : channels;
+  if (takes_degrees(slot_info, n_rows, n_radial, channels))
+    return launch_degrees<false>({zonal, radial, offsets, order, inv_sqrt_deg, out, n_edges, n_nodes, nullptr, nullptr,
+                                  nullptr, 0.0f},
+                                 n_radial, channels, stream);
   // Shared slots: one pass over each edge's radial block, rows served per slot.
   const int most = slot_rows(slot_info);
   if (vec4 && !(slot_info & kSlotsDistinct) && most >= 2 && most <= 8 && n_rows >= 1 && n_rows <= 64 &&
@@ -1456,7 +1719,17 @@ extern "C" int dpa4k_gie_rmsnorm_forward_csr(const float* zonal, const float* ra
                                              const float* inv_sqrt_deg, const float* scale, float eps, float* y,
                                              float* x_out, float* inverse_rms, int64_t n_edges, int64_t n_nodes,
                                              int64_t n_rows, int64_t n_radial, int64_t channels,
-                                             dpa4k_stream_t stream_handle) {
+                                             dpa4k_stream_t stream) {
+  return dpa4k_gie_rmsnorm_forward_slots(zonal, radial, offsets, order, radial_slot, inv_sqrt_deg, scale, eps, y,
+                                         x_out, inverse_rms, n_edges, n_nodes, n_rows, n_radial, channels, 0, stream);
+}
+
+extern "C" int dpa4k_gie_rmsnorm_forward_slots(const float* zonal, const float* radial, const int64_t* offsets,
+                                               const int64_t* order, const int64_t* radial_slot,
+                                               const float* inv_sqrt_deg, const float* scale, float eps, float* y,
+                                               float* x_out, float* inverse_rms, int64_t n_edges, int64_t n_nodes,
+                                               int64_t n_rows, int64_t n_radial, int64_t channels,
+                                               int32_t slot_info, dpa4k_stream_t stream_handle) {
   clear_error();
   if (int s = check_shapes(n_edges, n_nodes, n_rows, n_radial, channels, "GIE RMSNorm")) return s;
   if (!dpa4k_gie_rmsnorm_supported(n_rows, channels))
@@ -1472,6 +1745,10 @@ extern "C" int dpa4k_gie_rmsnorm_forward_csr(const float* zonal, const float* ra
       (scale != nullptr && !aligned16(scale)))
     return fail(DPA4K_EINVAL, "GIE RMSNorm: radial, scale and outputs must be 16-byte aligned");
   hipStream_t stream = as_stream(stream_handle);
+  if (takes_degrees(slot_info, n_rows, n_radial, channels))
+    return launch_degrees<true>({zonal, radial, offsets, order, inv_sqrt_deg, x_out, n_edges, n_nodes, scale, y,
+                                 inverse_rms, eps},
+                                n_radial, channels, stream);
   const int cpl = per_lane_for((n_rows + 1) * (channels / 4));
   return order != nullptr
              ? launch_gie_rmsnorm<true>(cpl, zonal, radial, offsets, order, radial_slot, inv_sqrt_deg, scale, eps, y,

@@ -558,8 +558,9 @@ def gie_group(dst, radial_slot, n_nodes: int, n_radial: int):
     """Destination CSR of an unsorted ``dst``: ``(offsets, order or None, info)``.
 
     ``order`` is None when ``dst`` is already non-decreasing; ``info`` bit 2
-    says every radial slot feeds at most one row and bits 16..23 hold the most
-    rows that read one slot.  The GIE kernels below take ``info`` as
+    says every radial slot feeds at most one row, bit 4 that each degree l has
+    one slot (l - 1) for its 2 l + 1 rows, and bits 16..23 hold the most rows
+    that read one slot.  The GIE kernels below take ``info`` as
     ``slot_info`` to pick their layout.  ValueError on out-of-range ``dst`` or
     ``radial_slot`` values.
     """
@@ -600,12 +601,14 @@ def gie_rmsnorm_supported(n_rows: int, channels: int) -> bool:
     return bool(_LIB.dpa4k_gie_rmsnorm_supported(int(n_rows), int(channels)))
 
 
-def gie_rmsnorm_forward_csr(zonal, radial, offsets, order, radial_slot, inv_sqrt_deg, scale, eps, keep_x=False):
+def gie_rmsnorm_forward_csr(zonal, radial, offsets, order, radial_slot, inv_sqrt_deg, scale, eps, keep_x=False,
+                            *, slot_info=0):
     """Fused GIE zonal scatter and RMSNorm over each node's flattened (n_rows + 1) * channels row.
 
     Returns ``(y, x, inverse_rms)``: ``y`` shaped ``(n_nodes, n_rows + 1, channels)``, the pre-norm
     GIE output ``x`` of the same shape when ``keep_x`` (else None) and ``inverse_rms`` ``(n_nodes,)``.
-    ``scale`` is a ``((n_rows + 1) * channels,)`` tensor or an empty one for no scale.
+    ``scale`` is a ``((n_rows + 1) * channels,)`` tensor or an empty one for no scale; ``slot_info`` is
+    :func:`gie_group`'s info of ``radial_slot``, or 0.
     """
     edges, rows = int(zonal.shape[0]), int(zonal.shape[1])
     n_radial, channels = int(radial.shape[1]), int(radial.shape[2])
@@ -622,10 +625,10 @@ def gie_rmsnorm_forward_csr(zonal, radial, offsets, order, radial_slot, inv_sqrt
     if nodes == 0:
         return y, x, inverse_rms
     with _on(zonal.device) as stream:
-        status = _LIB.dpa4k_gie_rmsnorm_forward_csr(
+        status = _LIB.dpa4k_gie_rmsnorm_forward_slots(
             _ptr(zonal), _ptr(radial), offsets.data_ptr(), _ptr(order), _ptr(radial_slot), inv_sqrt_deg.data_ptr(),
             _ptr(scale), float(eps), y.data_ptr(), None if x is None else x.data_ptr(), inverse_rms.data_ptr(),
-            edges, nodes, rows, n_radial, channels, stream,
+            edges, nodes, rows, n_radial, channels, int(slot_info), stream,
         )
     _lib.check(status)
     return y, x, inverse_rms

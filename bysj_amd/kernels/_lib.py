@@ -80,6 +80,8 @@ PROTOTYPES: dict[str, tuple[object, list[object]]] = {
     "dpa4k_gie_rmsnorm_supported": (_INT, [_I64, _I64]),
     "dpa4k_gie_rmsnorm_forward_csr": (
         _INT, [_P, _P, _P, _P, _P, _P, _P, _F32, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P]),
+    "dpa4k_gie_rmsnorm_forward_slots": (
+        _INT, [_P, _P, _P, _P, _P, _P, _P, _F32, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, ctypes.c_int32, _P]),
     "dpa4k_rmsnorm_forward": (_INT, [_P, _P, _P, _P, _I64, _I64, _F32, _P]),
     "dpa4k_rmsnorm_backward_workspace_size": (_SZ, [_I64, _I64]),
     "dpa4k_rmsnorm_backward": (_INT, [_P, _P, _P, _P, _P, _P, _I64, _I64, _P, _SZ, _P]),

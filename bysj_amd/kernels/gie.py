@@ -185,6 +185,11 @@ def gie_zonal_scatter(zonal, radial, dst, radial_slot, inv_sqrt_deg):
     return zonal_scatter(zonal, radial, dst, radial_slot, inv_sqrt_deg)
 
 
+# The bit of the grouping's info word for DeepMD's radial map: the fused kernel then reads each radial
+# element once per edge instead of once per row of its degree.
+_SLOT_PER_DEGREE = 4
+
+
 class _GIERMSNormFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, zonal, radial, dst, radial_slot, inv_sqrt_deg, scale, eps):
@@ -192,8 +197,9 @@ class _GIERMSNormFunction(torch.autograd.Function):
         n_nodes, n_radial = int(inv_sqrt_deg.shape[0]), int(radial.shape[1])
         offsets, order, info = _GROUPINGS.get(native, dst, radial_slot, n_nodes, n_radial)
         keep_x = any(ctx.needs_input_grad)
+        layout = {"slot_info": info} if info & _SLOT_PER_DEGREE else {}
         y, x, inverse_rms = native.gie_rmsnorm_forward_csr(zonal, radial, offsets, order, radial_slot,
-                                                          inv_sqrt_deg, scale, eps, keep_x)
+                                                          inv_sqrt_deg, scale, eps, keep_x, **layout)
         ctx.slot_info = info
         ctx.has_order = order is not None
         ctx.has_scale = scale.numel() != 0

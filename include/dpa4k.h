@@ -358,6 +358,8 @@ int dpa4k_edge_stream_combine(const dpa4k_edge_operand* a,
  * host_info (host pointer, may be NULL) receives a bit set:
  *   1 = dst was non-decreasing (the kernels may then take a NULL order),
  *   2 = every radial slot is referenced by at most one row,
+ *   4 = one slot per degree: R = (S + 1)^2 - 1 and the 2 l + 1 rows from
+ *       l^2 - 1 reference slot l - 1, for l = 1 to S,
  *   bits 16..23 = the most rows that reference one slot (capped at 255).
  * The GIE kernels below take this word as `slot_info` to pick their layout;
  * 0 means "unknown" and selects kernels that assume nothing about the map.
@@ -377,9 +379,9 @@ int dpa4k_gie_group(const int64_t* dst, const int64_t* radial_slot,
  * inv_sqrt_deg[N], out[N, R+1, C].  Sequential per-element accumulation:
  * equals the fp32 chain `gather -> mul -> index_add_ -> mul` bit for bit.
  * slot_info: dpa4k_gie_group's host_info for this radial_slot, or 0.  With
- * shared slots and at most 8 rows per slot it selects a kernel that reads
- * each radial element once per edge (same output); it must then describe
- * radial_slot truthfully. */
+ * one slot per degree (S <= 4, C = 32, 64 or 128) or with shared slots and at
+ * most 8 rows per slot it selects a kernel that reads each radial element
+ * once per edge (same output); it must then describe radial_slot truthfully. */
 int dpa4k_gie_zonal_scatter_forward_csr(const float* zonal, const float* radial,
                                         const int64_t* offsets,
                                         const int64_t* order,
@@ -450,6 +452,22 @@ int dpa4k_gie_rmsnorm_forward_csr(const float* zonal, const float* radial,
                                   int64_t n_nodes, int64_t n_rows,
                                   int64_t n_radial, int64_t channels,
                                   dpa4k_stream_t stream);
+
+/* The same with dpa4k_gie_group's host_info for this radial_slot (or 0, which
+ * is dpa4k_gie_rmsnorm_forward_csr): one slot per degree then reads each
+ * radial element once per edge, as in dpa4k_gie_zonal_scatter_forward_csr.
+ * Same output bit for bit. */
+int dpa4k_gie_rmsnorm_forward_slots(const float* zonal, const float* radial,
+                                    const int64_t* offsets,
+                                    const int64_t* order,
+                                    const int64_t* radial_slot,
+                                    const float* inv_sqrt_deg,
+                                    const float* scale, float eps, float* y,
+                                    float* x_out, float* inverse_rms,
+                                    int64_t n_edges, int64_t n_nodes,
+                                    int64_t n_rows, int64_t n_radial,
+                                    int64_t channels, int32_t slot_info,
+                                    dpa4k_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * RMSNorm

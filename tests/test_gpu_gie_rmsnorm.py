@@ -417,3 +417,40 @@ def test_gie_shared_slot_kernels_skip_absent_outputs():
                 assert_bitwise(got, reference, f"partial outputs {need}")
             else:
                 assert got is None
+
+
+@pytest.mark.parametrize("lmax", [1, 2, 3, 4])
+@pytest.mark.parametrize("channels", [32, 64, 128])
+@pytest.mark.parametrize("shuffle", [False, True], ids=["sorted", "shuffled"])
+def test_gie_slot_per_degree(lmax, channels, shuffle):
+    """One radial slot per degree: the grouping's bit, the kernels that hold every row of a channel in one
+    lane (two nodes per wave at 32 channels: an odd node count and unequal degrees), off 16-byte
+    alignment, and fused with RMSNorm; each equal to the sequential oracle or the two operators bit for
+    bit.  A map that only resembles it (two rows swapped between degrees) must not take the bit."""
+    announce("gie slot per degree", lmax, channels, shuffle)
+    slots = [l - 1 for l in range(1, lmax + 1) for _ in range(2 * l + 1)]
+    inputs = _shared_slot_case(slots, lmax, channels, shuffle, seed=17 + lmax)
+    zonal, radial, dst, radial_slot, inverse = _to(inputs)
+    inverse = torch.cat([inverse, inverse.new_ones(1)])  # 49 nodes, the last without edges
+    offsets, order, info = _C.gie_group(dst, radial_slot, inverse.numel(), lmax)
+    assert info & 4
+    expected = gie_ref.zonal_scatter_reference(*inputs[:4], inverse.cpu())
+    shifted = torch.empty(radial.numel() + 1, device=DEV)[1:].copy_(radial.reshape(-1)).view(radial.shape)
+    for values in (radial, shifted):
+        out = _C.gie_zonal_scatter_forward_csr(zonal, values, offsets, order, radial_slot, inverse, info)
+        assert_bitwise(out, expected, "forward")
+    width = (len(slots) + 1) * channels
+    if _C.gie_rmsnorm_supported(len(slots), channels):
+        scale = (torch.rand(width, generator=torch.Generator().manual_seed(3)) + 0.5).to(DEV)
+        got = _C.gie_rmsnorm_forward_csr(zonal, radial, offsets, order, radial_slot, inverse, scale, 1e-6, True,
+                                         slot_info=info)
+        want = _C.gie_rmsnorm_forward_csr(zonal, radial, offsets, order, radial_slot, inverse, scale, 1e-6, True)
+        y, inverse_rms = _C.rmsnorm_forward(out.reshape(-1, width), scale, 1e-6)
+        for a, b, c, name in zip(got, want, (y.view(out.shape), out, inverse_rms), ("y", "x", "inverse_rms")):
+            assert_bitwise(a, b, f"fused {name}, slots known or not")
+            assert_bitwise(a, c, f"fused {name} vs the two operators")
+    if lmax > 1:
+        swapped = radial_slot.clone()
+        swapped[0], swapped[-1] = radial_slot[-1], radial_slot[0]
+        assert not _C.gie_group(dst, swapped, inverse.numel(), lmax)[2] & 4
+    assert not _C.gie_group(dst, radial_slot, inverse.numel(), lmax + 1)[2] & 4
