@@ -343,18 +343,20 @@ __global__ __launch_bounds__(kBlock) void segment_sum_staged_kernel(
 // the rows non-temporally (small grids, see the launcher).  Bound by the
 // streams of src and grad_src.  Rows of several chunks per lane used to run a
 // wave per segment, 2 rows in flight: 3,000 segments of 90 rows of 1,024
-// floats took 483 us, here 452; 512 such segments 139 us, here 84.
+// floats took 483 us, 449 with a workgroup per segment.
 template <int G, int CPL, int U, bool kOrdered, bool kStreamRows, bool kStreamGrads>
 __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
     const float* __restrict__ grad_out, const float* __restrict__ src,
     const int64_t* __restrict__ offsets, const float* __restrict__ edge_scale,
     const float* __restrict__ node_scale, const int64_t* __restrict__ order,
     float* __restrict__ grad_src, float* __restrict__ grad_edge_scale,
-    float* __restrict__ grad_node_scale, int64_t n_edges, int64_t n_nodes, int64_t channels) {
+    float* __restrict__ grad_node_scale, int64_t n_edges, int64_t n_nodes, int64_t channels, int shares) {
   constexpr int SG = kBlock / G;
   __shared__ float partial[SG];
-  const int64_t segment = block_index();
+  const int64_t unit = block_index();
+  const int64_t segment = shares == 1 ? unit : unit / shares;
   if (segment >= n_nodes) return;
+  const int share = static_cast<int>(unit - segment * shares);
   const int lane = threadIdx.x % G;
   const int group = threadIdx.x / G;
   int64_t column[CPL];
@@ -387,6 +389,11 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
 
   int64_t begin, end;
   segment_bounds(offsets, segment, n_edges, begin, end);
+  if (shares > 1) {  // this workgroup's share of the segment's rows
+    const int64_t degree = end - begin;
+    end = begin + degree * (share + 1) / shares;
+    begin = begin + degree * share / shares;
+  }
   float node_sum = 0.0f;
   for (int64_t base = begin + group; base < end; base += static_cast<int64_t>(SG) * U) {
     int64_t edge[U];
@@ -464,13 +471,30 @@ int launch_staged_forward(const float* src, const int64_t* offsets, const float*
   return launched("segment_sum_staged_kernel");
 }
 
+// Workgroups per segment: a segment's rows are cut into shares of about 32 KB
+// (by the mean degree), one workgroup each, so that the chip reads and writes
+// one narrow window of src and grad_src at a time.  With a workgroup per segment
+// of 360 KB the thousand segments in flight are as many places in memory, which
+// cost 20% of the bandwidth: 3,000 segments of 90 rows of 1,024 floats 449 ->
+// 365 us (6.1 TB/s; shares of 16 KB 381, of 64 KB 410), 512 such segments 85 ->
+// 68; 90 or 60 rows of 256 floats in two shares 374 -> @P256@; rows gathered through
+// an order 463 -> 452.  The sum of grad_node_scale keeps one workgroup.
+constexpr int64_t kShareBytes = 32768;
+int backward_shares(int64_t n_edges, int64_t n_nodes, int64_t channels, bool want_node) {
+  if (want_node) return 1;
+  const double bytes = static_cast<double>(n_edges) / static_cast<double>(n_nodes) * static_cast<double>(channels) * 4.0;
+  const double shares = bytes / static_cast<double>(kShareBytes) + 0.5;
+  return static_cast<int>(shares < 1.0 ? 1.0 : (shares > 64.0 ? 64.0 : shares));
+}
+
 template <int G, int CPL>
 int launch_wide_backward_g(const float* grad_out, const float* src, const int64_t* offsets,
                            const float* edge_scale, const float* node_scale, const int64_t* order,
                            float* grad_src, float* grad_edge_scale, float* grad_node_scale, int64_t n_edges,
                            int64_t n_nodes, int64_t channels, hipStream_t stream) {
   constexpr int U = CPL >= 8 ? 1 : 8 / CPL;  // 8 chunks of a row set in flight per lane
-  const dim3 grid = launch_grid(n_nodes, kBlock);
+  const int shares = backward_shares(n_edges, n_nodes, channels, grad_node_scale != nullptr);
+  const dim3 grid = launch_grid(n_nodes * shares, kBlock);
   // Gradient rows are stored non-temporally, and on small grids the rows loaded so (config 1: 11.4 ->
   // 10.6-10.9 us; on large ones it does not pay, config 1R: 1,846 -> 1,886-1,903 us), except rows of several
   // chunks per lane that do not end on cache lines (C = 331: 419 -> 390 us forward and backward; C = 77, one
@@ -480,7 +504,7 @@ int launch_wide_backward_g(const float* grad_out, const float* src, const int64_
 #define DPA4K_SUM_BWD_WIDE(ORD, NT, NTG)                                                                \
   segment_sum_backward_wide_kernel<G, CPL, U, ORD, NT, NTG><<<grid, kBlock, 0, stream>>>(                \
       grad_out, src, offsets, edge_scale, node_scale, order, grad_src, grad_edge_scale, grad_node_scale, \
-      n_edges, n_nodes, channels)
+      n_edges, n_nodes, channels, shares)
   if constexpr (CPL > 1) {
     if (shared_lines) {
       if (order != nullptr) DPA4K_SUM_BWD_WIDE(true, false, false); else DPA4K_SUM_BWD_WIDE(false, false, false);
