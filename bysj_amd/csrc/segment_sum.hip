@@ -477,7 +477,7 @@ int launch_staged_forward(const float* src, const int64_t* offsets, const float*
 // of 360 KB the thousand segments in flight are as many places in memory, which
 // cost 20% of the bandwidth: 3,000 segments of 90 rows of 1,024 floats 449 ->
 // 365 us (6.1 TB/s; shares of 16 KB 381, of 64 KB 410), 512 such segments 85 ->
-// 68; 90 or 60 rows of 256 floats in two shares 374 -> @P256@; rows gathered through
+// 68; 90 or 60 rows of 256 floats in two shares 374 -> 344; rows gathered through
 // an order 463 -> 452.  The sum of grad_node_scale keeps one workgroup.
 constexpr int64_t kShareBytes = 32768;
 int backward_shares(int64_t n_edges, int64_t n_nodes, int64_t channels, bool want_node) {

@@ -442,6 +442,38 @@ def test_segment_sum_any_width(channels, use_order, nodes):
         assert_bitwise(got, want, f"{name} off alignment")
 
 
+@pytest.mark.parametrize("channels,mean", [(255, 50), (256, 47), (331, 120), (576, 64), (1024, 20), (2048, 13), (256, 3000)])
+@pytest.mark.parametrize("use_order", [False, True])
+def test_segment_sum_backward_in_shares(channels, mean, use_order):
+    """Segments of 48 KB and more on average, whose backward cuts each into shares: empty ones, ones with
+    fewer rows than shares and long ones; the same bits as the undivided backward that the node-scale
+    gradient asks for, and within the bounds of the oracle and 64 bits."""
+    announce("segment_sum shares", channels, mean, use_order)
+    degrees = np.random.default_rng(mean).poisson(mean, 13).astype(np.int64)
+    degrees[:5] = [0, 1, 2, 3, 4 * mean + 1]
+    dst_sorted = torch.from_numpy(workloads.dst_from_degrees(degrees))
+    if use_order:
+        dst, order, offsets = _shuffled(dst_sorted, seed=5)
+    else:
+        dst, order, offsets = dst_sorted, None, ref.segment_offsets(dst_sorted, degrees.size)
+    gen = torch.Generator().manual_seed(channels)
+    src = torch.randn(dst.numel(), channels, generator=gen)
+    w = torch.rand(dst.numel(), generator=gen) + 0.5
+    s = torch.rand(degrees.size, generator=gen) + 0.5
+    g = torch.randn(degrees.size, channels, generator=gen)
+    x, wd, sd = (t.to(DEV).requires_grad_(True) for t in (src, w, s))
+    place = dst.to(DEV), offsets.to(DEV)
+    index = None if order is None else order.to(DEV)
+    whole = torch.autograd.grad(kernels.segment_sum(x, *place, wd, sd, order=index), (x, wd, sd), g.to(DEV))
+    shared = torch.autograd.grad(kernels.segment_sum(x, *place, wd, s.to(DEV), order=index), (x, wd), g.to(DEV))
+    e_src, e_w, _ = ref.segment_sum_backward_reference(g, src, dst, offsets, w, s)
+    _, t_w, _ = segment_sum_backward_f64(g, src, dst, degrees.size, w, s)
+    assert_bitwise(shared[0], e_src, "grad_src")
+    assert_gradient(shared[1], e_w, t_w, "grad_edge_scale")
+    for got, want, name in zip(shared, whole, ("grad_src", "grad_edge_scale")):
+        assert_bitwise(got, want, f"{name} in shares")
+
+
 def test_segment_sum_node_scale_shape_and_empty_edges_backward():
     announce("segment_sum bwd shapes")
     dst, offsets = _graph([2, 1, 3])
