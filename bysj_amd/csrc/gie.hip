@@ -723,18 +723,38 @@ __global__ __launch_bounds__(kBlock) void gie_rmsnorm_forward_kernel(
   if (lane == 0) inverse_rms[node] = inv_rms;
 }
 
+// Two of the backward kernels give a node to a workgroup of kNodeWaves waves,
+// which take its edges in turn, so that the chip reads and writes one narrow
+// window of the edge arrays at a time.  A wave per node kept thousands of
+// places in flight, which cost bandwidth.  With one, two, four and eight waves
+// per node, 90 edges each: DeepMD's map at lmax 3, 2.22M edges of 64 channels 826,
+// 800, 731 and 784 us; at lmax 4, 0.74M edges 396, 414, 346 and 483; distinct
+// slots at lmax 3, 0.37M edges 627, 623, 598 and 584.
+constexpr int kNodeWaves = 4;
+
+// The waves' partial sums of a node, in wave order.
+template <int N, typename T>
+__device__ __forceinline__ T node_total(const T (&partial)[N]) {
+  T sum = partial[0];
+#pragma unroll
+  for (int w = 1; w < N; ++w) sum = sum + partial[w];
+  return sum;
+}
+
 // Distinct slots: lane owns (slot s, chunk c) pairs q = s * row_chunks + c of
 // one edge's radial block; RC = row_chunks lanes share a slot (power of two).
 template <int V, int CPL, int RC, bool kOrdered>
-__global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
+__global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_distinct_kernel(
     const float* __restrict__ grad_output, const float* __restrict__ zonal,
     const float* __restrict__ radial, const int64_t* __restrict__ offsets,
     const int64_t* __restrict__ order, const int64_t* __restrict__ radial_slot,
     const float* __restrict__ inv, float* __restrict__ grad_zonal, float* __restrict__ grad_radial,
     float* __restrict__ grad_inv, int64_t n_edges, int64_t n_nodes, int64_t n_rows,
     int64_t n_radial, int64_t channels) {
-  const int64_t node = block_index() * kWaves + (threadIdx.x >> 6);
+  __shared__ double inv_sum[kNodeWaves];
+  const int64_t node = block_index();
   if (node >= n_nodes) return;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
   const int64_t chunks = n_radial * RC;
   const int64_t edge_stride = n_radial * channels;
@@ -744,7 +764,8 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
   // (kNoRow where the lane has no row), so the edge loop keeps no 64-bit
   // addresses in registers.
   uint32_t col_at[CPL], zon_at[CPL], out_at[CPL], gz_at[CPL];
-  fvec<V> g[CPL], pre[CPL];
+  fvec<V> g[CPL];
+  double pre[CPL][V];  // the row before inv, the wave's edges: in 64 bits, so that the split costs no accuracy
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
     const int64_t q = lane + 64 * j;
@@ -767,13 +788,13 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
       for (int i = 0; i < V; ++i) g[j].v[i] = 0.0f;
     }
 #pragma unroll
-    for (int i = 0; i < V; ++i) pre[j].v[i] = 0.0f;
+    for (int i = 0; i < V; ++i) pre[j][i] = 0.0;
   }
   const int64_t radial_bytes = edge_stride * 4, zonal_bytes = n_rows * 4;
 
   int64_t begin, end;
   segment_bounds(offsets, node, n_edges, begin, end);
-  for (int64_t slot = begin; slot < end; ++slot) {
+  for (int64_t slot = begin + wave; slot < end; slot += kNodeWaves) {
     const int64_t e = uniform_i64(edge_of<kOrdered>(order, slot, n_edges));
     if (kOrdered && e < 0) continue;
     const BufferView rv = buffer_view(radial + e * edge_stride, radial_bytes);
@@ -797,7 +818,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
       fvec<V> out;
 #pragma unroll
       for (int i = 0; i < V; ++i) {
-        pre[j].v[i] = pre[j].v[i] + z[j] * x[j].v[i];
+        pre[j][i] = __builtin_fma(static_cast<double>(z[j]), static_cast<double>(x[j].v[i]), pre[j][i]);
         const float h = g[j].v[i] * sc;
         dot = dot + h * x[j].v[i];
         out.v[i] = h * z[j];
@@ -808,13 +829,15 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
     }
   }
   if (grad_inv != nullptr) {
-    float total = 0.0f;
+    double total = 0.0;
 #pragma unroll
     for (int j = 0; j < CPL; ++j)
 #pragma unroll
-      for (int i = 0; i < V; ++i) total = total + g[j].v[i] * pre[j].v[i];
+      for (int i = 0; i < V; ++i) total = __builtin_fma(static_cast<double>(g[j].v[i]), pre[j][i], total);
     total = group_sum<64>(total);
-    if (lane == 0) grad_inv[node] = total;
+    if (lane == 0) inv_sum[wave] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) grad_inv[node] = static_cast<float>(node_total(inv_sum));
   }
 }
 
@@ -957,7 +980,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_shared_kernel(
 // C / 8 lanes serve one edge (lane c of the group owns channels [8 c, 8 c +
 // 8) of every slot: S * 8 radial values) and EW = 64 / RC edges are handled
 // side by side, every lane busy.  The node's upstream rows g[r + 1, :] sit in
-// LDS (each wave its own node's), and the wave walks the rows slot by slot,
+// LDS, shared by its waves, and a wave walks the rows slot by slot,
 // in ascending order within a slot, with no masked iterations:
 //   dot                   = sum_c g[r, c] radial[e, s(r), c]   (8 FMAs, RC-lane butterfly)
 //   grad_zonal[e, r]      = inv * dot                          (kept by lane r mod RC)
@@ -969,10 +992,14 @@ __global__ __launch_bounds__(kBlock) void gie_backward_shared_kernel(
 // gie_backward_shared_kernel's to the bit (same channel split, butterfly and
 // row order); grad_inv adds the same terms over another lane partition.
 // Needs C = 8 RC, n_rows <= ZR * RC and n_rows * C <= kEdgeLaneRowFloats.
-constexpr int kEdgeLaneRowFloats = 4096;  // upstream floats staged per wave (16 KB)
+// MI355X, 2.22M edges: 64 channels 3 slots 826 -> 731 us (one wave per node
+// before), 128 channels half the edges 828 -> 743; against
+// gie_backward_shared_kernel 32 channels 3 slots 458 -> 379, 2 slots 287 -> 241,
+// 64 channels one slot 246 -> 230.
+constexpr int kEdgeLaneRowFloats = 4096;  // upstream floats staged per workgroup (16 KB)
 
 template <int RC, int S, int ZR, bool kOrdered>
-__global__ __launch_bounds__(kBlock) void gie_backward_edge_lanes_kernel(
+__global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_edge_lanes_kernel(
     const float* __restrict__ grad_output, const float* __restrict__ zonal,
     const float* __restrict__ radial, const int64_t* __restrict__ offsets,
     const int64_t* __restrict__ order, const int64_t* __restrict__ radial_slot,
@@ -982,24 +1009,22 @@ __global__ __launch_bounds__(kBlock) void gie_backward_edge_lanes_kernel(
   constexpr int V = 8;
   constexpr int EW = 64 / RC;        // edges per wave step
   constexpr int UU = 2;              // wave steps whose loads go out together
-  extern __shared__ float staged[];  // [kWaves][rows * C]
+  extern __shared__ float g_rows[];  // [rows * C]: the node's upstream rows
+  __shared__ float inv_sum[kNodeWaves];
   const int wave = threadIdx.x >> 6;
-  const int64_t node = block_index() * kWaves + wave;
-  const bool live = node < n_nodes;
+  const int64_t node = block_index();
+  if (node >= n_nodes) return;
   const int lane = threadIdx.x & 63;
   const int u = lane / RC, c = lane % RC;
   const int rows = static_cast<int>(n_rows);
   const int64_t edge_stride = S * channels;
-  float* g_rows = staged + wave * rows * channels;
-  const float scale = live ? inv[node] : 0.0f;
+  const float scale = inv[node];
 
-  // the node's upstream rows 1..R into this wave's LDS
-  if (live) {
-    const float* src = grad_output + (node * (n_rows + 1) + 1) * channels;
-    for (int64_t q = lane; q < rows * channels / 4; q += 64) store_vec<4>(g_rows + 4 * q, load_vec<4>(src + 4 * q));
-  }
+  // the node's upstream rows 1..R into its LDS
+  const float* upstream = grad_output + (node * (n_rows + 1) + 1) * channels;
+  for (int64_t q = threadIdx.x; q < rows * channels / 4; q += kNodeWaves * 64)
+    store_vec<4>(g_rows + 4 * q, load_vec<4>(upstream + 4 * q));
   __syncthreads();
-  if (!live) return;
 
   // the rows in slot order: lane k holds the k-th row of the slot-major list; first[s] bounds slot s
   int slot_of_row = lane < rows ? static_cast<int>(radial_slot[lane]) : -1;
@@ -1025,7 +1050,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_edge_lanes_kernel(
   float inv_partial = 0.0f;
   int64_t begin, end;
   segment_bounds(offsets, node, n_edges, begin, end);
-  for (int64_t base = begin; base < end; base += UU * EW) {
+  for (int64_t base = begin + wave * (UU * EW); base < end; base += kNodeWaves * UU * EW) {
     int64_t e[UU];
     float x[UU][S][V], zq[UU][ZR];
 #pragma unroll
@@ -1110,7 +1135,9 @@ __global__ __launch_bounds__(kBlock) void gie_backward_edge_lanes_kernel(
   }
   if (grad_inv != nullptr) {
     const float total = group_sum<64>(inv_partial);
-    if (lane == 0) grad_inv[node] = total;
+    if (lane == 0) inv_sum[wave] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) grad_inv[node] = node_total(inv_sum);
   }
 }
 
@@ -1274,9 +1301,9 @@ int launch_distinct(int cpl, const float* grad_output, const float* zonal, const
                     const float* inv, float* grad_zonal, float* grad_radial, float* grad_inv,
                     int64_t n_edges, int64_t n_nodes, int64_t n_rows, int64_t n_radial,
                     int64_t channels, hipStream_t stream) {
-  const dim3 grid = launch_grid((n_nodes + kWaves - 1) / kWaves, kBlock);
+  const dim3 grid = launch_grid(n_nodes, kNodeWaves * 64);
 #define DPA4K_GIE_DIST(C)                                                                     \
-  gie_backward_distinct_kernel<V, C, RC, kOrdered><<<grid, kBlock, 0, stream>>>(             \
+  gie_backward_distinct_kernel<V, C, RC, kOrdered><<<grid, kNodeWaves * 64, 0, stream>>>(             \
       grad_output, zonal, radial, offsets, order, radial_slot, inv, grad_zonal, grad_radial,  \
       grad_inv, n_edges, n_nodes, n_rows, n_radial, channels)
   switch (cpl) {
@@ -1409,21 +1436,24 @@ int dispatch_edge_lanes(const float* grad_output, const float* zonal, const floa
                         const int64_t* order, const int64_t* radial_slot, const float* inv, float* grad_zonal,
                         float* grad_radial, float* grad_inv, int64_t n_edges, int64_t n_nodes, int64_t n_rows,
                         int64_t n_radial, int64_t channels, hipStream_t stream) {
-  const dim3 grid = launch_grid((n_nodes + kWaves - 1) / kWaves, kBlock);
-  const size_t lds = sizeof(float) * kWaves * static_cast<size_t>(n_rows * channels);
+  const dim3 grid = launch_grid(n_nodes, kNodeWaves * 64);
+  const size_t lds = sizeof(float) * static_cast<size_t>(n_rows * channels);
   const int rc = static_cast<int>(channels / 8);
   const int zr = n_rows <= 2 * rc ? 2 : 4;
 #define DPA4K_GIE_EDGE_LANES(RC, S, ZR)                                                                 \
-  gie_backward_edge_lanes_kernel<RC, S, ZR, kOrdered><<<grid, kBlock, lds, stream>>>(                  \
+  gie_backward_edge_lanes_kernel<RC, S, ZR, kOrdered><<<grid, kNodeWaves * 64, lds, stream>>>(         \
       grad_output, zonal, radial, offsets, order, radial_slot, inv, grad_zonal, grad_radial, grad_inv, \
       n_edges, n_nodes, n_rows, channels)
 #define DPA4K_GIE_EDGE_LANES_S(RC, ZR)            \
-  switch (n_radial) {                             \
+  switch (n_radial) {                               \
+    case 1: DPA4K_GIE_EDGE_LANES(RC, 1, ZR); break; \
     case 2: DPA4K_GIE_EDGE_LANES(RC, 2, ZR); break; \
     case 3: DPA4K_GIE_EDGE_LANES(RC, 3, ZR); break; \
     default: DPA4K_GIE_EDGE_LANES(RC, 4, ZR); break; \
   }
-  if (rc == 8) {
+  if (rc == 4) {
+    DPA4K_GIE_EDGE_LANES_S(4, 4)
+  } else if (rc == 8) {
     if (zr == 2) { DPA4K_GIE_EDGE_LANES_S(8, 2) } else { DPA4K_GIE_EDGE_LANES_S(8, 4) }
   } else {
     if (zr == 2) { DPA4K_GIE_EDGE_LANES_S(16, 2) } else { DPA4K_GIE_EDGE_LANES_S(16, 4) }
@@ -1562,8 +1592,8 @@ extern "C" int dpa4k_gie_zonal_scatter_backward_csr(
                                              n_rows, n_radial, channels, stream);
   }
   // Shared slots, a few of them: one lane group per edge, every lane busy.
-  if (vec4 && !(slot_info & kSlotsDistinct) && (channels == 64 || channels == 128) && n_radial >= 2 &&
-      n_radial <= 4 && n_rows <= 4 * (channels / 8) && n_rows * channels <= kEdgeLaneRowFloats)
+  if (vec4 && !(slot_info & kSlotsDistinct) && (channels == 32 || channels == 64 || channels == 128) &&
+      n_radial >= 1 && n_radial <= 4 && n_rows <= 4 * (channels / 8) && n_rows * channels <= kEdgeLaneRowFloats)
     return order != nullptr
                ? dispatch_edge_lanes<true>(grad_output, zonal, radial, offsets, order, radial_slot, inv_sqrt_deg,
                                            grad_zonal, grad_radial, grad_inv_sqrt_deg, n_edges, n_nodes, n_rows,

@@ -454,3 +454,30 @@ def test_gie_slot_per_degree(lmax, channels, shuffle):
         swapped[0], swapped[-1] = radial_slot[-1], radial_slot[0]
         assert not _C.gie_group(dst, swapped, inverse.numel(), lmax)[2] & 4
     assert not _C.gie_group(dst, radial_slot, inverse.numel(), lmax + 1)[2] & 4
+
+
+@pytest.mark.parametrize("slots,n_radial,channels", [
+    (_DEEPMD_SLOTS, 3, 32), ([0] * 3, 1, 32), ([0] * 16, 1, 32), ([1, 0], 4, 32), (_DEEPMD_SLOTS, 3, 64), ([0] * 3, 1, 64),
+    ([0] * 15, 1, 128), (list(range(15)), 15, 64), (list(range(24)), 24, 2)])
+@pytest.mark.parametrize("shuffle", [False, True], ids=["sorted", "shuffled"])
+def test_gie_backward_node_in_one_workgroup(slots, n_radial, channels, shuffle):
+    """The backward's waves share a node: degrees on both sides of what one wave, one step and one turn of
+    all waves take, at 32 channels, with one slot and with distinct slots; grad_inv sums over the waves."""
+    announce("gie backward waves", slots, n_radial, channels, shuffle)
+    degrees = torch.tensor([0, 1, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 0, 127, 128, 129, 301, 1])
+    generator = torch.Generator().manual_seed(channels + n_radial)
+    dst = torch.repeat_interleave(torch.arange(degrees.numel()), degrees)
+    zonal = torch.randn((dst.numel(), len(slots)), generator=generator)
+    radial = torch.randn((dst.numel(), n_radial, channels), generator=generator)
+    inverse = torch.rsqrt(degrees.to(torch.float32) + 1.0)
+    if shuffle:
+        dst = dst[torch.randperm(dst.numel(), generator=generator)]
+    inputs = zonal, radial, dst, torch.tensor(slots), inverse
+    up = torch.randn((degrees.numel(), len(slots) + 1, channels), generator=generator)
+    z, r, d, k, inv = _to(inputs)
+    leaves = [t.requires_grad_(True) for t in (z, r, inv)]
+    grads = torch.autograd.grad(kernels.zonal_scatter(z, r, d, k, inv), leaves, up.to(DEV))
+    oracle = gie_ref.zonal_scatter_backward_reference(up, *inputs)
+    truth = zonal_scatter_backward_f64(up, *inputs)
+    for label, actual, wanted, exact in zip(("zonal", "radial", "inverse"), grads, oracle, truth):
+        assert_gradient(actual, wanted, exact, f"grad {label}")
