@@ -1059,7 +1059,8 @@ __global__ __launch_bounds__(kThreads, 2) void finish_private_kernel(
 //           the status word.
 //
 // The group ranks with wave_match_ranks (the lanes of equal coarse digits
-// found through LDS words instead of one ballot per digit bit), the gather
+// found through LDS words instead of one ballot per digit bit; spans in order
+// already with ballots), the gather
 // with wave_ballot_ranks (one ballot per fine digit bit).  The gather is
 // instantiated for 64 or 128 fine digits and 1024 or 2048 tiles; the wider
 // instances hold more per thread and spill a few registers, still well ahead
@@ -1283,8 +1284,14 @@ __global__ __launch_bounds__(kThreads, 6) void tile_group_kernel(const int64_t* 
   const auto digit = [&](int r) { return (key[r] >> fine_bits) & digit_mask; };
   uint32_t rank[kScatterRounds];
   uint32_t* counter = wave_count + wave * kMaxBuckets;
-  wave_match_ranks<kDigitBits, kScatterRounds>(digit, ok, counter, tables.match.leader[wave],
-                                               tables.match.masks[wave], rank);
+  // Where the wave's span is in order already, its lanes mostly share a digit, and 64 lanes OR into one
+  // mask word one after the other: ballots instead (5.9M sorted keys: 36.1 -> 22.7 us; shuffled ones
+  // 24 with masks, 26 with ballots).  A span without elements counts as in order (three tiles: 12.3 -> 8.7).
+  if (__ballot(flags & kFlagUnsorted) != 0ull)
+    wave_match_ranks<kDigitBits, kScatterRounds>(digit, ok, counter, tables.match.leader[wave],
+                                                 tables.match.masks[wave], rank);
+  else
+    wave_ballot_ranks<kDigitBits, kScatterRounds>(digit, ok, counter, rank);
 #pragma unroll
   for (int r = 0; r < kScatterRounds; ++r) asm volatile("" : "+v"(key[r]));
   asm volatile("" : "+v"(ok));

@@ -119,6 +119,19 @@ def test_counting_sort_bucket_chunks(edges, nodes):
     _check_grouping_against_numpy(keys, nodes, f"chunks E={edges} N={nodes}")
 
 
+@pytest.mark.parametrize("edges,nodes", [(8193, 64), (3 * 8192 + 77, 300), (200_001, 65536), (600_000, 40_000)])
+@pytest.mark.parametrize("swap", [None, 0, 63, 1022, 1023, 1024, 8191, -2])
+def test_counting_sort_of_nearly_sorted_keys(edges, nodes, swap):
+    """Sorted keys but for one inverted pair, inside a wave's span of a tile, across two spans, two tiles
+    and at the end: spans in order are ranked another way than the others."""
+    announce("counting sort: nearly sorted", edges, nodes, swap)
+    keys = np.sort(workloads.rng(edges + nodes).integers(0, nodes, size=edges)).astype(np.int64)
+    if swap is not None:
+        at = swap % edges
+        keys[at], keys[at + 1] = nodes - 1, 0
+    _check_grouping_against_numpy(keys, nodes, f"nearly sorted E={edges} N={nodes} swap={swap}")
+
+
 @pytest.mark.parametrize("edges,nodes", [(16_777_217, 2**16), (2_000_000, 2**18)])
 def test_counting_sort_past_the_grouped_limits(edges, nodes):
     """Keys that the grouped path does not take: more tiles than it holds (2,048 tiles of 8,192 keys;
