@@ -141,6 +141,37 @@ def test_counting_sort_past_the_grouped_limits(edges, nodes):
     _check_grouping_against_numpy(keys, nodes, f"four-launch E={edges} N={nodes}")
 
 
+def test_grouping_flags_of_concurrent_calls():
+    """Each call reads its own flags: threads on their own streams, half of them with a key out of range."""
+    import threading
+
+    announce("counting sort: concurrent flags")
+    good = torch.from_numpy(workloads.rng(6).integers(0, 500, size=20_000).astype(np.int64)).to(DEV)
+    bad = good.clone()
+    bad[777] = 500
+    expected = torch.sort(good, stable=True).indices
+    torch.cuda.synchronize()
+    wrong = []
+
+    def calls(keys, in_range):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(40):
+                try:
+                    order, _ = kernels.group_by_source(keys, 500)
+                    if not in_range or not torch.equal(order, expected):
+                        wrong.append(in_range)
+                except ValueError:
+                    if in_range:
+                        wrong.append(in_range)
+
+    threads = [threading.Thread(target=calls, args=((good, True) if k % 2 else (bad, False))) for k in range(8)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert not wrong
+
+
 def test_group_by_key_async_status_and_capture():
     """The asynchronous build reports the status bits on the device, allocates nothing when given its
     buffers, and replays from a HIP graph with the same result as the synchronous call."""
