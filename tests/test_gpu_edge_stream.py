@@ -145,3 +145,32 @@ def test_edge_stream_refusals_and_empty_shapes():
     # a gate activation whose rows are all silu needs no gate tensor
     silu_rows = edge_stream.edge_stream_combine([(1.0, x)], activation="gate", gate_rows=[-1] * 4)
     assert_bitwise(silu_rows, edge_stream.edge_stream_combine([(1.0, x)], activation="silu"), "all rows silu")
+
+
+@pytest.mark.parametrize("channels", [3, 4, 5, 7, 8, 61, 63, 65])
+@pytest.mark.parametrize("activation", [None, "silu", "gate"])
+def test_edge_stream_chunks_off_alignment(channels, activation):
+    """Widths and bases off 16 bytes: the chunked kernel, whose last chunk repeats columns, against the
+    oracle and, bit for bit, against the single-float kernel that an aliased output takes."""
+    announce("edge stream off alignment", channels, activation)
+    g = torch.Generator().manual_seed(channels)
+    shape = (311, 4, channels)
+    acc = torch.randn(*shape, generator=g)
+    flat = torch.randn(2 * 311 * 4 * channels + 3, generator=g)
+    rows_apart = flat[1:1 + 311 * 4 * channels].view(*shape)
+    terms = [(1.0, acc), (0.5, rows_apart, torch.randn(311, 4, 1, generator=g)),
+             (-2.0, torch.randn(channels, generator=g), torch.randn(311, 1, channels, generator=g))]
+    rows, gate = ([-1, 0, 0, 1], torch.randn(311, 2, channels, generator=g)) if activation == "gate" else (None, None)
+    want = es_ref.edge_stream_combine_reference(terms, activation, gate, rows)
+    device = _to_device(terms)
+    storage = flat.to(DEV)
+    device[1] = (0.5, storage[1:1 + acc.numel()].view(*shape), device[1][2])
+    options = dict(activation=activation, gate=None if gate is None else gate.to(DEV), gate_rows=rows)
+    got = edge_stream.edge_stream_combine(device, **options)
+    if activation is None:
+        assert_bitwise(got, want, "float32 chain")
+    else:
+        assert_close_scaled(got, want, what=f"{activation} vs float32 chain")
+    off = torch.empty(acc.numel() + 1, device=DEV)[1:].view(*shape)
+    assert_bitwise(edge_stream.edge_stream_combine(device, out=off, **options), got, "output off alignment")
+    assert_bitwise(edge_stream.edge_stream_combine(device, out=device[0][1], **options), got, "in place")
