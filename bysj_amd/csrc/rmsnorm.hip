@@ -29,7 +29,8 @@ constexpr int64_t kRegisterMaxWidth = 64 * 16 * 4;  // widest row the register k
 // Column partials of dpa4k_rmsnorm_backward_noalloc: one row per workgroup of
 // the grad_scale backward (at most kPartialWaves / kWaves of them) of at most
 // kRegisterMaxWidth floats, the most the register kernels ever write
-// (DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES).  Every device the library runs on
+// (DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES); wider rows take no more shares than
+// fit.  Every device the library runs on
 // holds its own copy until the process ends.  Host code never uses this name
 // as an address: it reaches the array through the per-device pointer that
 // scratch_for_stream() obtains from hipGetSymbolAddress.
@@ -504,7 +505,7 @@ size_t backward_workspace_bytes(int64_t rows, int64_t width) {
 }
 
 // The backward with its column partials in `workspace` (checked against the size the
-// shape needs; only the register kernels with a scale gradient use it), or, with
+// shape needs; only a scale gradient uses it), or, with
 // `static_scratch`, in this device's `scratch` array.
 int rmsnorm_backward(const float* grad, const float* x, const float* scale, const float* inverse_rms,
                      float* grad_x, float* grad_scale, int64_t rows, int64_t width, void* workspace,
