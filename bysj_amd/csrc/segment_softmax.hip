@@ -1324,7 +1324,8 @@ __global__ __launch_bounds__(SW == 1 ? kBlock : SW * 64) void softmax_backward_s
         const double total = __builtin_fma(static_cast<double>(a0[v]), static_cast<double>(g0[v]),
                                            span_sum<LS, 64>(dot[v]));
         expect[v] = static_cast<float>(total);
-        rest[v] = static_cast<float>(total - static_cast<double>(expect[v]));
+        // no remainder of an infinite S, whose gradients stay infinities
+        rest[v] = __builtin_isfinite(expect[v]) ? static_cast<float>(total - static_cast<double>(expect[v])) : 0.0f;
       }
     };
     const auto add_products = [&](const float(&xs)[R][4], const float(&gs)[R][4], int tiles) {

@@ -711,6 +711,40 @@ def test_segment_softmax_slab_edges(channels, filler, use_order):
     assert_gradient(grads[2], e_gn, t_gn, "grad_null")
 
 
+@pytest.mark.parametrize("channels", [5, 64, 260])
+@pytest.mark.parametrize("use_order", [False, True])
+def test_segment_softmax_backward_with_an_infinite_sum(channels, use_order):
+    """Where sum(alpha * grad_alpha) of a column is infinite (an infinite upstream value here),
+    grad_logit is alpha * (grad_alpha - sum) in fp32 all the same: infinities, and NaN for inf - inf
+    only.  Segments that stay in registers and one (1,000 rows) that is streamed, at widths of the slab
+    kernels (the lane-group kernels of 1 to 4 and 8 channels compensate a streamed sum: NaN there)."""
+    announce("softmax infinite sum", channels, use_order)
+    sizes = [5, 40, 1000, 7]
+    dst, offsets = _graph(sizes)
+    order = None
+    if use_order:
+        dst, order, offsets = _shuffled(dst, 3)
+    gen = torch.Generator().manual_seed(channels)
+    edges = dst.numel()
+    logit, env = torch.randn(edges, channels, generator=gen), torch.rand(edges, generator=gen) + 0.5
+    upstream = torch.randn(edges, channels, generator=gen)
+    rows = [order[offsets[n]:offsets[n + 1]] if use_order else torch.arange(offsets[n], offsets[n + 1]) for n in range(4)]
+    upstream[rows[0][1], 1] = float("inf")
+    upstream[rows[2][77], 3] = float("-inf")
+    leaf = logit.to(DEV).requires_grad_(True)
+    alpha = kernels.segment_softmax(leaf, env.to(DEV), offsets.to(DEV), order=None if order is None else order.to(DEV))
+    grad, = torch.autograd.grad(alpha, leaf, upstream.to(DEV))
+    grad, alpha = grad.cpu(), alpha.detach().cpu()
+    expected = torch.empty_like(grad)
+    for r in rows:
+        total = (alpha[r].double() * upstream[r].double()).sum(0).float()
+        expected[r] = alpha[r] * (upstream[r] - total)
+    infinite = ~torch.isfinite(expected)
+    assert int(infinite.sum()) == 5 + 1000
+    assert_bitwise(grad[infinite], expected[infinite], "infinite gradients")
+    assert_close_scaled(grad[~infinite], expected[~infinite], what="the other columns")
+
+
 def test_segment_softmax_plan_lists_the_long_segments():
     from bysj_amd.kernels import _C
 
