@@ -29,15 +29,13 @@ constexpr int64_t kRegisterMaxWidth = 64 * 16 * 4;  // widest row the register k
 // Column partials of dpa4k_rmsnorm_backward_noalloc: one row per workgroup of
 // the grad_scale backward (at most kPartialWaves / kWaves of them) of at most
 // kRegisterMaxWidth floats, the most the register kernels ever write
-// (DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES); wider rows take no more shares than
-// fit.  Every device the library runs on
+// (DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES); wider rows do not use it.  Every device the library runs on
 // holds its own copy until the process ends.  Host code never uses this name
 // as an address: it reaches the array through the per-device pointer that
 // scratch_for_stream() obtains from hipGetSymbolAddress.
 static_assert(int64_t(kPartialWaves / kWaves) * kRegisterMaxWidth * 4 == DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES,
               "the header's scratch size must match the partial matrix bound");
-constexpr int64_t kScratchFloats = DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES / 4;
-__device__ __align__(256) float scratch[kScratchFloats];
+__device__ __align__(256) float scratch[DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES / 4];
 
 __device__ __forceinline__ float inverse_rms_of(float sum_squares, int64_t width, float eps) {
   return 1.0f / sqrtf(sum_squares / static_cast<float>(width) + eps);
@@ -352,20 +350,49 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_backward_wide_kernel(
   }
 }
 
-// grad_scale of wide rows: a thread per column and share of the rows (shares
-// along y), its rows summed in order, one row of the partial matrix per share.
-__global__ __launch_bounds__(kBlock) void rmsnorm_scale_columns_kernel(
-    const float* __restrict__ grad, const float* __restrict__ x,
-    const float* __restrict__ inverse_rms, float* __restrict__ partial, int64_t rows, int64_t per_share,
-    int64_t width) {
-  const int64_t col = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
-  if (col >= width) return;
-  const int64_t first = blockIdx.y * per_share;
-  const int64_t last = first + per_share < rows ? first + per_share : rows;
-  float sum = 0.0f;
-  for (int64_t row = first; row < last; ++row)
-    sum = sum + grad[row * width + col] * (x[row * width + col] * inverse_rms[row]);
-  partial[blockIdx.y * width + col] = sum;
+// grad_scale without a partial matrix, for rows that the register kernels do
+// not hold and for calls without a workspace: a workgroup per 32 columns, whose
+// kColumnGroups half waves take the rows in turn (128 bytes of one row per load,
+// four rows in flight each) and meet in LDS, added in group order.  The sums are
+// kept in 64 bits.  A thread per column over all rows took 2.5 ms for 6,000 rows
+// of 5,000 floats, this one 78 us; shares of the rows in a partial matrix took
+// 48 us, but needed memory that two overlapping calls would share.
+constexpr int kColumnGroups = 2 * kColumnWaves;
+
+__global__ __launch_bounds__(kColumnWaves * 64) void rmsnorm_scale_columns_kernel(
+    const float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ inverse_rms,
+    float* __restrict__ grad_scale, int64_t rows, int64_t width) {
+  constexpr int U = 4;
+  __shared__ double group_total[kColumnGroups][32];
+  const int lane = threadIdx.x & 31;
+  const int group = threadIdx.x >> 5;
+  const int64_t column = block_index() * 32 + lane;
+  const bool live = column < width;
+  double sum = 0.0;
+  if (live) {
+    int64_t row = group;
+    for (; row + (U - 1) * kColumnGroups < rows; row += U * kColumnGroups) {
+      float g[U], xv[U], inv[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t at = row + u * kColumnGroups;
+        g[u] = __builtin_nontemporal_load(grad + at * width + column);
+        xv[u] = __builtin_nontemporal_load(x + at * width + column);
+        inv[u] = inverse_rms[at];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) sum += static_cast<double>(g[u] * (xv[u] * inv[u]));
+    }
+    for (; row < rows; row += kColumnGroups)
+      sum += static_cast<double>(grad[row * width + column] * (x[row * width + column] * inverse_rms[row]));
+  }
+  group_total[group][lane] = sum;
+  __syncthreads();
+  if (group == 0 && live) {
+#pragma unroll
+    for (int k = 1; k < kColumnGroups; ++k) sum += group_total[k][lane];
+    grad_scale[column] = static_cast<float>(sum);
+  }
 }
 
 // The register kernels' shape for a row of `width` floats: chunks of V floats
@@ -449,17 +476,12 @@ int launch_backward(unsigned int grid, const float* grad, const float* x,
   return launched("rmsnorm_backward_kernel");
 }
 
-// Rows of the partial matrix that the scale gradient takes: the backward's
-// workgroups, or the shares of wide rows (at least 64 rows each, and no more
-// than `scratch` holds, so that both entry points add in the same order).
+// Rows of the partial matrix of the register kernels' scale gradient: the
+// backward's workgroups.
 unsigned int partial_blocks(int64_t rows, int64_t width) {
-  const RowShape shape = shape_for(width);
-  int64_t cap = kPartialWaves / kWaves;
-  int64_t wanted = (rows + 63) / 64;
-  if (fits_registers(width)) wanted = row_blocks(shape, 1, rows);
-  else cap = cap < kScratchFloats / width ? cap : kScratchFloats / width;
-  wanted = wanted > cap ? cap : wanted;
-  return static_cast<unsigned int>(wanted < 1 ? 1 : wanted);
+  const int64_t cap = kPartialWaves / kWaves;
+  const int64_t wanted = row_blocks(shape_for(width), 1, rows);
+  return static_cast<unsigned int>(wanted > cap ? cap : (wanted < 1 ? 1 : wanted));
 }
 
 // Device address of `scratch` on the device that runs `stream`, looked up once
@@ -500,12 +522,12 @@ int scratch_for_stream(hipStream_t stream, float*& out) {
 }
 
 size_t backward_workspace_bytes(int64_t rows, int64_t width) {
-  if (rows <= 0 || width <= 0) return 0;
+  if (rows <= 0 || width <= 0 || !fits_registers(width)) return 0;
   return round_up_256(static_cast<size_t>(partial_blocks(rows, width)) * static_cast<size_t>(width) * 4);
 }
 
 // The backward with its column partials in `workspace` (checked against the size the
-// shape needs; only a scale gradient uses it), or, with
+// shape needs; only the register kernels with a scale gradient use it), or, with
 // `static_scratch`, in this device's `scratch` array.
 int rmsnorm_backward(const float* grad, const float* x, const float* scale, const float* inverse_rms,
                      float* grad_x, float* grad_scale, int64_t rows, int64_t width, void* workspace,
@@ -514,7 +536,7 @@ int rmsnorm_backward(const float* grad, const float* x, const float* scale, cons
   if (width <= 0) return fail(DPA4K_EINVAL, "RMSNorm feature dimension must be positive");
   if (grad_scale != nullptr && scale == nullptr)
     return fail(DPA4K_EINVAL, "cannot compute a scale gradient when scale is omitted");
-  // the scale gradient takes one thread per column along one grid row
+  // the scale gradient of register rows takes its columns along one grid row
   if (grad_scale != nullptr && width > 4294967295LL / kBlock * kBlock)
     return fail(DPA4K_EINVAL, "RMSNorm scale gradient: feature dimension exceeds the launch limit");
   if (rows == 0) {
@@ -523,50 +545,46 @@ int rmsnorm_backward(const float* grad, const float* x, const float* scale, cons
   }
   if (grad == nullptr || x == nullptr || inverse_rms == nullptr || grad_x == nullptr)
     return fail(DPA4K_EINVAL, "RMSNorm backward: null pointer");
+  // Rows of more than 1,024 floats, unless whole aligned chunks, have always been
+  // accepted without a workspace (the header asks for one): the columns kernel takes these.
+  const size_t needed = backward_workspace_bytes(rows, width);
+  const bool chunked = width % 4 == 0 && aligned16(grad) && aligned16(x) && aligned16(grad_x) && aligned16(scale);
+  const bool short_workspace = !static_scratch && (workspace == nullptr || workspace_bytes < needed);
   const bool wide = !fits_registers(width);
+  const bool columns = grad_scale != nullptr && (wide || (short_workspace && width > 1024 && !chunked));
   if (wide) {
     const dim3 grid = launch_grid((rows + kWaves - 1) / kWaves, kBlock);
     rmsnorm_backward_wide_kernel<<<grid, kBlock, 0, stream>>>(grad, x, scale, inverse_rms, grad_x, rows, width);
     if (int s = launched("rmsnorm_backward_wide_kernel")) return s;
-    if (grad_scale == nullptr) return DPA4K_OK;
-  } else if (grad_scale == nullptr) {
+  } else if (grad_scale == nullptr || columns) {
     // the register kernel strides over rows: one row of blocks covers any count
     const RowShape shape = shape_for(width);
     const int64_t wanted = row_blocks(shape, 1, rows);
     const int64_t limit = row_block_limit(kBlock);
     const unsigned int grid = static_cast<unsigned int>(wanted < limit ? wanted : limit);
-    return launch_backward(grid, grad, x, scale, inverse_rms, grad_x, nullptr, rows, width, stream);
+    if (int s = launch_backward(grid, grad, x, scale, inverse_rms, grad_x, nullptr, rows, width, stream)) return s;
   }
-  unsigned int parts = partial_blocks(rows, width);
-  const size_t needed = backward_workspace_bytes(rows, width);
-  if (static_scratch && !(wide && parts == 1)) {
-    if (needed > static_cast<size_t>(DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES) + 256)
+  if (grad_scale == nullptr) return DPA4K_OK;
+  if (columns) {
+    rmsnorm_scale_columns_kernel<<<launch_grid((width + 31) / 32, kColumnWaves * 64), kColumnWaves * 64, 0, stream>>>(
+        grad, x, inverse_rms, grad_scale, rows, width);
+    return launched("rmsnorm_scale_columns_kernel");
+  }
+  if (static_scratch) {
+    if (needed > static_cast<size_t>(DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES))
       return fail(DPA4K_EINVAL,
                   "RMSNorm backward (no allocation): %zu bytes of column partials exceed the %d-byte scratch",
                   needed, DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES);
     float* address = nullptr;
     if (int s = scratch_for_stream(stream, address)) return s;
     workspace = address;
-    workspace_bytes = needed;  // the partials fit; only their size's rounding may not
+  } else if (short_workspace) {
+    return fail(DPA4K_EWORKSPACE, "RMSNorm backward: workspace of %zu bytes is smaller than %zu", workspace_bytes,
+                needed);
   }
-  if (workspace == nullptr || workspace_bytes < needed) {
-    if (!wide)
-      return fail(DPA4K_EWORKSPACE, "RMSNorm backward: workspace of %zu bytes is smaller than %zu",
-                  workspace_bytes, needed);
-    parts = 1;  // wide rows also run without a workspace, a thread per column over all rows
-  }
+  const unsigned int parts = partial_blocks(rows, width);
   float* partial = static_cast<float*>(workspace);
-  if (wide) {
-    const int64_t per_share = (rows + parts - 1) / parts;
-    float* target = parts > 1 ? partial : grad_scale;
-    rmsnorm_scale_columns_kernel<<<dim3(blocks_for(width, kBlock), parts), kBlock, 0, stream>>>(
-        grad, x, inverse_rms, target, rows, per_share, width);
-    if (int s = launched("rmsnorm_scale_columns_kernel")) return s;
-    if (parts == 1) return DPA4K_OK;
-  } else {
-    const int s = launch_backward(parts, grad, x, scale, inverse_rms, grad_x, partial, rows, width, stream);
-    if (s) return s;
-  }
+  if (int s = launch_backward(parts, grad, x, scale, inverse_rms, grad_x, partial, rows, width, stream)) return s;
   partial_columns_kernel<<<static_cast<unsigned int>((width + 63) / 64), kColumnWaves * 64, 0, stream>>>(
       partial, parts, width, grad_scale);
   return launched("partial_columns_kernel");

@@ -485,7 +485,11 @@ int dpa4k_rmsnorm_forward(const float* x, const float* scale, float* y,
  *   u = grad * scale;  grad_x = inv u - x inv^3 mean(x u)
  *   grad_scale[w] = sum_rows grad * x * inv      (if grad_scale != NULL)
  * grad_scale is reduced over rows in a fixed two-stage order (no atomics);
- * it needs workspace >= dpa4k_rmsnorm_backward_workspace_size(rows, W). */
+ * it needs workspace >= dpa4k_rmsnorm_backward_workspace_size(rows, W), which
+ * is 0 for W > 4096.  A missing or short workspace is DPA4K_EWORKSPACE, except
+ * for rows of more than 1024 floats that are not whole 16-byte chunks (W % 4
+ * != 0, or a base off 16 bytes): grad_scale is then summed by another kernel,
+ * which reads grad and x once more and rounds differently. */
 size_t dpa4k_rmsnorm_backward_workspace_size(int64_t rows, int64_t width);
 int dpa4k_rmsnorm_backward(const float* grad, const float* x,
                            const float* scale, const float* inverse_rms,
@@ -496,15 +500,15 @@ int dpa4k_rmsnorm_backward(const float* grad, const float* x,
 /* dpa4k_rmsnorm_backward without a workspace argument, for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.
- * It calls no hipMalloc/hipFree: the column partials of grad_scale live in a
- * library-owned static device array of DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES
- * (768 rows of at most 4096 floats, 12 MiB), one per device, held until the
- * process ends; its address is looked up once per device on the first call.
+ * It calls no hipMalloc/hipFree: the column partials of grad_scale (W <= 4096)
+ * live in a library-owned static device array of
+ * DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES (768 rows of at most 4096 floats, 12
+ * MiB), one per device, held until the process ends; wider rows have none; its address is looked up once per device on the first call.
  * Same kernels as dpa4k_rmsnorm_backward, so the results are the same bit
  * for bit.  Every row of partials a call uses is written before it is read:
- * nothing needs clearing between calls.  Calls that overlap on one device
- * (concurrent streams or threads) race on the array and must be serialised
- * by the caller.  Returns DPA4K_EINVAL if a shape would need more partials
+ * nothing needs clearing between calls.  Calls with a grad_scale and W <= 4096
+ * that overlap on one device (concurrent streams or threads) race on the array
+ * and must be serialised by the caller.  Returns DPA4K_EINVAL if a shape would need more partials
  * than the array holds (no shape the kernels accept does). */
 #define DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES 12582912
 int dpa4k_rmsnorm_backward_noalloc(const float* grad, const float* x,

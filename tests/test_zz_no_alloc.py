@@ -86,6 +86,53 @@ def test_noalloc_backward_of_streamed_rows(rows, width):
     assert_bitwise(got_scale, want_scale, "grad_scale")
 
 
+@pytest.mark.parametrize("rows,width", [(700, 5003), (1, 4097), (129, 8192)])
+def test_streamed_rows_share_no_memory(rows, width):
+    """Rows past 4,096 floats use neither workspace nor scratch: the scale gradient is the same bit for bit with any
+    workspace or none, and calls of the no-allocation form that overlap on two streams do not disturb each other."""
+    library = _lib.load()
+    announce("rmsnorm backward, streamed rows, two streams", rows, width)
+    assert library.dpa4k_rmsnorm_backward_workspace_size(rows, width) == 0
+    cases = [_inputs(rows, width, seed=s) for s in (1, 2)]
+    want = [_with_workspace(library, *case) for case in cases]
+    for (grad, x, scale, _), (_, got) in zip(cases, want):
+        _, truth = rmsnorm_backward_f64(grad, x, scale, 1e-6)
+        assert_close_scaled(got, truth, what="grad_scale vs fp64 closed form")
+    streams = [torch.cuda.Stream(DEV) for _ in cases]
+    torch.cuda.synchronize()
+    got = [(torch.empty_like(x), torch.empty_like(scale)) for _, x, scale, _ in cases]
+    for _ in range(8):
+        for stream, (grad, x, scale, inverse_rms), (grad_x, grad_scale) in zip(streams, cases, got):
+            _lib.check(library.dpa4k_rmsnorm_backward_noalloc(
+                grad.data_ptr(), x.data_ptr(), scale.data_ptr(), inverse_rms.data_ptr(), grad_x.data_ptr(),
+                grad_scale.data_ptr(), rows, width, stream.cuda_stream))
+    torch.cuda.synchronize()
+    for (got_x, got_scale), (want_x, want_scale) in zip(got, want):
+        assert_bitwise(got_x, want_x, "grad_x")
+        assert_bitwise(got_scale, want_scale, "grad_scale")
+
+
+@pytest.mark.parametrize("rows,width,offset", [(300, 2777, 0), (70, 2048, 1), (3, 1025, 3)])
+def test_backward_without_a_workspace_where_it_is_accepted(rows, width, offset):
+    """Rows of more than 1,024 floats that are not whole aligned chunks run without a workspace; others are refused."""
+    library = _lib.load()
+    announce("rmsnorm backward without a workspace", rows, width, offset)
+    grad, x, scale, inverse_rms = _inputs(rows, width, seed=rows, offset=offset)
+    stream = torch.cuda.current_stream().cuda_stream
+    grad_x, grad_scale = torch.empty_like(x), torch.empty_like(scale)
+
+    def call(rows, width, grad, x, grad_x):
+        return library.dpa4k_rmsnorm_backward(grad.data_ptr(), x.data_ptr(), scale.data_ptr(),
+                                              inverse_rms.data_ptr(), grad_x.data_ptr(), grad_scale.data_ptr(),
+                                              rows, width, None, 0, stream)
+
+    _lib.check(call(rows, width, grad, x, grad_x))
+    truth_x, truth_scale = rmsnorm_backward_f64(grad, x, scale, 1e-6)
+    assert_close_scaled(grad_x, truth_x, what="grad_x vs fp64 closed form")
+    assert_close_scaled(grad_scale, truth_scale, what="grad_scale vs fp64 closed form")
+    assert call(1, 1024, grad.clone(), x.clone(), grad_x.clone()) == _lib.EWORKSPACE
+
+
 def test_noalloc_backward_without_scale_gradient_and_empty_rows():
     library = _lib.load()
     announce("rmsnorm backward noalloc: no scale gradient, zero rows")
