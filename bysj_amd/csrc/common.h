@@ -325,6 +325,18 @@ __device__ __forceinline__ void store_chunk_stream(float* __restrict__ p, const 
   __builtin_nontemporal_store(raw, reinterpret_cast<f32x4u*>(p));
 }
 
+// A row's last chunk without the `skip` columns it repeats, where the output
+// may lie on an input that the neighbour's lane still reads.
+__device__ __forceinline__ void store_own(float* __restrict__ p, const fvec<4>& value, int skip) {
+  if (skip == 0) {
+    store_chunk(p, value);
+    return;
+  }
+#pragma unroll
+  for (int i = 1; i < 4; ++i)
+    if (i >= skip) p[i] = value.v[i];
+}
+
 // ---------------------------------------------------------------------------
 // Device: buffer views
 // ---------------------------------------------------------------------------

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_forward_wide_kernel(
       out.v[i] = value.v[i] * inv;
       if (scale != nullptr) out.v[i] = out.v[i] * s.v[i];
     }
-    store_chunk(yr + column, out);
+    store_own(yr + column, out, static_cast<int>(c - column));  // y may be x
   }
   if (lane == 0) inverse_rms[row] = inv;
 }
@@ -346,7 +346,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_backward_wide_kernel(
       const float u = scale != nullptr ? g.v[i] * s.v[i] : g.v[i];
       out.v[i] = inv * u - xv.v[i] * inv3 * mean_dot;
     }
-    store_chunk(grad_x + row * width + column, out);
+    store_own(grad_x + row * width + column, out, static_cast<int>(c - column));  // grad_x may be grad or x
   }
 }
 
@@ -552,23 +552,23 @@ int rmsnorm_backward(const float* grad, const float* x, const float* scale, cons
   const bool short_workspace = !static_scratch && (workspace == nullptr || workspace_bytes < needed);
   const bool wide = !fits_registers(width);
   const bool columns = grad_scale != nullptr && (wide || (short_workspace && width > 1024 && !chunked));
+  if (columns) {  // first: grad_x may be grad or x
+    rmsnorm_scale_columns_kernel<<<launch_grid((width + 31) / 32, kColumnWaves * 64), kColumnWaves * 64, 0, stream>>>(
+        grad, x, inverse_rms, grad_scale, rows, width);
+    if (int s = launched("rmsnorm_scale_columns_kernel")) return s;
+  }
   if (wide) {
     const dim3 grid = launch_grid((rows + kWaves - 1) / kWaves, kBlock);
     rmsnorm_backward_wide_kernel<<<grid, kBlock, 0, stream>>>(grad, x, scale, inverse_rms, grad_x, rows, width);
-    if (int s = launched("rmsnorm_backward_wide_kernel")) return s;
-  } else if (grad_scale == nullptr || columns) {
+    return launched("rmsnorm_backward_wide_kernel");
+  }
+  if (grad_scale == nullptr || columns) {
     // the register kernel strides over rows: one row of blocks covers any count
     const RowShape shape = shape_for(width);
     const int64_t wanted = row_blocks(shape, 1, rows);
     const int64_t limit = row_block_limit(kBlock);
     const unsigned int grid = static_cast<unsigned int>(wanted < limit ? wanted : limit);
-    if (int s = launch_backward(grid, grad, x, scale, inverse_rms, grad_x, nullptr, rows, width, stream)) return s;
-  }
-  if (grad_scale == nullptr) return DPA4K_OK;
-  if (columns) {
-    rmsnorm_scale_columns_kernel<<<launch_grid((width + 31) / 32, kColumnWaves * 64), kColumnWaves * 64, 0, stream>>>(
-        grad, x, inverse_rms, grad_scale, rows, width);
-    return launched("rmsnorm_scale_columns_kernel");
+    return launch_backward(grid, grad, x, scale, inverse_rms, grad_x, nullptr, rows, width, stream);
   }
   if (static_scratch) {
     if (needed > static_cast<size_t>(DPA4K_RMSNORM_NOALLOC_SCRATCH_BYTES))

@@ -987,6 +987,9 @@ __global__ __launch_bounds__(kBlock) void softmax_backward_kernel(BackwardArgs a
 // Any C >= 4 and any 4-byte alignment: the row's last chunk starts at column
 // C - 4, so it repeats up to three columns of its neighbour, which compute and
 // store the same bits in both lanes and are left out of the row sums (`skip`).
+// Where outputs lie on inputs, both lanes must be of one wave, which loads a
+// row before it stores it: a row whose last chunk would be alone in its slab is
+// then cut `shift` chunks earlier (slab_shift).
 //
 // Bound by the row streams: C = 256 over 741k edges of 8,192 segments takes
 // 274 us forward (5.6 TB/s) and 380 us backward (6.0), where staging whole rows
@@ -1122,7 +1125,7 @@ __device__ __forceinline__ void slab_forward_stores(const ForwardArgs& a, const 
 }
 
 template <int LOG_LS, int R, typename Id>
-__global__ __launch_bounds__(kBlock) void softmax_forward_slab_kernel(ForwardArgs a, int64_t slabs) {
+__global__ __launch_bounds__(kBlock) void softmax_forward_slab_kernel(ForwardArgs a, int64_t slabs, int shift) {
   using T = SlabRows<LOG_LS, R, Id>;
   constexpr int LS = T::LS, PR = T::PR, CAP = T::CAP;
   const int64_t unit = uniform_i64(block_index() * kWaves + (threadIdx.x >> 6));
@@ -1130,8 +1133,8 @@ __global__ __launch_bounds__(kBlock) void softmax_forward_slab_kernel(ForwardArg
   if (segment >= a.n_nodes) return;
   const int64_t slab = unit - segment * slabs;
   const int lane = threadIdx.x & 63;
-  const int64_t chunk = slab * LS + (lane & (LS - 1));
-  const bool live = chunk * 4 < a.channels;
+  const int64_t chunk = slab * LS + (lane & (LS - 1)) - shift;
+  const bool live = chunk >= 0 && chunk * 4 < a.channels;
   const int64_t column = live ? (chunk * 4 + 4 <= a.channels ? chunk * 4 : a.channels - 4) : 0;
   const bool has_null = a.null_logit != nullptr;
   int64_t begin, end;
@@ -1290,8 +1293,8 @@ __device__ __forceinline__ void slab_backward_loads(const BackwardArgs& a, SlabR
 // SW waves share a segment (SW > 1), or every wave has a segment of its own
 // (SW = 1, rows of one slab).
 template <int LOG_LS, int R, int SW, typename Id>
-__global__ __launch_bounds__(SW == 1 ? kBlock : SW * 64) void softmax_backward_slab_kernel(BackwardArgs a,
-                                                                                         int64_t slabs) {
+__global__ __launch_bounds__(SW == 1 ? kBlock : SW * 64) void softmax_backward_slab_kernel(
+    BackwardArgs a, int64_t slabs, int shift) {
   using T = SlabRows<LOG_LS, R, Id>;
   constexpr int LS = T::LS, PR = T::PR, CAP = T::CAP;
   constexpr int kSegments = SW == 1 ? kWaves : 1;  // segments per workgroup
@@ -1308,8 +1311,8 @@ __global__ __launch_bounds__(SW == 1 ? kBlock : SW * 64) void softmax_backward_s
   segment_bounds(a.offsets, segment, a.n_edges, begin, end);
 
   for (int64_t round = 0; round < slabs; round += SW) {
-    const int64_t chunk = (round + part) * LS + (lane & (LS - 1));
-    const bool live = chunk * 4 < a.channels;
+    const int64_t chunk = (round + part) * LS + (lane & (LS - 1)) - shift;
+    const bool live = chunk >= 0 && chunk * 4 < a.channels;
     const int64_t column = live ? (chunk * 4 + 4 <= a.channels ? chunk * 4 : a.channels - 4) : 0;
     const int skip = live ? static_cast<int>(chunk * 4 - column) : 4;  // columns a neighbour accounts for
     const bool last = round + SW >= slabs;
@@ -1597,66 +1600,86 @@ RowIds row_ids(const int64_t* order, int64_t n_edges, int64_t channels) {
 int slab_lanes_log(int64_t channels) { return channels <= 8 ? 1 : (channels <= 16 ? 2 : 3); }
 
 template <int LOG_LS, typename Id>
-int launch_forward_slabs(const ForwardArgs& a, int rows, int64_t slabs, hipStream_t stream) {
+int launch_forward_slabs(const ForwardArgs& a, int rows, int64_t slabs, int shift, hipStream_t stream) {
   constexpr int PR = 64 >> LOG_LS;
   const dim3 grid = launch_grid((a.n_nodes * slabs + kWaves - 1) / kWaves, kBlock);
   if constexpr (!__is_same(Id, int64_t)) {
-    if (rows == 64) softmax_forward_slab_kernel<LOG_LS, 64 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs);
-    if (rows == 96) softmax_forward_slab_kernel<LOG_LS, 96 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs);
+    if (rows == 64) softmax_forward_slab_kernel<LOG_LS, 64 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
+    if (rows == 96) softmax_forward_slab_kernel<LOG_LS, 96 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
     if (rows != 128) return launched("softmax_forward_slab_kernel");
   }
-  softmax_forward_slab_kernel<LOG_LS, 128 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs);
+  softmax_forward_slab_kernel<LOG_LS, 128 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
   return launched("softmax_forward_slab_kernel");
 }
 
 template <int LOG_LS, int SW, typename Id>
-int launch_backward_slabs_of(const BackwardArgs& a, int rows, int64_t slabs, hipStream_t stream) {
+int launch_backward_slabs_of(const BackwardArgs& a, int rows, int64_t slabs, int shift, hipStream_t stream) {
   constexpr int PR = 64 >> LOG_LS;
   constexpr int kThreads = SW == 1 ? kBlock : SW * 64;
   const dim3 grid = launch_grid(SW == 1 ? (a.n_nodes + kWaves - 1) / kWaves : a.n_nodes, kThreads);
   if constexpr (!__is_same(Id, int64_t)) {
-    if (rows == 64) softmax_backward_slab_kernel<LOG_LS, 64 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs);
-    if (rows == 96) softmax_backward_slab_kernel<LOG_LS, 96 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs);
+    if (rows == 64) softmax_backward_slab_kernel<LOG_LS, 64 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
+    if (rows == 96) softmax_backward_slab_kernel<LOG_LS, 96 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
     if (rows != 128) return launched("softmax_backward_slab_kernel");
   }
-  softmax_backward_slab_kernel<LOG_LS, 128 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs);
+  softmax_backward_slab_kernel<LOG_LS, 128 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
   return launched("softmax_backward_slab_kernel");
 }
 
 template <int LOG_LS, typename Id>
-int launch_backward_slabs(const BackwardArgs& a, int rows, int64_t slabs, hipStream_t stream) {
+int launch_backward_slabs(const BackwardArgs& a, int rows, int64_t slabs, int shift, hipStream_t stream) {
   if constexpr (LOG_LS == 3) {
-    if (slabs > 4) return launch_backward_slabs_of<LOG_LS, kSlabWaves, Id>(a, rows, slabs, stream);
-    if (slabs > 2) return launch_backward_slabs_of<LOG_LS, 4, Id>(a, rows, slabs, stream);
-    if (slabs > 1) return launch_backward_slabs_of<LOG_LS, 2, Id>(a, rows, slabs, stream);
+    if (slabs > 4) return launch_backward_slabs_of<LOG_LS, kSlabWaves, Id>(a, rows, slabs, shift, stream);
+    if (slabs > 2) return launch_backward_slabs_of<LOG_LS, 4, Id>(a, rows, slabs, shift, stream);
+    if (slabs > 1) return launch_backward_slabs_of<LOG_LS, 2, Id>(a, rows, slabs, shift, stream);
   }
-  return launch_backward_slabs_of<LOG_LS, 1, Id>(a, rows, slabs, stream);
+  return launch_backward_slabs_of<LOG_LS, 1, Id>(a, rows, slabs, shift, stream);
 }
 
 #define DPA4K_SLABS(LAUNCH, ID)                                                         \
-  (log_ls == 1 ? LAUNCH<1, ID>(a, rows, slabs, stream)                                   \
-               : (log_ls == 2 ? LAUNCH<2, ID>(a, rows, slabs, stream) : LAUNCH<3, ID>(a, rows, slabs, stream)))
+  (log_ls == 1 ? LAUNCH<1, ID>(a, rows, slabs, shift, stream)                                   \
+               : (log_ls == 2 ? LAUNCH<2, ID>(a, rows, slabs, shift, stream) : LAUNCH<3, ID>(a, rows, slabs, shift, stream)))
+
+// Whether [a, a + floats) and [b, b + floats) share memory.
+bool overlap(const float* a, const float* b, int64_t floats) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  const uintptr_t bytes = static_cast<uintptr_t>(floats) * 4u;
+  return a != nullptr && b != nullptr && x < y + bytes && y < x + bytes;
+}
+
+// Chunks by which the slabs of a call in place start early: half a slab where the last chunk repeats columns of the
+// slab before it.
+int slab_shift(int64_t channels, bool in_place) {
+  return in_place && channels > 32 && channels % 32 >= 1 && channels % 32 <= 3 ? 4 : 0;
+}
 
 int forward_slabs(const ForwardArgs& a, hipStream_t stream) {
+  const int shift = slab_shift(a.channels, overlap(a.alpha, a.logit, a.n_edges * a.channels) ||
+                                               overlap(a.null_alpha, a.null_logit, a.n_nodes * a.channels));
   const int log_ls = slab_lanes_log(a.channels);
-  const int64_t slabs = ((a.channels + 3) / 4 + (1 << log_ls) - 1) >> log_ls;
+  const int64_t slabs = ((a.channels + 3) / 4 + shift + (1 << log_ls) - 1) >> log_ls;
   const int rows = slab_rows(a.n_edges, a.n_nodes);
   if (!grid_fits(a.n_nodes * slabs, kBlock)) return fail(DPA4K_EINVAL, "segment softmax: grid too large");
   switch (row_ids(a.order, a.n_edges, a.channels)) {
     case RowIds::kViews: return DPA4K_SLABS(launch_forward_slabs, Views);
-    case RowIds::kSharedViews: return launch_forward_slabs<3, SharedViews>(a, rows, slabs, stream);
+    case RowIds::kSharedViews: return launch_forward_slabs<3, SharedViews>(a, rows, slabs, shift, stream);
     case RowIds::kNarrow: return DPA4K_SLABS(launch_forward_slabs, uint32_t);
     default: return DPA4K_SLABS(launch_forward_slabs, int64_t);
   }
 }
 
 int backward_slabs(const BackwardArgs& a, hipStream_t stream) {
+  const int64_t elements = a.n_edges * a.channels, null_elements = a.n_nodes * a.channels;
+  const int shift =
+      slab_shift(a.channels, overlap(a.grad_logit, a.grad_alpha, elements) || overlap(a.grad_logit, a.alpha, elements) ||
+                                 overlap(a.grad_null_logit, a.grad_null_alpha, null_elements) ||
+                                 overlap(a.grad_null_logit, a.null_alpha, null_elements));
   const int log_ls = slab_lanes_log(a.channels);
-  const int64_t slabs = ((a.channels + 3) / 4 + (1 << log_ls) - 1) >> log_ls;
+  const int64_t slabs = ((a.channels + 3) / 4 + shift + (1 << log_ls) - 1) >> log_ls;
   const int rows = slab_rows(a.n_edges, a.n_nodes);
   switch (row_ids(a.order, a.n_edges, a.channels)) {
     case RowIds::kViews: return DPA4K_SLABS(launch_backward_slabs, Views);
-    case RowIds::kSharedViews: return launch_backward_slabs<3, SharedViews>(a, rows, slabs, stream);
+    case RowIds::kSharedViews: return launch_backward_slabs<3, SharedViews>(a, rows, slabs, shift, stream);
     case RowIds::kNarrow: return DPA4K_SLABS(launch_backward_slabs, uint32_t);
     default: return DPA4K_SLABS(launch_backward_slabs, int64_t);
   }

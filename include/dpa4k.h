@@ -16,6 +16,8 @@
  *  - The library never allocates device memory.  Functions that need scratch
  *    memory take a caller-provided workspace and have a *_workspace_size
  *    query.
+ *  - Outputs overlap neither inputs nor each other, unless an entry point says
+ *    which arrays may be the same (element for element).
  *  - Return value: DPA4K_OK (0) on success, otherwise an error code; the
  *    message of the last error raised on the calling thread is returned by
  *    dpa4k_last_error().  No C++ exception crosses this boundary.
@@ -150,7 +152,8 @@ int dpa4k_segment_sum_backward(const float* grad_out, const float* src,
  * Evaluated in base 2 with the hardware exp2/log2/reciprocal (relative error
  * below 1e-6 against the natural-base chain).
  * logit[E, C], env[E], null_logit[N, C] or NULL, order[E] or NULL,
- * alpha[E, C], null_alpha[N, C] (required iff null_logit is given). */
+ * alpha[E, C], null_alpha[N, C] (required iff null_logit is given).  alpha may
+ * be the logit array and null_alpha the null_logit array. */
 int dpa4k_segment_softmax_forward(const float* logit, const float* env,
                                   const int64_t* offsets, const float* null_logit,
                                   const int64_t* order, float* alpha,
@@ -162,7 +165,9 @@ int dpa4k_segment_softmax_forward(const float* logit, const float* env,
  *   S = sum_e alpha * grad_alpha + null_alpha * grad_null_alpha
  *   grad_logit = alpha (grad_alpha - S); grad_null_logit = null_alpha (grad_null_alpha - S)
  *   grad_env[e] = (sum_c grad_logit[e, c]) * 2 / env[e]  (0 where !(env > 0))
- * null_alpha, grad_null_alpha and grad_null_logit are all given or all NULL. */
+ * null_alpha, grad_null_alpha and grad_null_logit are all given or all NULL.
+ * grad_logit may be the alpha or the grad_alpha array, grad_null_logit the
+ * null_alpha or the grad_null_alpha array. */
 int dpa4k_segment_softmax_backward(const float* alpha, const float* grad_alpha,
                                    const float* env, const int64_t* offsets,
                                    const float* null_alpha,
@@ -476,7 +481,7 @@ int dpa4k_gie_rmsnorm_forward_slots(const float* zonal, const float* radial,
 /* Replaces rmsnorm_forward_hip (csrc/rmsnorm.cpp:99).
  * y = x * (1 / sqrt(mean(x^2) + eps)) * scale over rows of width W.
  * x[rows, W], scale[W] or NULL, y[rows, W], inverse_rms[rows].  W >= 1,
- * eps finite and > 0. */
+ * eps finite and > 0.  y may be the x array. */
 int dpa4k_rmsnorm_forward(const float* x, const float* scale, float* y,
                           float* inverse_rms, int64_t rows, int64_t width,
                           float eps, dpa4k_stream_t stream);
@@ -484,6 +489,7 @@ int dpa4k_rmsnorm_forward(const float* x, const float* scale, float* y,
 /* Replaces rmsnorm_backward_hip (csrc/rmsnorm.cpp:123).
  *   u = grad * scale;  grad_x = inv u - x inv^3 mean(x u)
  *   grad_scale[w] = sum_rows grad * x * inv      (if grad_scale != NULL)
+ * grad_x may be the grad or the x array.
  * grad_scale is reduced over rows in a fixed two-stage order (no atomics);
  * it needs workspace >= dpa4k_rmsnorm_backward_workspace_size(rows, W), which
  * is 0 for W > 4096.  A missing or short workspace is DPA4K_EWORKSPACE, except

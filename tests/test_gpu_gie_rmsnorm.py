@@ -11,7 +11,7 @@ import pytest
 import torch
 
 from bysj_amd import kernels, workloads
-from bysj_amd.kernels import _C
+from bysj_amd.kernels import _C, _lib
 from oracle import gie as gie_ref
 from oracle import loops
 from oracle.rmsnorm import rmsnorm as reference_rmsnorm
@@ -220,6 +220,41 @@ def test_rmsnorm_zero_input_no_scale_and_stream():
     e_x, _ = rmsnorm_backward_reference(torch.ones(9, 131), xs, None, 1e-6)
     t_x, _ = rmsnorm_backward_f64(torch.ones(9, 131), xs, None, 1e-6)
     assert_gradient(grad_x, e_x, t_x, "grad_x without scale")
+
+
+@pytest.mark.parametrize("width", [3, 66, 1001, 4096, 4097, 4610, 5000])
+def test_rmsnorm_in_place(width):
+    """C ABI: y on x and grad_x on grad or x give the bits of separate arrays (W mod 256 of 1 to 3 past 4,096: the last
+    chunk repeats columns that the wave's previous step wrote)."""
+    announce("rmsnorm in place", width)
+    library, rows, stream = _lib.load(), 37, torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device=DEV).manual_seed(width)
+    x, up = (torch.randn(rows, width, generator=gen, device=DEV) for _ in range(2))
+    scale, inv = torch.rand(width, generator=gen, device=DEV) + 0.5, torch.empty(rows, device=DEV)
+    size = library.dpa4k_rmsnorm_backward_workspace_size(rows, width)
+    workspace = torch.empty(max(size, 1), dtype=torch.uint8, device=DEV)
+
+    def forward(a, y):
+        _lib.check(library.dpa4k_rmsnorm_forward(a.data_ptr(), scale.data_ptr(), y.data_ptr(), inv.data_ptr(), rows,
+                                                 width, 1e-6, stream))
+
+    def backward(g, a, out):
+        grad_scale = torch.empty(width, device=DEV)
+        _lib.check(library.dpa4k_rmsnorm_backward(g.data_ptr(), a.data_ptr(), scale.data_ptr(), inv.data_ptr(),
+                                                  out.data_ptr(), grad_scale.data_ptr(), rows, width,
+                                                  workspace.data_ptr(), size, stream))
+        return grad_scale
+
+    y, same, grad = torch.empty_like(x), x.clone(), torch.empty_like(x)
+    forward(x, y)
+    forward(same, same)
+    assert_bitwise(same, y, "y on x")
+    grad_scale = backward(up, x, grad)
+    for on_x in (False, True):
+        g, a = up.clone(), x.clone()
+        got = backward(g, a, a if on_x else g)
+        assert_bitwise(a if on_x else g, grad, f"grad_x in place (on x: {on_x})")
+        assert_bitwise(got, grad_scale, "grad_scale")
 
 
 def test_gie_then_rmsnorm_config3_reduced():

@@ -15,6 +15,7 @@ import pytest
 import torch
 
 from bysj_amd import kernels, workloads
+from bysj_amd.kernels import _lib
 from oracle import gie as gie_ref
 from oracle import loops
 from oracle import segment as ref
@@ -175,7 +176,7 @@ def test_grouping_flags_of_concurrent_calls():
 def test_group_by_key_async_status_and_capture():
     """The asynchronous build reports the status bits on the device, allocates nothing when given its
     buffers, and replays from a HIP graph with the same result as the synchronous call."""
-    from bysj_amd.kernels import _C, _lib
+    from bysj_amd.kernels import _C
 
     announce("group_by_key async")
     keys = torch.from_numpy(workloads.rng(5).integers(0, 70000, size=90000).astype(np.int64)).to(DEV)
@@ -901,6 +902,57 @@ def test_segment_softmax_config2_full_size_and_determinism():
     assert_close_scaled(null_alpha, e_null, what="config 2 null_alpha")
     total = torch.zeros_like(null_alpha).index_add_(0, d["dst"], alpha) + null_alpha
     assert_close_scaled(total, torch.ones_like(total), what="sum to one")
+
+
+@pytest.mark.parametrize("channels", [3, 8, 13, 33, 66, 257, 290])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_segment_softmax_in_place(channels, ordered):
+    """C ABI: outputs on top of inputs give the values of separate arrays, also where a row's last chunk repeats columns
+    of the slab before it (C mod 32 of 1 to 3) and on segments that are streamed."""
+    announce("softmax in place", channels, ordered)
+    library = _lib.load()
+    dst, offsets = _graph([5, 0, 140, 700, 31, 1, 64] + [40] * 60)
+    if ordered:
+        _, order, offsets = _shuffled(dst, channels)
+        order = order.to(DEV)
+    edges, nodes, stream = dst.numel(), offsets.numel() - 1, torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device=DEV).manual_seed(channels)
+    logit, up = (torch.randn(edges, channels, generator=gen, device=DEV) for _ in range(2))
+    null, up_null = (torch.randn(nodes, channels, generator=gen, device=DEV) for _ in range(2))
+    env, offsets = torch.rand(edges, generator=gen, device=DEV) + 0.05, offsets.to(DEV)
+    order_ptr = order.data_ptr() if ordered else None
+
+    def forward(x, null_x, alpha, null_alpha):
+        _lib.check(library.dpa4k_segment_softmax_forward(
+            x.data_ptr(), env.data_ptr(), offsets.data_ptr(), null_x.data_ptr(), order_ptr, alpha.data_ptr(),
+            null_alpha.data_ptr(), edges, nodes, channels, stream))
+
+    def backward(alpha, grad, null_alpha, grad_null, out, null_out):
+        grad_env = torch.empty(edges, device=DEV)
+        _lib.check(library.dpa4k_segment_softmax_backward(
+            alpha.data_ptr(), grad.data_ptr(), env.data_ptr(), offsets.data_ptr(), null_alpha.data_ptr(),
+            grad_null.data_ptr(), order_ptr, out.data_ptr(), null_out.data_ptr(), grad_env.data_ptr(), edges, nodes,
+            channels, stream))
+        return grad_env
+
+    alpha, null_alpha = torch.empty_like(logit), torch.empty_like(null)
+    forward(logit, null, alpha, null_alpha)
+    x, null_x = logit.clone(), null.clone()
+    forward(x, null_x, x, null_x)
+    assert_bitwise(x, alpha, "alpha on logit")
+    assert_bitwise(null_x, null_alpha, "null_alpha on null_logit")
+    grad, grad_null = torch.empty_like(logit), torch.empty_like(null)
+    grad_env = backward(alpha, up, null_alpha, up_null, grad, grad_null)
+    for on_alpha in (False, True):
+        a, g, na, gn = alpha.clone(), up.clone(), null_alpha.clone(), up_null.clone()
+        out, null_out = (a, na) if on_alpha else (g, gn)
+        got = backward(a, g, na, gn, out, null_out)
+        assert_bitwise(out, grad, f"grad_logit in place (on alpha: {on_alpha})")
+        assert_bitwise(null_out, grad_null, f"grad_null_logit in place (on alpha: {on_alpha})")
+        # the slabs of a row start elsewhere where the last chunk would be alone in one, so its C terms are added in
+        # another order: each order is within C * 2^-24 of their sum of magnitudes
+        bound = 2.0 * channels * 2.0**-24 * grad.double().abs().sum(1) * 2.0 / env.double()
+        assert bool(((got - grad_env).double().abs() <= bound).all()), "grad_env"
 
 
 # ---------------------------------------------------------------------------
