@@ -68,6 +68,11 @@ struct RowChunks {
     if constexpr (kOwnView) return first + static_cast<uint32_t>(j * LG * V * 4);
     else return start[j];
   }
+  // Stores leave the lanes past the row out by the execution mask: dropped by
+  // the view, they still take the lane's turn (two chunks a lane: 200,000 rows
+  // of 300 floats, 11 of 64 lanes in the second, 160 -> 137 us with the scale gradient; with one chunk a lane the
+  // branch costs more than the lanes).
+  __device__ __forceinline__ bool live(int j, int64_t width) const { return at(j) < static_cast<uint32_t>(width) * 4u; }
   __device__ __forceinline__ bool counts(int j, int i) const {
     if constexpr (kTail) return i >= skip[j];
     else return true;
@@ -134,13 +139,14 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_forward_kernel(
         out.v[i] = value[r][j].v[i] * inv;
         if (scale != nullptr) out.v[i] = out.v[i] * s[j].v[i];
       }
-      buffer_store_vec_stream<V>(rows_y, group_at + chunks.at(j), out);
+      if (CPL != 2 || chunks.live(j, width)) buffer_store_vec_stream<V>(rows_y, group_at + chunks.at(j), out);
     }
     if (lane == 0 && base + r * GPW + group < rows) inverse_rms[base + r * GPW + group] = inv;
   }
 }
 
 // Rows wider than the register kernels hold: a wave per row, two passes.
+template <bool kTail>
 __global__ __launch_bounds__(kBlock) void rmsnorm_forward_wide_kernel(
     const float* __restrict__ x, const float* __restrict__ scale, float* __restrict__ y,
     float* __restrict__ inverse_rms, int64_t rows, int64_t width, float eps) {
@@ -151,15 +157,15 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_forward_wide_kernel(
   float* yr = y + row * width;
   float sum = 0.0f;
   for (int64_t c = lane * 4; c < width; c += 256) {
-    const int64_t column = c + 4 <= width ? c : width - 4;
+    const int64_t column = !kTail || c + 4 <= width ? c : width - 4;
     const fvec<4> value = load_chunk(xr + column);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sum = sum + (column + i >= c ? value.v[i] * value.v[i] : 0.0f);
+    for (int i = 0; i < 4; ++i) sum = sum + (!kTail || column + i >= c ? value.v[i] * value.v[i] : 0.0f);
   }
   sum = group_sum<64>(sum);
   const float inv = inverse_rms_of(sum, width, eps);
   for (int64_t c = lane * 4; c < width; c += 256) {
-    const int64_t column = c + 4 <= width ? c : width - 4;
+    const int64_t column = !kTail || c + 4 <= width ? c : width - 4;
     const fvec<4> value = load_chunk(xr + column);
     fvec<4> out, s;
     if (scale != nullptr) s = load_chunk(scale + column);
@@ -242,7 +248,7 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_backward_kernel(
           out.v[i] = inv[r] * u - xv[r][j].v[i] * inv3 * mean_dot;
           if (partial != nullptr) column[j].v[i] = column[j].v[i] + g[r][j].v[i] * (xv[r][j].v[i] * inv[r]);
         }
-        buffer_store_vec_stream<V>(rows_o, group_at + chunks.at(j), out);
+        if (CPL != 2 || chunks.live(j, width)) buffer_store_vec_stream<V>(rows_o, group_at + chunks.at(j), out);
       }
     }
   }
@@ -310,6 +316,7 @@ __global__ __launch_bounds__(kColumnWaves * 64) void partial_columns_kernel(cons
 }
 
 // Streaming grad_x for wide rows: two passes over the row.
+template <bool kTail>
 __global__ __launch_bounds__(kBlock) void rmsnorm_backward_wide_kernel(
     const float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ scale,
     const float* __restrict__ inverse_rms, float* __restrict__ grad_x, int64_t rows,
@@ -321,21 +328,21 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_backward_wide_kernel(
   const float* xr = x + row * width;
   float dot = 0.0f;
   for (int64_t c = lane * 4; c < width; c += 256) {
-    const int64_t column = c + 4 <= width ? c : width - 4;
+    const int64_t column = !kTail || c + 4 <= width ? c : width - 4;
     const fvec<4> g = load_chunk(gr + column);
     const fvec<4> xv = load_chunk(xr + column);
     fvec<4> s;
     if (scale != nullptr) s = load_chunk(scale + column);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      dot = dot + (column + i >= c ? xv.v[i] * (scale != nullptr ? g.v[i] * s.v[i] : g.v[i]) : 0.0f);
+      dot = dot + (!kTail || column + i >= c ? xv.v[i] * (scale != nullptr ? g.v[i] * s.v[i] : g.v[i]) : 0.0f);
   }
   dot = group_sum<64>(dot);
   const float mean_dot = dot / static_cast<float>(width);
   const float inv = inverse_rms[row];
   const float inv3 = inv * inv * inv;
   for (int64_t c = lane * 4; c < width; c += 256) {
-    const int64_t column = c + 4 <= width ? c : width - 4;
+    const int64_t column = !kTail || c + 4 <= width ? c : width - 4;
     const fvec<4> g = load_chunk(gr + column);
     const fvec<4> xv = load_chunk(xr + column);
     fvec<4> s;
@@ -414,11 +421,15 @@ RowShape shape_for(int64_t width) {
 
 // Row sets in flight per wave: forward 4 for the lane groups below a wave where
 // the grid fills the chip (16 waves on each CU) all the same, else 1 (rows of
-// 512 took 25.3 us with two against 23.4 us with one, 32,768 rows); backward 4
-// and 2, and 1 where a row alone takes 128 registers (2,048 columns on: 139 us
-// with two, spilling past the wave's own registers, 120 us with one).
+// 512 took 25.3 us with two against 23.4 us with one, 32,768 rows).  Backward,
+// where a wave has several (with a scale gradient the grid is bounded): 4 for
+// the lane groups, 2 for two to eight chunks a lane, 1 for one chunk (300,000 rows of
+// 200: 126 us, 141 with two) and where a row alone takes 128 registers (2,048
+// columns on: 139 us with two, spilling past the wave's own registers, 120 us
+// with one).  Without a scale gradient every wave has one set: 400,000 rows of 66
+// floats 55 us, 106 while three sets of four lay past the rows.
 constexpr int forward_rows(int lanes) { return lanes < 64 ? 4 : 1; }
-constexpr int backward_rows(int lanes, int cpl) { return cpl >= 16 ? 1 : (lanes < 64 ? 4 : 2); }
+constexpr int backward_rows(int lanes, int cpl) { return cpl >= 16 || (lanes == 64 && cpl == 1) ? 1 : (lanes < 64 ? 4 : 2); }
 constexpr int64_t kFullGrid = 4096;  // waves
 
 // Calls LAUNCH(V, LG, CPL) for a row shape.
@@ -462,15 +473,28 @@ int launch_forward(const float* x, const float* scale, float* y, float* inverse_
   return launched("rmsnorm_forward_kernel");
 }
 
+template <int V, int LG, int CPL, int NR>
+void launch_backward_rows(unsigned int grid, const float* grad, const float* x, const float* scale,
+                          const float* inverse_rms, float* grad_x, float* partial, int64_t rows, int64_t width,
+                          hipStream_t stream) {
+  const size_t lds = partial != nullptr ? kWaves * CPL * 64 * V * sizeof(float) : 0;
+  if (V == 4 && width % 4 != 0)
+    rmsnorm_backward_kernel<V, LG, CPL, NR, V == 4><<<grid, kBlock, lds, stream>>>(grad, x, scale, inverse_rms, grad_x,
+                                                                                   partial, rows, width);
+  else
+    rmsnorm_backward_kernel<V, LG, CPL, NR, false><<<grid, kBlock, lds, stream>>>(grad, x, scale, inverse_rms, grad_x,
+                                                                                  partial, rows, width);
+}
+
 int launch_backward(unsigned int grid, const float* grad, const float* x,
                     const float* scale, const float* inverse_rms, float* grad_x, float* partial,
                     int64_t rows, int64_t width, hipStream_t stream) {
   const RowShape shape = shape_for(width);
-#define DPA4K_RMS_BWD(V, LG, CPL)                                                                              \
-  ((V == 4 && width % 4 != 0 ? rmsnorm_backward_kernel<V, LG, CPL, backward_rows(LG, CPL), V == 4>                  \
-                             : rmsnorm_backward_kernel<V, LG, CPL, backward_rows(LG, CPL), false>))                 \
-      <<<grid, kBlock, partial != nullptr ? kWaves * CPL * 64 * V * sizeof(float) : 0, stream>>>(               \
-          grad, x, scale, inverse_rms, grad_x, partial, rows, width)
+  // one row set per wave: further ones would lie past the rows, and be loaded, reduced and dropped all the same
+  const bool single = row_blocks(shape, 1, rows) <= static_cast<int64_t>(grid);
+#define DPA4K_RMS_BWD(V, LG, CPL)                                                                               \
+  (single ? launch_backward_rows<V, LG, CPL, 1> : launch_backward_rows<V, LG, CPL, backward_rows(LG, CPL)>)(    \
+      grid, grad, x, scale, inverse_rms, grad_x, partial, rows, width, stream)
   DPA4K_ROW_SHAPES(shape, DPA4K_RMS_BWD)
 #undef DPA4K_RMS_BWD
   return launched("rmsnorm_backward_kernel");
@@ -559,7 +583,10 @@ int rmsnorm_backward(const float* grad, const float* x, const float* scale, cons
   }
   if (wide) {
     const dim3 grid = launch_grid((rows + kWaves - 1) / kWaves, kBlock);
-    rmsnorm_backward_wide_kernel<<<grid, kBlock, 0, stream>>>(grad, x, scale, inverse_rms, grad_x, rows, width);
+    if (width % 4 != 0)
+      rmsnorm_backward_wide_kernel<true><<<grid, kBlock, 0, stream>>>(grad, x, scale, inverse_rms, grad_x, rows, width);
+    else
+      rmsnorm_backward_wide_kernel<false><<<grid, kBlock, 0, stream>>>(grad, x, scale, inverse_rms, grad_x, rows, width);
     return launched("rmsnorm_backward_wide_kernel");
   }
   if (grad_scale == nullptr || columns) {
@@ -610,8 +637,11 @@ extern "C" int dpa4k_rmsnorm_forward(const float* x, const float* scale, float* 
     return fail(DPA4K_EINVAL, "RMSNorm: null pointer");
   hipStream_t stream = as_stream(stream_handle);
   if (fits_registers(width)) return launch_forward(x, scale, y, inverse_rms, rows, width, eps, stream);
-  rmsnorm_forward_wide_kernel<<<launch_grid((rows + kWaves - 1) / kWaves, kBlock), kBlock, 0, stream>>>(
-      x, scale, y, inverse_rms, rows, width, eps);
+  const dim3 grid = launch_grid((rows + kWaves - 1) / kWaves, kBlock);
+  if (width % 4 != 0)
+    rmsnorm_forward_wide_kernel<true><<<grid, kBlock, 0, stream>>>(x, scale, y, inverse_rms, rows, width, eps);
+  else
+    rmsnorm_forward_wide_kernel<false><<<grid, kBlock, 0, stream>>>(x, scale, y, inverse_rms, rows, width, eps);
   return launched("rmsnorm_forward_wide_kernel");
 }
 

@@ -222,6 +222,24 @@ def test_rmsnorm_zero_input_no_scale_and_stream():
     assert_gradient(grad_x, e_x, t_x, "grad_x without scale")
 
 
+@pytest.mark.parametrize("rows,width", [(26003, 3), (26003, 64), (13001, 66), (13001, 128), (7001, 200), (7001, 301),
+                                        (7001, 512), (7001, 1030)])
+def test_rmsnorm_backward_row_sets(rows, width):
+    """More rows than one set for every wave of the bounded grid: grad_scale against 64 bits, and grad_x the bits of a
+    frozen scale, whose waves take one set each."""
+    announce("rmsnorm row sets", rows, width)
+    gen = torch.Generator(device=DEV).manual_seed(width)
+    x, up = (torch.randn(rows, width, generator=gen, device=DEV) for _ in range(2))
+    scale = torch.rand(width, generator=gen, device=DEV) + 0.5
+    _, inverse_rms = _C.rmsnorm_forward(x, scale, 1e-6)
+    grad_x, grad_scale = _C.rmsnorm_backward(up, x, scale, inverse_rms, True)
+    truth_x, truth_scale = rmsnorm_backward_f64(up, x, scale, eps=1e-6)
+    assert_close_scaled(grad_x, truth_x, what="grad_x")
+    assert_close_scaled(grad_scale, truth_scale, what="grad_scale")
+    frozen, _ = _C.rmsnorm_backward(up, x, scale, inverse_rms, False)
+    assert_bitwise(frozen, grad_x, "grad_x with a frozen scale")
+
+
 @pytest.mark.parametrize("width", [3, 66, 1001, 4096, 4097, 4610, 5000])
 def test_rmsnorm_in_place(width):
     """C ABI: y on x and grad_x on grad or x give the bits of separate arrays (W mod 256 of 1 to 3 past 4,096: the last
