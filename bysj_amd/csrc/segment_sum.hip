@@ -141,12 +141,15 @@ __global__ __launch_bounds__(kBlock) void segment_sum_forward_kernel(
 // `accumulate` adds the partial dots of this channel window to the values
 // written by the previous window (channels wider than one window).
 //
-// Any width of at least 4 runs in 16-byte chunks, whatever its alignment; one
-// float a lane took 463 us at C = 77 (1.98M edges; now 263 us by the workgroup
-// kernel) and 166 us at C = 13 (now 85).  Natural-order rows of up to 16 floats
-// share lines with the next slots' rows, and their gradients are stored with
-// the default policy, which merges them (C = 8: 99 -> 60 us, C = 16 even).
-template <int V, int G, int CPL, int U, bool kOrdered>
+// Any width of at least 4 runs in 16-byte chunks, whatever its alignment (but
+// see scalar_backward); one float a lane took 463 us at C = 77 (1.98M edges; now
+// 263 us by the workgroup kernel).  kTail: a row's last chunk repeats columns of
+// its neighbour, which count in no dot product.  Natural-order rows of up to 16
+// floats, and ragged ones of up to 32, share lines with the next slots' rows, and
+// their gradients are stored with the default policy, which merges them (C = 8:
+// 99 -> 60 us, C = 16 even; C = 17, degree 30: 109 -> 58, C = 31: 134 -> 114);
+// ragged rows of up to 16 through an order likewise (C = 13: 144 -> 132).
+template <int V, int G, int CPL, int U, bool kOrdered, bool kTail>
 __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
     const float* __restrict__ grad_out, const float* __restrict__ src,
     const int64_t* __restrict__ offsets, const float* __restrict__ edge_scale,
@@ -155,6 +158,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
     float* __restrict__ grad_node_scale, int64_t n_edges, int64_t n_nodes, int64_t channels,
     int64_t chunk_base, int accumulate) {
   constexpr int kSegments = kBlock / G;
+  constexpr bool kStream = kTail ? G > (kOrdered ? 4 : 8) : kOrdered || G * CPL * V > 16;
   const int64_t segment = block_index() * kSegments + threadIdx.x / G;
   if (segment >= n_nodes) return;
   const int lane = threadIdx.x % G;
@@ -170,7 +174,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
   for (int j = 0; j < CPL; ++j) {
     const int64_t chunk = chunk_base + lane + static_cast<int64_t>(G) * j;
     column[j] = chunk_column<V>(chunk, channels, live[j]);
-    skip[j] = live[j] ? static_cast<int>(chunk * V - column[j]) : 0;
+    skip[j] = kTail && live[j] ? static_cast<int>(chunk * V - column[j]) : 0;
   }
 
   const float scale = node_scale != nullptr ? node_scale[segment] : 1.0f;
@@ -219,7 +223,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
         fvec<V> out;
 #pragma unroll
         for (int i = 0; i < V; ++i) out.v[i] = has_edge_scale ? gs[j].v[i] * weight[u] : gs[j].v[i];
-        store_row_chunk<V, (kOrdered || G * CPL * V > 16)>(grad_src + edge[u] * channels + column[j], out);
+        store_row_chunk<V, kStream>(grad_src + edge[u] * channels + column[j], out);
       }
     }
     if (need_dot) {
@@ -229,7 +233,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_kernel(
 #pragma unroll
         for (int j = 0; j < CPL; ++j)
 #pragma unroll
-          for (int i = 0; i < V; ++i) d = d + (V == 1 || i >= skip[j] ? g[j].v[i] * x[u][j].v[i] : 0.0f);
+          for (int i = 0; i < V; ++i) d = d + (!kTail || i >= skip[j] ? g[j].v[i] * x[u][j].v[i] : 0.0f);
         dot[u] = group_sum<G>(d);
       }
 #pragma unroll
@@ -344,7 +348,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_staged_kernel(
 // streams of src and grad_src.  Rows of several chunks per lane used to run a
 // wave per segment, 2 rows in flight: 3,000 segments of 90 rows of 1,024
 // floats took 483 us, 449 with a workgroup per segment.
-template <int G, int CPL, int U, bool kOrdered, bool kStreamRows, bool kStreamGrads>
+template <int G, int CPL, int U, bool kOrdered, bool kStreamRows, bool kStreamGrads, bool kTail>
 __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
     const float* __restrict__ grad_out, const float* __restrict__ src,
     const int64_t* __restrict__ offsets, const float* __restrict__ edge_scale,
@@ -354,7 +358,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
   constexpr int SG = kBlock / G;
   __shared__ float partial[SG];
   const int64_t unit = block_index();
-  const int64_t segment = shares == 1 ? unit : unit / shares;
+  const int64_t segment = uniform_i64(shares == 1 ? unit : unit / shares);
   if (segment >= n_nodes) return;
   const int share = static_cast<int>(unit - segment * shares);
   const int lane = threadIdx.x % G;
@@ -366,7 +370,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
   for (int j = 0; j < CPL; ++j) {
     const int64_t chunk = lane + static_cast<int64_t>(G) * j;
     column[j] = chunk_column<4>(chunk, channels, live[j]);
-    skip[j] = live[j] ? static_cast<int>(chunk * 4 - column[j]) : 0;
+    skip[j] = kTail && live[j] ? static_cast<int>(chunk * 4 - column[j]) : 0;
   }
   const bool want_edge = grad_edge_scale != nullptr;
   const bool want_node = grad_node_scale != nullptr;
@@ -436,7 +440,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
 #pragma unroll
         for (int j = 0; j < CPL; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) d = d + (i >= skip[j] ? g[j].v[i] * x[u][j].v[i] : 0.0f);
+          for (int i = 0; i < 4; ++i) d = d + (!kTail || i >= skip[j] ? g[j].v[i] * x[u][j].v[i] : 0.0f);
         d = group_sum<G>(d);
         if (edge[u] < 0) continue;
         if (want_edge && lane == 0) grad_edge_scale[edge[u]] = scale * d;
@@ -480,6 +484,7 @@ int launch_staged_forward(const float* src, const int64_t* offsets, const float*
 // 68; 90 or 60 rows of 256 floats in two shares 374 -> 344; rows gathered through
 // an order 463 -> 452.  The sum of grad_node_scale keeps one workgroup.
 constexpr int64_t kShareBytes = 32768;
+constexpr int64_t kStreamedFloats = int64_t(1) << 24;
 int backward_shares(int64_t n_edges, int64_t n_nodes, int64_t channels, bool want_node) {
   if (want_node) return 1;
   const double bytes = static_cast<double>(n_edges) / static_cast<double>(n_nodes) * static_cast<double>(channels) * 4.0;
@@ -495,27 +500,31 @@ int launch_wide_backward_g(const float* grad_out, const float* src, const int64_
   constexpr int U = CPL >= 8 ? 1 : 8 / CPL;  // 8 chunks of a row set in flight per lane
   const int shares = backward_shares(n_edges, n_nodes, channels, grad_node_scale != nullptr);
   const dim3 grid = launch_grid(n_nodes * shares, kBlock);
-  // Gradient rows are stored non-temporally, and on small grids the rows loaded so (config 1: 11.4 ->
-  // 10.6-10.9 us; on large ones it does not pay, config 1R: 1,846 -> 1,886-1,903 us), except rows of several
+  // Gradient rows are stored non-temporally, and on small grids of little data the rows loaded so (config 1: 11.4 ->
+  // 10.6-10.9 us; on large ones it does not pay, config 1R: 1,846 -> 1,886-1,903 us, nor on few segments of
+  // much data, 2,604 gathered segments of 30 rows of 512: 69 against 61 us), except rows of several
   // chunks per lane that do not end on cache lines (C = 331: 419 -> 390 us forward and backward; C = 77, one
   // chunk per lane, the other way round: 402 against 424 us).
-  const bool stream_rows = n_nodes < 4096;
+  const bool stream_rows = n_nodes < 4096 && n_edges * channels < kStreamedFloats;  // (64 MB)
   const bool shared_lines = CPL > 1 && channels % 32 != 0;
-#define DPA4K_SUM_BWD_WIDE(ORD, NT, NTG)                                                                \
-  segment_sum_backward_wide_kernel<G, CPL, U, ORD, NT, NTG><<<grid, kBlock, 0, stream>>>(                \
+#define DPA4K_SUM_BWD_WIDE_T(ORD, NT, NTG, TAIL)                                                         \
+  segment_sum_backward_wide_kernel<G, CPL, U, ORD, NT, NTG, TAIL><<<grid, kBlock, 0, stream>>>(          \
       grad_out, src, offsets, edge_scale, node_scale, order, grad_src, grad_edge_scale, grad_node_scale, \
       n_edges, n_nodes, channels, shares)
+#define DPA4K_SUM_BWD_WIDE(ORD, NT, NTG)                                                                \
+  if (channels % 4 != 0) DPA4K_SUM_BWD_WIDE_T(ORD, NT, NTG, true); else DPA4K_SUM_BWD_WIDE_T(ORD, NT, NTG, false)
   if constexpr (CPL > 1) {
     if (shared_lines) {
-      if (order != nullptr) DPA4K_SUM_BWD_WIDE(true, false, false); else DPA4K_SUM_BWD_WIDE(false, false, false);
+      if (order != nullptr) { DPA4K_SUM_BWD_WIDE(true, false, false); } else { DPA4K_SUM_BWD_WIDE(false, false, false); }
       return launched("segment_sum_backward_wide_kernel");
     }
   }
   if (order != nullptr) {
-    if (stream_rows) DPA4K_SUM_BWD_WIDE(true, true, true); else DPA4K_SUM_BWD_WIDE(true, false, true);
+    if (stream_rows) { DPA4K_SUM_BWD_WIDE(true, true, true); } else { DPA4K_SUM_BWD_WIDE(true, false, true); }
   } else {
-    if (stream_rows) DPA4K_SUM_BWD_WIDE(false, true, true); else DPA4K_SUM_BWD_WIDE(false, false, true);
+    if (stream_rows) { DPA4K_SUM_BWD_WIDE(false, true, true); } else { DPA4K_SUM_BWD_WIDE(false, false, true); }
   }
+#undef DPA4K_SUM_BWD_WIDE_T
 #undef DPA4K_SUM_BWD_WIDE
   return launched("segment_sum_backward_wide_kernel");
 }
@@ -541,13 +550,31 @@ int launch_wide_backward(const float* grad_out, const float* src, const int64_t*
 // rows of 16 to 64 whole chunks (64 to 256 channels) on grids of fewer than
 // kWideSegments segments; on larger grids the lane-group kernel's several rows
 // in flight per lane stream faster (config 1R: 1.03 ms against 1.07-1.17 ms).
-// The backward uses its workgroup kernel on every grid for rows of 16 to 512
-// chunks (config 1R: 1.75 ms against 2.15 ms for the lane-group kernel).
+// The backward uses its workgroup kernel for rows of 16 to 512 chunks (config
+// 1R: 1.75 ms against 2.15 ms for the lane-group kernel) where a segment has
+// enough rows for its workgroup (use_wide_backward).  Lane groups against
+// workgroups, 160 MB of rows, us: C = 64 degree 8 55 / 183, 16 58 / 106, 30 59 /
+// 65, 60 62 / 52; C = 128 8 54 / 114, 16 57 / 69, 30 57 / 53; C = 256 8 54 / 73,
+// 16 54 / 53; C = 260, whose second chunk one lane holds, 30 67 / 80, 90 83 / 78;
+// C = 512 4 58 / 62, 8 57 / 52; C = 1024 4 61 / 55.  Without dot products, which
+// read no rows of src, the workgroups win earlier: C = 256 degree 12 34 / 27.
 constexpr int64_t kWideSegments = 4096;
+double mean_degree(int64_t n_edges, int64_t n_nodes) {
+  return static_cast<double>(n_edges) / static_cast<double>(n_nodes);
+}
 bool use_wide_forward(int64_t n_nodes, int64_t channels) {
   return n_nodes < kWideSegments && channels % 4 == 0 && channels >= 64 && channels <= 256;
 }
-bool use_wide_backward(int64_t channels) { return channels > 60 && channels <= 2048; }
+bool use_wide_backward(int64_t n_edges, int64_t n_nodes, int64_t channels, bool need_dot) {
+  if (channels <= 60 || channels > 2048) return false;
+  if (n_nodes < kWideSegments && channels <= 256) return true;
+  const double degree = mean_degree(n_edges, n_nodes);
+  if (channels <= 128) return degree >= 24.0;
+  if (!need_dot && channels <= 384) return degree >= 8.0;
+  if (channels <= 256) return degree >= 16.0;
+  if (channels <= 384) return degree >= (channels % 4 == 0 ? 48.0 : 20.0);
+  return degree * static_cast<double>(channels) >= 3072.0;
+}
 
 // Lane-group geometry for a row of `chunks` vector chunks.
 struct Geometry {
@@ -565,7 +592,26 @@ Geometry geometry_for(int64_t chunks) {
   }
   return g;
 }
-int64_t chunks_for(int64_t channels) { return channels < 4 ? channels : (channels + 3) / 4; }
+bool ragged(int64_t channels) { return channels >= 4 && channels % 4 != 0; }
+
+// Chunks of a row, and floats per chunk.
+struct Chunks {
+  int width;
+  int64_t count;
+};
+Chunks chunks_for(int64_t channels, bool scalar) {
+  return channels < 4 || scalar ? Chunks{1, channels} : Chunks{4, (channels + 3) / 4};
+}
+// Whether rows that are no whole chunks run one float a lane after all: on long segments a group of few lanes walks
+// them too slowly (us, 16-byte chunks and single floats: forward C = 13, degree 90 through an order 101 / 80; backward
+// 159 / 138; 64 segments of 23,000 rows, C = 31, forward 2,764 / 1,734, backward 6,360 / 5,740).
+bool scalar_forward(int64_t n_edges, int64_t n_nodes, int64_t channels) {
+  return ragged(channels) && channels < 100 && mean_degree(n_edges, n_nodes) > (channels < 16 ? 48.0 : 512.0);
+}
+bool scalar_backward(int64_t n_edges, int64_t n_nodes, int64_t channels, bool ordered) {
+  return ragged(channels) && channels <= 60 &&
+         mean_degree(n_edges, n_nodes) > (channels < 16 && ordered ? 48.0 : 512.0);
+}
 
 // Slots per round: about 32 loaded floats per lane, or 128 when the grid is
 // too small to fill the chip (then each lane must keep more bytes in flight).
@@ -579,7 +625,7 @@ int launch_forward_u(const float* src, const int64_t* offsets, const float* edge
                      const float* node_scale, const int64_t* order, float* out, int64_t n_edges,
                      int64_t n_nodes, int64_t channels, hipStream_t stream) {
   // windows of G * CPL chunks are further units of the grid
-  const int64_t windows = (chunks_for(channels) + G * CPL - 1) / (G * CPL);
+  const int64_t windows = ((channels + V - 1) / V + G * CPL - 1) / (G * CPL);
   const dim3 grid = launch_grid((n_nodes * windows + kBlock / G - 1) / (kBlock / G), kBlock);
 #define DPA4K_SUM_FWD(SCALE, ORD, NT)                                                                 \
   segment_sum_forward_kernel<V, G, CPL, U, SCALE, ORD, NT><<<grid, kBlock, 0, stream>>>(             \
@@ -590,10 +636,10 @@ int launch_forward_u(const float* src, const int64_t* offsets, const float* edge
   } else {                                                                                            \
     if (order != nullptr) DPA4K_SUM_FWD(false, true, NT); else DPA4K_SUM_FWD(false, false, NT);       \
   }
-  // Rows under 64 bytes share most of their lines with the next slots' rows: the default policy keeps those
-  // (C = 13, 1.98M edges: 48 -> 41 us).
-  if constexpr (G * CPL * V <= 16) {
-    if (channels < 16 && order == nullptr) {
+  // Rows that share lines with others are loaded with the default policy, which keeps those (C = 13, 1.98M edges: 48
+  // -> 41 us; C = 31, degree 90: 44.5 -> 29, through an order 86 -> 75, both with eight slots a round).
+  if constexpr (CPL == 1) {
+    if ((channels < 16 && order == nullptr) || (V == 4 && ragged(channels))) {
       DPA4K_SUM_FWD_ANY(false)
       return launched("segment_sum_forward_kernel");
     }
@@ -631,11 +677,16 @@ template <int V, int G, int CPL>
 int launch_forward(const float* src, const int64_t* offsets, const float* edge_scale,
                    const float* node_scale, const int64_t* order, float* out, int64_t n_edges,
                    int64_t n_nodes, int64_t channels, hipStream_t stream) {
-  if constexpr (CPL == 1) {
-    if (small_grid(n_nodes, G))
-      return launch_forward_u<V, G, CPL, unroll_for<V, CPL>(true)>(src, offsets, edge_scale, node_scale, order, out,
-                                                                   n_edges, n_nodes, channels, stream);
+  // Ragged rows: eight slots a round (us at degrees 8, 30 and 90 with 32 slots and with 8: C = 13 28, 27, 34 and 19, 25,
+  // 29; C = 45 55, 39, 38 and 29, 30, 31), unless the grid has few waves.
+  if constexpr (V == 4 && CPL == 1) {
+    if (ragged(channels) && !small_grid(n_nodes * 4, G))
+      return launch_forward_u<V, G, CPL, 8>(src, offsets, edge_scale, node_scale, order, out, n_edges, n_nodes,
+                                            channels, stream);
   }
+  if (small_grid(n_nodes, G))
+    return launch_forward_u<V, G, CPL, 32 / CPL>(src, offsets, edge_scale, node_scale, order, out, n_edges, n_nodes,
+                                                 channels, stream);
   if (order == nullptr)
     return launch_forward_u<V, G, CPL, contiguous_unroll_for<V, CPL>()>(src, offsets, edge_scale, node_scale,
                                                                         order, out, n_edges, n_nodes, channels,
@@ -651,14 +702,16 @@ int launch_backward_u(const float* grad_out, const float* src, const int64_t* of
                       int64_t n_edges, int64_t n_nodes, int64_t channels, int64_t chunk_base,
                       int accumulate, hipStream_t stream) {
   const dim3 grid = launch_grid((n_nodes + kBlock / G - 1) / (kBlock / G), kBlock);
-  if (order != nullptr)
-    segment_sum_backward_kernel<V, G, CPL, U, true><<<grid, kBlock, 0, stream>>>(
-        grad_out, src, offsets, edge_scale, node_scale, order, grad_src, grad_edge_scale,
-        grad_node_scale, n_edges, n_nodes, channels, chunk_base, accumulate);
-  else
-    segment_sum_backward_kernel<V, G, CPL, U, false><<<grid, kBlock, 0, stream>>>(
-        grad_out, src, offsets, edge_scale, node_scale, order, grad_src, grad_edge_scale,
-        grad_node_scale, n_edges, n_nodes, channels, chunk_base, accumulate);
+#define DPA4K_SUM_BWD(ORD, TAIL)                                                                          \
+  segment_sum_backward_kernel<V, G, CPL, U, ORD, TAIL><<<grid, kBlock, 0, stream>>>(                      \
+      grad_out, src, offsets, edge_scale, node_scale, order, grad_src, grad_edge_scale, grad_node_scale, \
+      n_edges, n_nodes, channels, chunk_base, accumulate)
+  if (V == 4 && (ragged(channels) || (CPL == 8 && order != nullptr))) {
+    if (order != nullptr) DPA4K_SUM_BWD(true, V == 4); else DPA4K_SUM_BWD(false, V == 4);
+  } else {
+    if (order != nullptr) DPA4K_SUM_BWD(true, false); else DPA4K_SUM_BWD(false, false);
+  }
+#undef DPA4K_SUM_BWD
   return launched("segment_sum_backward_kernel");
 }
 
@@ -668,6 +721,19 @@ int launch_backward(const float* grad_out, const float* src, const int64_t* offs
                     float* grad_src, float* grad_edge_scale, float* grad_node_scale,
                     int64_t n_edges, int64_t n_nodes, int64_t channels, int64_t chunk_base,
                     int accumulate, hipStream_t stream) {
+  // Ragged rows: eight slots a round in natural order (C = 45 at degrees 4, 30, 90: 75, 119, 107 us with four, 72, 96,
+  // 101 with eight), two through an order (C = 45, degree 30: 142 with four, 131).
+  if constexpr (V == 4 && CPL == 1) {
+    const bool full = !small_grid(n_nodes * 4, G);
+    if (ragged(channels) && order == nullptr && full)
+      return launch_backward_u<V, G, CPL, 8>(grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
+                                             grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, chunk_base,
+                                             accumulate, stream);
+    if (ragged(channels) && order != nullptr && full && G <= 16)
+      return launch_backward_u<V, G, CPL, 2>(grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
+                                             grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, chunk_base,
+                                             accumulate, stream);
+  }
   // the backward holds its rows for the dot products: half the forward's depth
   if (small_grid(n_nodes, G))
     return launch_backward_u<V, G, CPL, unroll_for<V, CPL>(true) / 2>(
@@ -736,13 +802,18 @@ extern "C" int dpa4k_segment_sum_forward(const float* src, const int64_t* offset
   if (use_wide_forward(n_nodes, channels))
     return launch_staged_forward(src, offsets, edge_scale, node_scale, order, out, n_edges, n_nodes, channels,
                                  stream);
-  Geometry geo = geometry_for(chunks_for(channels));
-  // a grid too small to fill the chip takes one chunk per lane, and a wave per window of the row
-  if (small_grid(n_nodes, geo.group)) geo.per_lane = 1;
-  return channels >= 4 ? dispatch_geometry<4, ForwardLauncher>(geo, src, offsets, edge_scale, node_scale, order, out,
-                                                               n_edges, n_nodes, channels, stream)
-                       : dispatch_geometry<1, ForwardLauncher>(geo, src, offsets, edge_scale, node_scale, order, out,
-                                                               n_edges, n_nodes, channels, stream);
+  const Chunks chunks = chunks_for(channels, scalar_forward(n_edges, n_nodes, channels));
+  Geometry geo = geometry_for(chunks.count);
+  // A grid too small to fill the chip takes one chunk per lane, and a wave per window of the row, where the windows
+  // are full and the segments longer than half a round (1,500 segments of 8 rows of 512: 9.0 us in windows, 7.3 without;
+  // C = 260 gathered, degree 90: 65 and 54; an order is read once per window).
+  const bool full = chunks.count > (order != nullptr ? 128 : 96);
+  if (small_grid(n_nodes, geo.group) && full && mean_degree(n_edges, n_nodes) >= 16.0) geo.per_lane = 1;
+  return chunks.width == 4
+             ? dispatch_geometry<4, ForwardLauncher>(geo, src, offsets, edge_scale, node_scale, order, out, n_edges,
+                                                     n_nodes, channels, stream)
+             : dispatch_geometry<1, ForwardLauncher>(geo, src, offsets, edge_scale, node_scale, order, out, n_edges,
+                                                     n_nodes, channels, stream);
 }
 
 extern "C" int dpa4k_segment_sum_backward(const float* grad_out, const float* src,
@@ -763,20 +834,21 @@ extern "C" int dpa4k_segment_sum_backward(const float* grad_out, const float* sr
   if (grad_node_scale != nullptr && node_scale == nullptr)
     return fail(DPA4K_EINVAL, "segment sum backward: grad_node_scale needs node_scale");
   hipStream_t stream = as_stream(stream_handle);
-  if (use_wide_backward(channels))
+  if (use_wide_backward(n_edges, n_nodes, channels, grad_edge_scale != nullptr || grad_node_scale != nullptr))
     return launch_wide_backward(grad_out, src, offsets, edge_scale, node_scale, order, grad_src, grad_edge_scale,
                                 grad_node_scale, n_edges, n_nodes, channels, stream);
-  const int64_t chunks = chunks_for(channels);
-  const Geometry geo = geometry_for(chunks);
+  const Chunks chunks = chunks_for(channels, scalar_backward(n_edges, n_nodes, channels, order != nullptr));
+  const Geometry geo = geometry_for(chunks.count);
   int accumulate = 0;
-  for (int64_t base = 0; base < chunks; base += geo.window()) {
+  for (int64_t base = 0; base < chunks.count; base += geo.window()) {
     const int status =
-        channels >= 4 ? dispatch_geometry<4, BackwardLauncher>(geo, grad_out, src, offsets, edge_scale, node_scale,
-                                                               order, grad_src, grad_edge_scale, grad_node_scale,
-                                                               n_edges, n_nodes, channels, base, accumulate, stream)
-                      : dispatch_geometry<1, BackwardLauncher>(geo, grad_out, src, offsets, edge_scale, node_scale,
-                                                               order, grad_src, grad_edge_scale, grad_node_scale,
-                                                               n_edges, n_nodes, channels, base, accumulate, stream);
+        chunks.width == 4
+            ? dispatch_geometry<4, BackwardLauncher>(geo, grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
+                                                     grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, base,
+                                                     accumulate, stream)
+            : dispatch_geometry<1, BackwardLauncher>(geo, grad_out, src, offsets, edge_scale, node_scale, order, grad_src,
+                                                     grad_edge_scale, grad_node_scale, n_edges, n_nodes, channels, base,
+                                                     accumulate, stream);
     if (status) return status;
     accumulate = 1;
   }

@@ -296,6 +296,41 @@ def test_segment_sum_with_order_is_bit_exact(channels):
     assert_bitwise(out, ref.segment_sum_reference(src, dst, offsets, w, s), "segment_sum with order")
 
 
+@pytest.mark.parametrize("channels", [5, 13, 15, 31, 45, 61, 64, 77, 128, 256, 260, 331, 520])
+@pytest.mark.parametrize("sizes", ["short", "middle", "long", "few"])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_segment_sum_routes(channels, sizes, ordered):
+    """The kernels chosen by width and mean degree (lane groups in chunks or single floats, a workgroup per segment, shares,
+    windows): the forward bit for bit, the gradients against 64 bits, each with and without the dot products."""
+    announce("segment_sum routes", channels, sizes, ordered)
+    degrees = {"short": [0, 3, 1, 9] * 1100, "middle": [30, 0, 61] * 60, "long": [700, 1, 900],
+               "few": [2, 5, 0, 17]}[sizes]
+    dst, offsets = _graph(degrees)
+    order = None
+    if ordered:
+        dst, order, offsets = _shuffled(dst, channels)
+    nodes, gen = offsets.numel() - 1, torch.Generator().manual_seed(channels)
+    src = torch.randn(dst.numel(), channels, generator=gen)
+    w, s = torch.rand(dst.numel(), generator=gen) + 0.5, torch.rand(nodes, generator=gen) + 0.5
+    up = torch.randn(nodes, channels, generator=gen)
+    expected = ref.segment_sum_reference(src, dst, offsets, w, s)
+    t_src, t_w, t_s = segment_sum_backward_f64(up, src, dst, nodes, w, s)
+    d = [t.to(DEV) for t in (dst, offsets)]
+    for want_w, want_s in ((False, False), (True, False), (True, True)):
+        x, wd, sd = src.to(DEV).requires_grad_(True), w.to(DEV).requires_grad_(want_w), s.to(DEV).requires_grad_(want_s)
+        out = kernels.segment_sum(x, *d, wd, sd, order=None if order is None else order.to(DEV))
+        assert_bitwise(out.detach(), expected, "forward")
+        leaves = [x] + [t for t in (wd, sd) if t.requires_grad]
+        grads = torch.autograd.grad(out, leaves, up.to(DEV))
+        for grad, truth in zip(grads[:2], (t_src, t_w)):
+            assert_close_scaled(grad, truth, what=f"gradients ({want_w}, {want_s})")
+        if want_s:  # a sum over a segment's rows and columns: its rounding is within (C + rows) * 2^-24 of the magnitudes
+            terms = torch.zeros(nodes, dtype=torch.float64).index_add_(
+                0, dst, (up[dst].double() * src.double()).abs().sum(1) * w.double())
+            bound = (channels + max(degrees) + 2) * 2.0**-24 * terms
+            assert bool(((grads[2].cpu().double() - t_s).abs() <= bound).all()), "grad_node_scale"
+
+
 @pytest.mark.parametrize("channels", [64, 128, 256])
 def test_segment_sum_nan_edge_scale_propagates_with_order(channels):
     """A NaN in edge_scale reaches the output of its segment, with or without an order, on the
