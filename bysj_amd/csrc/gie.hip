@@ -431,12 +431,13 @@ struct DegreeArgs {
   float eps;
 };
 
-template <int LMAX, int F, int NPW, bool kOrdered, bool kNorm>
+template <int LMAX, int F, int NPW, bool kOrdered, bool kNorm, bool kShort>
 __global__ __launch_bounds__(kBlock) void gie_forward_degrees_kernel(DegreeArgs a) {
   constexpr int R = (LMAX + 1) * (LMAX + 1) - 1;
   constexpr int C = 64 * F / NPW;
   constexpr int ZR = (R + 15) / 16;                       // zonal values a lane loads per edge
-  constexpr int U = 64 / (LMAX * F + ZR) < 16 ? 64 / (LMAX * F + ZR) : 16;  // edges whose loads go out together
+  // edges whose loads go out together
+  constexpr int U = kShort ? 4 : (64 / (LMAX * F + ZR) < 16 ? 64 / (LMAX * F + ZR) : 16);
   constexpr int W = (R + 1) * C;
   __shared__ float tile[kNorm ? kWaves * NPW * W : 1];
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -573,8 +574,19 @@ bool takes_degrees(int32_t slot_info, int64_t n_rows, int64_t n_radial, int64_t 
 template <int LMAX, int F, int NPW, bool kNorm>
 void launch_degrees_of(const DegreeArgs& a, hipStream_t stream) {
   const dim3 grid = launch_grid((a.n_nodes + kWaves * NPW - 1) / (kWaves * NPW), kBlock);
-  if (a.order != nullptr) gie_forward_degrees_kernel<LMAX, F, NPW, true, kNorm><<<grid, kBlock, 0, stream>>>(a);
-  else gie_forward_degrees_kernel<LMAX, F, NPW, false, kNorm><<<grid, kBlock, 0, stream>>>(a);
+#define DPA4K_GIE_DEGREES(SHORT)                                                                                   \
+  if (a.order != nullptr) gie_forward_degrees_kernel<LMAX, F, NPW, true, kNorm, SHORT><<<grid, kBlock, 0, stream>>>(a); \
+  else gie_forward_degrees_kernel<LMAX, F, NPW, false, kNorm, SHORT><<<grid, kBlock, 0, stream>>>(a)
+  // A round of 16 edges is loaded whole: with one slot an edge, short segments take rounds of 4 (lmax 1, C = 64, 641k
+  // edges of 320k nodes: 453 us with 16, 125 with 4; 231 in gie_forward_shared_kernel).
+  if constexpr (LMAX == 1) {
+    if (a.n_edges < 6 * a.n_nodes) {
+      DPA4K_GIE_DEGREES(true);
+      return;
+    }
+  }
+  DPA4K_GIE_DEGREES(false);
+#undef DPA4K_GIE_DEGREES
 }
 
 template <int LMAX, bool kNorm>
@@ -723,7 +735,8 @@ __global__ __launch_bounds__(kBlock) void gie_rmsnorm_forward_kernel(
   if (lane == 0) inverse_rms[node] = inv_rms;
 }
 
-// Two of the backward kernels give a node to a workgroup of kNodeWaves waves,
+// Two of the backward kernels give a node to a workgroup of kNodeWaves waves (NW
+// of them; with NW = 1 the workgroup has a node per wave, for low degrees),
 // which take its edges in turn, so that the chip reads and writes one narrow
 // window of the edge arrays at a time.  A wave per node kept thousands of
 // places in flight, which cost bandwidth.  With one, two, four and eight waves
@@ -731,6 +744,28 @@ __global__ __launch_bounds__(kBlock) void gie_rmsnorm_forward_kernel(
 // 800, 731 and 784 us; at lmax 4, 0.74M edges 396, 414, 346 and 483; distinct
 // slots at lmax 3, 0.37M edges 627, 623, 598 and 584.
 constexpr int kNodeWaves = 4;
+static_assert(kNodeWaves == kWaves, "a workgroup holds one node or a wave per node");
+
+// Whether a node gets a workgroup rather than a wave: from a mean degree of `enough` edges on, or of `some` where the
+// nodes are too few to fill the chip with a wave each.  Below, most of the waves only stage rows and wait at the
+// barrier behind grad_inv.  DeepMD's map at lmax 3, 600k edges, a workgroup and a wave per node, us: C = 64 degree 8 559 /
+// 307, 16 313 / 223, 24 235 / 221, 48 192 / 232, without grad_inv 24 203 / 221; C = 32 16 283 / 130, 24 209 / 117, 48 111 /
+// 118; C = 128 8 720 / 574, 24 380 / 443.  Distinct slots, C = 64, 200k edges: 2 687 / 376, 16 296 / 333.  1,000 nodes of 20
+// edges, C = 64: 10 / 16.
+bool split_nodes(int64_t n_edges, int64_t n_nodes, double enough, double some) {
+  const double degree = static_cast<double>(n_edges) / static_cast<double>(n_nodes);
+  return degree >= enough || (n_nodes < 4096 && degree >= some);
+}
+dim3 node_grid(int64_t n_nodes, bool split) {
+  return launch_grid(split ? n_nodes : (n_nodes + kWaves - 1) / kWaves, kBlock);
+}
+
+template <bool kFirst, typename A, typename B>
+struct conditional { using type = A; };
+template <typename A, typename B>
+struct conditional<false, A, B> { using type = B; };
+template <bool kFirst, typename A, typename B>
+using conditional_t = typename conditional<kFirst, A, B>::type;
 
 // The waves' partial sums of a node, in wave order.
 template <int N, typename T>
@@ -743,18 +778,21 @@ __device__ __forceinline__ T node_total(const T (&partial)[N]) {
 
 // Distinct slots: lane owns (slot s, chunk c) pairs q = s * row_chunks + c of
 // one edge's radial block; RC = row_chunks lanes share a slot (power of two).
-template <int V, int CPL, int RC, bool kOrdered>
-__global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_distinct_kernel(
+template <int V, int CPL, int RC, int NW, bool kOrdered>
+__global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
     const float* __restrict__ grad_output, const float* __restrict__ zonal,
     const float* __restrict__ radial, const int64_t* __restrict__ offsets,
     const int64_t* __restrict__ order, const int64_t* __restrict__ radial_slot,
     const float* __restrict__ inv, float* __restrict__ grad_zonal, float* __restrict__ grad_radial,
     float* __restrict__ grad_inv, int64_t n_edges, int64_t n_nodes, int64_t n_rows,
     int64_t n_radial, int64_t channels) {
-  __shared__ double inv_sum[kNodeWaves];
-  const int64_t node = block_index();
-  if (node >= n_nodes) return;
+  // the row before inv, the wave's edges: split over waves in 64 bits, so that the split costs no accuracy
+  using Sum = conditional_t<(NW > 1), double, float>;
+  __shared__ Sum inv_sum[NW];
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int member = NW > 1 ? wave : 0;
+  const int64_t node = NW > 1 ? block_index() : block_index() * kWaves + wave;
+  if (node >= n_nodes) return;
   const int lane = threadIdx.x & 63;
   const int64_t chunks = n_radial * RC;
   const int64_t edge_stride = n_radial * channels;
@@ -765,7 +803,7 @@ __global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_distinct_kernel(
   // addresses in registers.
   uint32_t col_at[CPL], zon_at[CPL], out_at[CPL], gz_at[CPL];
   fvec<V> g[CPL];
-  double pre[CPL][V];  // the row before inv, the wave's edges: in 64 bits, so that the split costs no accuracy
+  Sum pre[CPL][V];
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
     const int64_t q = lane + 64 * j;
@@ -788,13 +826,13 @@ __global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_distinct_kernel(
       for (int i = 0; i < V; ++i) g[j].v[i] = 0.0f;
     }
 #pragma unroll
-    for (int i = 0; i < V; ++i) pre[j][i] = 0.0;
+    for (int i = 0; i < V; ++i) pre[j][i] = 0;
   }
   const int64_t radial_bytes = edge_stride * 4, zonal_bytes = n_rows * 4;
 
   int64_t begin, end;
   segment_bounds(offsets, node, n_edges, begin, end);
-  for (int64_t slot = begin + wave; slot < end; slot += kNodeWaves) {
+  for (int64_t slot = begin + member; slot < end; slot += NW) {
     const int64_t e = uniform_i64(edge_of<kOrdered>(order, slot, n_edges));
     if (kOrdered && e < 0) continue;
     const BufferView rv = buffer_view(radial + e * edge_stride, radial_bytes);
@@ -818,7 +856,8 @@ __global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_distinct_kernel(
       fvec<V> out;
 #pragma unroll
       for (int i = 0; i < V; ++i) {
-        pre[j][i] = __builtin_fma(static_cast<double>(z[j]), static_cast<double>(x[j].v[i]), pre[j][i]);
+        if constexpr (NW > 1) pre[j][i] = __builtin_fma(static_cast<double>(z[j]), static_cast<double>(x[j].v[i]), pre[j][i]);
+        else pre[j][i] = pre[j][i] + z[j] * x[j].v[i];
         const float h = g[j].v[i] * sc;
         dot = dot + h * x[j].v[i];
         out.v[i] = h * z[j];
@@ -829,15 +868,22 @@ __global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_distinct_kernel(
     }
   }
   if (grad_inv != nullptr) {
-    double total = 0.0;
+    Sum total = 0;
 #pragma unroll
     for (int j = 0; j < CPL; ++j)
 #pragma unroll
-      for (int i = 0; i < V; ++i) total = __builtin_fma(static_cast<double>(g[j].v[i]), pre[j][i], total);
+      for (int i = 0; i < V; ++i) {
+        if constexpr (NW > 1) total = __builtin_fma(static_cast<double>(g[j].v[i]), pre[j][i], total);
+        else total = total + g[j].v[i] * pre[j][i];
+      }
     total = group_sum<64>(total);
-    if (lane == 0) inv_sum[wave] = total;
-    __syncthreads();
-    if (threadIdx.x == 0) grad_inv[node] = static_cast<float>(node_total(inv_sum));
+    if constexpr (NW > 1) {
+      if (lane == 0) inv_sum[wave] = total;
+      __syncthreads();
+      if (threadIdx.x == 0) grad_inv[node] = static_cast<float>(node_total(inv_sum));
+    } else {
+      if (lane == 0) grad_inv[node] = total;
+    }
   }
 }
 
@@ -998,8 +1044,8 @@ __global__ __launch_bounds__(kBlock) void gie_backward_shared_kernel(
 // 64 channels one slot 246 -> 230.
 constexpr int kEdgeLaneRowFloats = 4096;  // upstream floats staged per workgroup (16 KB)
 
-template <int RC, int S, int ZR, bool kOrdered>
-__global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_edge_lanes_kernel(
+template <int RC, int S, int ZR, int NW, bool kOrdered>
+__global__ __launch_bounds__(kBlock) void gie_backward_edge_lanes_kernel(
     const float* __restrict__ grad_output, const float* __restrict__ zonal,
     const float* __restrict__ radial, const int64_t* __restrict__ offsets,
     const int64_t* __restrict__ order, const int64_t* __restrict__ radial_slot,
@@ -1009,22 +1055,25 @@ __global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_edge_lanes_kerne
   constexpr int V = 8;
   constexpr int EW = 64 / RC;        // edges per wave step
   constexpr int UU = 2;              // wave steps whose loads go out together
-  extern __shared__ float g_rows[];  // [rows * C]: the node's upstream rows
-  __shared__ float inv_sum[kNodeWaves];
+  extern __shared__ float staged[];  // [nodes of the workgroup][rows * C]: their upstream rows
+  __shared__ float inv_sum[NW];
   const int wave = threadIdx.x >> 6;
-  const int64_t node = block_index();
-  if (node >= n_nodes) return;
+  const int member = NW > 1 ? wave : 0;
+  const int64_t node = NW > 1 ? block_index() : block_index() * kWaves + wave;
+  if (node >= n_nodes) return;  // the whole workgroup, or a wave that shares nothing
   const int lane = threadIdx.x & 63;
   const int u = lane / RC, c = lane % RC;
   const int rows = static_cast<int>(n_rows);
   const int64_t edge_stride = S * channels;
   const float scale = inv[node];
+  float* g_rows = staged + (NW > 1 ? 0 : wave * rows * channels);
 
   // the node's upstream rows 1..R into its LDS
   const float* upstream = grad_output + (node * (n_rows + 1) + 1) * channels;
-  for (int64_t q = threadIdx.x; q < rows * channels / 4; q += kNodeWaves * 64)
+  for (int64_t q = member * 64 + lane; q < rows * channels / 4; q += NW * 64)
     store_vec<4>(g_rows + 4 * q, load_vec<4>(upstream + 4 * q));
-  __syncthreads();
+  if constexpr (NW > 1) __syncthreads();
+  else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 
   // the rows in slot order: lane k holds the k-th row of the slot-major list; first[s] bounds slot s
   int slot_of_row = lane < rows ? static_cast<int>(radial_slot[lane]) : -1;
@@ -1050,7 +1099,7 @@ __global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_edge_lanes_kerne
   float inv_partial = 0.0f;
   int64_t begin, end;
   segment_bounds(offsets, node, n_edges, begin, end);
-  for (int64_t base = begin + wave * (UU * EW); base < end; base += kNodeWaves * UU * EW) {
+  for (int64_t base = begin + member * (UU * EW); base < end; base += NW * UU * EW) {
     int64_t e[UU];
     float x[UU][S][V], zq[UU][ZR];
 #pragma unroll
@@ -1135,9 +1184,13 @@ __global__ __launch_bounds__(kNodeWaves * 64) void gie_backward_edge_lanes_kerne
   }
   if (grad_inv != nullptr) {
     const float total = group_sum<64>(inv_partial);
-    if (lane == 0) inv_sum[wave] = total;
-    __syncthreads();
-    if (threadIdx.x == 0) grad_inv[node] = node_total(inv_sum);
+    if constexpr (NW > 1) {
+      if (lane == 0) inv_sum[wave] = total;
+      __syncthreads();
+      if (threadIdx.x == 0) grad_inv[node] = node_total(inv_sum);
+    } else {
+      if (lane == 0) grad_inv[node] = total;
+    }
   }
 }
 
@@ -1301,11 +1354,13 @@ int launch_distinct(int cpl, const float* grad_output, const float* zonal, const
                     const float* inv, float* grad_zonal, float* grad_radial, float* grad_inv,
                     int64_t n_edges, int64_t n_nodes, int64_t n_rows, int64_t n_radial,
                     int64_t channels, hipStream_t stream) {
-  const dim3 grid = launch_grid(n_nodes, kNodeWaves * 64);
-#define DPA4K_GIE_DIST(C)                                                                     \
-  gie_backward_distinct_kernel<V, C, RC, kOrdered><<<grid, kNodeWaves * 64, 0, stream>>>(             \
+  const bool split = split_nodes(n_edges, n_nodes, 12.0, 4.0);
+  const dim3 grid = node_grid(n_nodes, split);
+#define DPA4K_GIE_DIST_NW(C, NW)                                                              \
+  gie_backward_distinct_kernel<V, C, RC, NW, kOrdered><<<grid, kBlock, 0, stream>>>(          \
       grad_output, zonal, radial, offsets, order, radial_slot, inv, grad_zonal, grad_radial,  \
       grad_inv, n_edges, n_nodes, n_rows, n_radial, channels)
+#define DPA4K_GIE_DIST(C) if (split) DPA4K_GIE_DIST_NW(C, kNodeWaves); else DPA4K_GIE_DIST_NW(C, 1)
   switch (cpl) {
     case 1: DPA4K_GIE_DIST(1); break;
     case 2: DPA4K_GIE_DIST(2); break;
@@ -1313,6 +1368,7 @@ int launch_distinct(int cpl, const float* grad_output, const float* zonal, const
     default: DPA4K_GIE_DIST(8); break;
   }
 #undef DPA4K_GIE_DIST
+#undef DPA4K_GIE_DIST_NW
   return launched("gie_backward_distinct_kernel");
 }
 
@@ -1436,14 +1492,18 @@ int dispatch_edge_lanes(const float* grad_output, const float* zonal, const floa
                         const int64_t* order, const int64_t* radial_slot, const float* inv, float* grad_zonal,
                         float* grad_radial, float* grad_inv, int64_t n_edges, int64_t n_nodes, int64_t n_rows,
                         int64_t n_radial, int64_t channels, hipStream_t stream) {
-  const dim3 grid = launch_grid(n_nodes, kNodeWaves * 64);
-  const size_t lds = sizeof(float) * static_cast<size_t>(n_rows * channels);
   const int rc = static_cast<int>(channels / 8);
+  const double step = 128.0 / rc;  // edges of a wave step
+  const bool split = split_nodes(n_edges, n_nodes, (grad_inv != nullptr ? 2.5 : 1.5) * step, rc == 4 ? 0.5 * step : step);
+  const dim3 grid = node_grid(n_nodes, split);
+  const size_t lds = sizeof(float) * static_cast<size_t>(n_rows * channels) * (split ? 1 : kWaves);
   const int zr = n_rows <= 2 * rc ? 2 : 4;
-#define DPA4K_GIE_EDGE_LANES(RC, S, ZR)                                                                 \
-  gie_backward_edge_lanes_kernel<RC, S, ZR, kOrdered><<<grid, kNodeWaves * 64, lds, stream>>>(         \
+#define DPA4K_GIE_EDGE_LANES_NW(RC, S, ZR, NW)                                                          \
+  gie_backward_edge_lanes_kernel<RC, S, ZR, NW, kOrdered><<<grid, kBlock, lds, stream>>>(              \
       grad_output, zonal, radial, offsets, order, radial_slot, inv, grad_zonal, grad_radial, grad_inv, \
       n_edges, n_nodes, n_rows, channels)
+#define DPA4K_GIE_EDGE_LANES(RC, S, ZR) \
+  if (split) DPA4K_GIE_EDGE_LANES_NW(RC, S, ZR, kNodeWaves); else DPA4K_GIE_EDGE_LANES_NW(RC, S, ZR, 1)
 #define DPA4K_GIE_EDGE_LANES_S(RC, ZR)            \
   switch (n_radial) {                               \
     case 1: DPA4K_GIE_EDGE_LANES(RC, 1, ZR); break; \
@@ -1460,6 +1520,7 @@ int dispatch_edge_lanes(const float* grad_output, const float* zonal, const floa
   }
 #undef DPA4K_GIE_EDGE_LANES_S
 #undef DPA4K_GIE_EDGE_LANES
+#undef DPA4K_GIE_EDGE_LANES_NW
   return launched("gie_backward_edge_lanes_kernel");
 }
 

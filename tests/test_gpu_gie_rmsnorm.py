@@ -534,3 +534,32 @@ def test_gie_backward_node_in_one_workgroup(slots, n_radial, channels, shuffle):
     truth = zonal_scatter_backward_f64(up, *inputs)
     for label, actual, wanted, exact in zip(("zonal", "radial", "inverse"), grads, oracle, truth):
         assert_gradient(actual, wanted, exact, f"grad {label}")
+
+
+@pytest.mark.parametrize("slots,n_radial,channels", [
+    (_DEEPMD_SLOTS, 3, 32), ([0] * 3, 1, 32), ([0] * 3, 1, 64), ([0] * 3, 1, 128), (_DEEPMD_SLOTS, 3, 64),
+    (_DEEPMD_SLOTS, 3, 128), (list(range(15)), 15, 64), (list(range(24)), 24, 2)])
+@pytest.mark.parametrize("shuffle", [False, True], ids=["sorted", "shuffled"])
+def test_gie_wave_per_node(slots, n_radial, channels, shuffle):
+    """Graphs of many nodes and a low mean degree: a wave per node in the backward, short rounds in the forward, with
+    segments of every length among them."""
+    announce("gie waves per node", slots, n_radial, channels, shuffle)
+    degrees = torch.tensor([0, 1, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33, 65, 0, 129, 1, 2] + [0, 1, 2] * 1401)
+    generator = torch.Generator().manual_seed(channels + n_radial)
+    dst = torch.repeat_interleave(torch.arange(degrees.numel()), degrees)
+    zonal = torch.randn((dst.numel(), len(slots)), generator=generator)
+    radial = torch.randn((dst.numel(), n_radial, channels), generator=generator)
+    inverse = torch.rsqrt(degrees.to(torch.float32) + 1.0)
+    if shuffle:
+        dst = dst[torch.randperm(dst.numel(), generator=generator)]
+    inputs = zonal, radial, dst, torch.tensor(slots), inverse
+    up = torch.randn((degrees.numel(), len(slots) + 1, channels), generator=generator)
+    z, r, d, k, inv = _to(inputs)
+    leaves = [t.requires_grad_(True) for t in (z, r, inv)]
+    out = kernels.zonal_scatter(z, r, d, k, inv)
+    assert_bitwise(out, gie_ref.zonal_scatter_reference(*inputs), "forward")
+    grads = torch.autograd.grad(out, leaves, up.to(DEV))
+    oracle = gie_ref.zonal_scatter_backward_reference(up, *inputs)
+    truth = zonal_scatter_backward_f64(up, *inputs)
+    for label, actual, wanted, exact in zip(("zonal", "radial", "inverse"), grads, oracle, truth):
+        assert_gradient(actual, wanted, exact, f"grad {label}")
