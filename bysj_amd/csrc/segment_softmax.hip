@@ -184,16 +184,12 @@ constexpr int short_capacity(int v, int lc) { return (24 / v) * ((lc > 32 ? lc :
 // Lanes per short group: 32, or LC when a row is wider.  (16-lane groups
 // with twice the tiles fit a config-2-like graph into one dispatch round
 // but need over 96 VGPRs, which halves the occupancy, and ran slower.)
-constexpr int short_group_log(int v, int log_lc, bool backward) {
-  (void)v;
-  (void)backward;
-  return log_lc > 5 ? log_lc : 5;
-}
+constexpr int short_group_log(int log_lc) { return log_lc > 5 ? log_lc : 5; }
 
-template <int V, int LOG_LC, bool kBackward = false>
+template <int V, int LOG_LC>
 struct Geo {
   static constexpr int LC = 1 << LOG_LC;               // lanes per edge row
-  static constexpr int LOG_G = short_group_log(V, LOG_LC, kBackward);
+  static constexpr int LOG_G = short_group_log(LOG_LC);
   static constexpr int G = 1 << LOG_G;                 // lanes per short segment
   static constexpr int GPW = 64 / G;                   // short segments per wave
   static constexpr int PG = G / LC;                    // rows per group load
@@ -263,11 +259,10 @@ struct Tiles {
   }
 };
 
-// Lane roles inside a workgroup for rows of LC lanes (short groups of the
-// forward or the backward geometry).
-template <int V, int LOG_LC, bool kBackward = false>
+// Lane roles inside a workgroup for rows of LC lanes.
+template <int V, int LOG_LC>
 struct Lanes {
-  using S = Geo<V, LOG_LC, kBackward>;
+  using S = Geo<V, LOG_LC>;
   int lane, wave, k, p, pb, gidx;
   bool live;
   int64_t column;
@@ -766,7 +761,7 @@ __device__ __forceinline__ Tiles<R, STEP, kOrdered> backward_tiles(const Backwar
 // grad_logit rows of the tiles from alpha, grad_alpha and the segment's S;
 // grad_env of each row from the row sum over the LC lanes of the row.
 template <int V, int LOG_LC, int R, int STEP, bool kOrdered>
-__device__ __forceinline__ void backward_rows(const BackwardArgs& a, const Lanes<V, LOG_LC, true>& L,
+__device__ __forceinline__ void backward_rows(const BackwardArgs& a, const Lanes<V, LOG_LC>& L,
                                               const Tiles<R, STEP, kOrdered>& t, int64_t column,
                                               const float (&x)[R][V], const float (&g)[R][V],
                                               const float (&expect)[V], const float (&envelope)[R],
@@ -806,7 +801,7 @@ __device__ void backward_long(const BackwardArgs& a, int64_t segment, int64_t be
   begin = uniform_i64(begin);  // one segment per workgroup
   end = uniform_i64(end);
   constexpr int LC = S::LC, PB = S::PB, RMAXB = S::RMAXB;
-  const Lanes<V, LOG_LC, true> L(a.channels / V);
+  const Lanes<V, LOG_LC> L(a.channels / V);
   const int64_t column = L.live ? L.column : 0;
   const int64_t degree = end - begin;
   float a0[V], g0[V], expect[V];
@@ -885,9 +880,9 @@ __device__ void backward_long(const BackwardArgs& a, int64_t segment, int64_t be
 template <int V, int LOG_LC, bool kNull, bool kOrdered>
 __device__ __forceinline__ void backward_short(const BackwardArgs& a, int64_t segment, int64_t begin, int64_t end,
                                                int64_t base) {
-  using S = Geo<V, LOG_LC, true>;
+  using S = Geo<V, LOG_LC>;
   constexpr int LC = S::LC, G = S::G, PG = S::PG, RMAX = S::RMAX;
-  const Lanes<V, LOG_LC, true> L(a.channels / V);
+  const Lanes<V, LOG_LC> L(a.channels / V);
   const int64_t column = L.live ? L.column : 0;
   float a0[V], g0[V], expect[V];
 #pragma unroll
@@ -926,7 +921,7 @@ __device__ __forceinline__ void backward_short(const BackwardArgs& a, int64_t se
 template <int V, int LOG_LC, bool kNull, bool kOrdered, bool kPlanned>
 __global__ __launch_bounds__(kBlock) void softmax_backward_kernel(BackwardArgs a, const int64_t* __restrict__ plan,
                                                                   int64_t n_long) {
-  using S = Geo<V, LOG_LC, true>;
+  using S = Geo<V, LOG_LC>;
   __shared__ float partial[kWaves][2][S::LC * V];
   constexpr bool planned = kPlanned;
   const int64_t block = block_index();
@@ -1073,7 +1068,7 @@ struct SlabRows {
 };
 
 // The logit chunks and envelopes of every tile, all loads issued before any use.
-template <int LOG_LS, int R, typename Id>
+template <int LOG_LS, int R, bool kKeep = false, typename Id>
 __device__ __forceinline__ void slab_forward_loads(const ForwardArgs& a, SlabRows<LOG_LS, R, Id>& t, int64_t column,
                                                    float (&value)[R][4], float (&envelope)[R]) {
   t.find(a.order, a.n_edges);
@@ -1082,7 +1077,7 @@ __device__ __forceinline__ void slab_forward_loads(const ForwardArgs& a, SlabRow
     const BufferView env = t.view(a.env, 1);
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      const fvec<4> x = buffer_load_vec<4, kRowPolicy<Id>>(logit, t.at(i));
+      const fvec<4> x = buffer_load_vec<4, kKeep ? 0 : kRowPolicy<Id>>(logit, t.at(i));
       envelope[i] = buffer_load_f32(env, t.scalar_at(i));
 #pragma unroll
       for (int v = 0; v < 4; ++v) value[i][v] = x.v[v];
@@ -1091,7 +1086,8 @@ __device__ __forceinline__ void slab_forward_loads(const ForwardArgs& a, SlabRow
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int64_t e = t.edge(i);
-      const fvec<4> x = load_chunk_stream(a.logit + e * a.channels + column);
+      const float* row = a.logit + e * a.channels + column;
+      const fvec<4> x = kKeep ? load_chunk(row) : load_chunk_stream(row);
       envelope[i] = a.env[e];
 #pragma unroll
       for (int v = 0; v < 4; ++v) value[i][v] = x.v[v];
@@ -1200,7 +1196,7 @@ __global__ __launch_bounds__(kBlock) void softmax_forward_slab_kernel(ForwardArg
     for (int64_t base = begin; base < end; base += CAP) {
       T t(base, end, live, column, a.channels);
       float value[R][4], envelope[R];
-      slab_forward_loads(a, t, column, value, envelope);
+      slab_forward_loads<LOG_LS, R, true>(a, t, column, value, envelope);
       // a round's maximum first, then one rescale and the round's terms
 #pragma unroll
       for (int i = 0; i < R; ++i) {
@@ -1249,7 +1245,7 @@ __global__ __launch_bounds__(kBlock) void softmax_forward_slab_kernel(ForwardArg
 }
 
 // alpha and grad_alpha chunks of every tile (zeros without a row).
-template <int LOG_LS, int R, typename Id>
+template <int LOG_LS, int R, bool kKeep = false, typename Id>
 __device__ __forceinline__ void slab_backward_loads(const BackwardArgs& a, SlabRows<LOG_LS, R, Id>& t,
                                                     int64_t column, float (&x)[R][4], float (&g)[R][4]) {
   t.find(a.order, a.n_edges);
@@ -1258,8 +1254,8 @@ __device__ __forceinline__ void slab_backward_loads(const BackwardArgs& a, SlabR
     const BufferView grad = t.view(a.grad_alpha, a.channels);
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      const fvec<4> xv = buffer_load_vec<4, kRowPolicy<Id>>(alpha, t.at(i));
-      const fvec<4> gv = buffer_load_vec<4, kRowPolicy<Id>>(grad, t.at(i));
+      const fvec<4> xv = buffer_load_vec<4, kKeep ? 0 : kRowPolicy<Id>>(alpha, t.at(i));
+      const fvec<4> gv = buffer_load_vec<4, kKeep ? 0 : kRowPolicy<Id>>(grad, t.at(i));
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         x[i][v] = xv.v[v];
@@ -1271,8 +1267,9 @@ __device__ __forceinline__ void slab_backward_loads(const BackwardArgs& a, SlabR
 #pragma unroll
     for (int i = 0; i < R; ++i) {
       const int64_t e = t.edge(i);
-      const fvec<4> xv = load_chunk_stream(a.alpha + e * a.channels + column);
-      const fvec<4> gv = load_chunk_stream(a.grad_alpha + e * a.channels + column);
+      const float *alpha = a.alpha + e * a.channels + column, *grad = a.grad_alpha + e * a.channels + column;
+      const fvec<4> xv = kKeep ? load_chunk(alpha) : load_chunk_stream(alpha);
+      const fvec<4> gv = kKeep ? load_chunk(grad) : load_chunk_stream(grad);
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         x[i][v] = xv.v[v];
@@ -1406,7 +1403,7 @@ __global__ __launch_bounds__(SW == 1 ? kBlock : SW * 64) void softmax_backward_s
     } else {
       for (int64_t base = begin; base < end; base += CAP) {
         T t(base, end, live, column, a.channels);
-        slab_backward_loads(a, t, column, x, g);
+        slab_backward_loads<LOG_LS, R, true>(a, t, column, x, g);
         add_products(x, g, R);
       }
       split();
@@ -1531,25 +1528,48 @@ int lanes_log_for(int64_t chunks) {
   return log;
 }
 
-// Rows of at most two aligned chunks (C = 4, 8) and of fewer than four
-// columns run the lane-group kernels, everything else the slab kernels.
-bool uses_slabs(int64_t channels, bool vec4) { return channels > 4 && !(channels == 8 && vec4); }
+// Mean degree of a graph with at least one segment.
+double mean_degree(int64_t n_edges, int64_t n_nodes) {
+  return static_cast<double>(n_edges) / static_cast<double>(n_nodes);
+}
+
+// Whether the slab kernels run these rows.  Aligned rows of two chunks (C = 8) and rows of up to four
+// columns run the lane-group kernels, rows past 256 columns and rows that are not whole aligned chunks the slab kernels.
+// Between, the lane groups take the mean degrees at which slabs are mostly empty or re-read their segments.  Lane
+// groups against slabs, forward / backward, 96 MB of logits, us:
+//   C = 16   degree 8 54 / 78 and 70 / 115, 12 44 / 61 and 70 / 92, 20 35 / 50 and 50 / 64 (gathered 81 / 129 and 81 / 129),
+//            60 66 / 84 and 36 / 54, 90 47 / 63 and 35 / 52, 150 36 / 50 and 43 / 60, 200 35 / 48 and 44 / 65
+//   C = 32   8 35 / 52 and 60 / 100, 12 35 / 49 and 44 / 70, 20 43 / 59 and 35 / 52, 30 61 / 79 and 38 / 53, 60 36 / 53 and
+//            34 / 53, 90 34 / 47 and 37 / 53, 150 52 / 78 and 42 / 62, 300 55 / 81 and 47 / 73
+//   C = 128  5 53 / 67 and 83 / 138, 12 52 / 62 and 44 / 68, 16 41 / 53 and 37 / 56, 30 46 / 63 and 37 / 53, 90 60 / 84 and
+//            37 / 52, 200 62 / 86 and 40 / 68
+// 64 segments of 12,000 rows and more take twice as long as slabs up to 32 columns, and half as long past that.  At
+// degrees of 20 to 100 the sums stay in 64 bits also where lane groups, whose sums have 32, would be up to 1.4 times as
+// fast (C = 16, degree 20).
+bool uses_slabs(int64_t channels, bool vec4, int64_t n_edges, int64_t n_nodes) {
+  if (channels <= 4 || (vec4 && channels == 8)) return false;
+  if (!vec4 || channels > 256) return true;
+  const double degree = mean_degree(n_edges, n_nodes);
+  if (channels <= 16) return degree >= 20.0 && degree <= 112.0;
+  if (channels <= 32) return degree >= 18.0 && (degree <= 130.0 || (degree <= 1000.0 && n_nodes >= 1024));
+  return degree >= 14.0;
+}
 
 // Short-path capacity of the lane-group kernel that runs `channels` with
 // (vec4) or without 128-bit rows; 0 for the slab kernels (no plan use).
-int64_t capacity_for(int64_t channels, bool vec4) {
-  if (uses_slabs(channels, vec4)) return 0;
+int64_t capacity_for(int64_t channels, bool vec4, int64_t n_edges, int64_t n_nodes) {
+  if (uses_slabs(channels, vec4, n_edges, n_nodes)) return 0;
   return short_capacity(vec4 ? 4 : 1, 1 << lanes_log_for(vec4 ? channels / 4 : channels));
 }
 
-int64_t short_blocks(int64_t n_nodes, int v, int log_lc, bool backward) {
-  const int64_t per_block = kBlock >> short_group_log(v, log_lc, backward);
+int64_t short_blocks(int64_t n_nodes, int log_lc) {
+  const int64_t per_block = kBlock >> short_group_log(log_lc);
   return (n_nodes + per_block - 1) / per_block;
 }
 
 template <int V, int LOG_LC>
 int launch_forward(const ForwardArgs& a, const int64_t* plan, int64_t n_long, hipStream_t stream) {
-  const dim3 grid = launch_grid((plan != nullptr ? n_long : 0) + short_blocks(a.n_nodes, V, LOG_LC, false), kBlock);
+  const dim3 grid = launch_grid((plan != nullptr ? n_long : 0) + short_blocks(a.n_nodes, LOG_LC), kBlock);
 #define DPA4K_SOFTMAX_FWD(NULLV, ORD)                                                                      \
   (plan != nullptr                                                                                        \
        ? softmax_forward_kernel<V, LOG_LC, NULLV, ORD, true>                                               \
@@ -1566,7 +1586,7 @@ int launch_forward(const ForwardArgs& a, const int64_t* plan, int64_t n_long, hi
 
 template <int V, int LOG_LC>
 int launch_backward(const BackwardArgs& a, const int64_t* plan, int64_t n_long, hipStream_t stream) {
-  const dim3 grid = launch_grid((plan != nullptr ? n_long : 0) + short_blocks(a.n_nodes, V, LOG_LC, true), kBlock);
+  const dim3 grid = launch_grid((plan != nullptr ? n_long : 0) + short_blocks(a.n_nodes, LOG_LC), kBlock);
 #define DPA4K_SOFTMAX_BWD(NULLV, ORD)                                                                       \
   (plan != nullptr                                                                                         \
        ? softmax_backward_kernel<V, LOG_LC, NULLV, ORD, true>                                               \
@@ -1582,11 +1602,20 @@ int launch_backward(const BackwardArgs& a, const int64_t* plan, int64_t n_long, 
 }
 
 // Rows a slab wave holds in registers: the mean degree and 3.5 of its standard
-// deviations (Poisson), so that only outliers are streamed; 64, 96 or 128.
-int slab_rows(int64_t n_edges, int64_t n_nodes) {
-  const double mean = static_cast<double>(n_edges) / static_cast<double>(n_nodes);
+// deviations (Poisson), or nearly, so that only outliers are streamed.  Every
+// tile costs instructions also where it holds no rows (C = 64, degree 16: 37 /
+// 56 us with 32 rows, 54 / 74 with 64), so the rows are not more than needed.  Slabs of four chunks have
+// registers for 256 rows (C = 13, degree 200 through an order), of two for 512;
+// slabs of four take 128 from a degree of 48 on (C = 16, two populations of
+// degree 20 and 100 through an order: 110 / 171 us with 96, 83 / 130 with 128).
+int slab_rows(int64_t n_edges, int64_t n_nodes, int log_ls) {
+  const double mean = mean_degree(n_edges, n_nodes);
   const double rows = mean + 3.5 * sqrt(mean);
-  return rows <= 64.0 ? 64 : (rows <= 96.0 ? 96 : 128);
+  if (rows <= 40.0) return 32;
+  if (rows <= 72.0) return 64;
+  if (rows <= 100.0 && log_ls >= 2) return log_ls == 2 ? 128 : 96;
+  if (rows <= 140.0 || log_ls == 3) return 128;
+  return rows <= 300.0 || log_ls == 2 ? 256 : 512;
 }
 
 // Natural order through 32-bit view offsets, edge ids in 32 bits, or in 64.
@@ -1604,8 +1633,14 @@ int launch_forward_slabs(const ForwardArgs& a, int rows, int64_t slabs, int shif
   constexpr int PR = 64 >> LOG_LS;
   const dim3 grid = launch_grid((a.n_nodes * slabs + kWaves - 1) / kWaves, kBlock);
   if constexpr (!__is_same(Id, int64_t)) {
+    if (rows == 32) softmax_forward_slab_kernel<LOG_LS, 32 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
     if (rows == 64) softmax_forward_slab_kernel<LOG_LS, 64 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
-    if (rows == 96) softmax_forward_slab_kernel<LOG_LS, 96 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
+    if constexpr (LOG_LS == 3)
+      if (rows == 96) softmax_forward_slab_kernel<LOG_LS, 96 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
+    if constexpr (LOG_LS == 1)
+      if (rows == 512) softmax_forward_slab_kernel<LOG_LS, 512 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
+    if constexpr (LOG_LS < 3)
+      if (rows == 256) softmax_forward_slab_kernel<LOG_LS, 256 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
     if (rows != 128) return launched("softmax_forward_slab_kernel");
   }
   softmax_forward_slab_kernel<LOG_LS, 128 / PR, Id><<<grid, kBlock, 0, stream>>>(a, slabs, shift);
@@ -1618,8 +1653,14 @@ int launch_backward_slabs_of(const BackwardArgs& a, int rows, int64_t slabs, int
   constexpr int kThreads = SW == 1 ? kBlock : SW * 64;
   const dim3 grid = launch_grid(SW == 1 ? (a.n_nodes + kWaves - 1) / kWaves : a.n_nodes, kThreads);
   if constexpr (!__is_same(Id, int64_t)) {
+    if (rows == 32) softmax_backward_slab_kernel<LOG_LS, 32 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
     if (rows == 64) softmax_backward_slab_kernel<LOG_LS, 64 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
-    if (rows == 96) softmax_backward_slab_kernel<LOG_LS, 96 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
+    if constexpr (LOG_LS == 3)
+      if (rows == 96) softmax_backward_slab_kernel<LOG_LS, 96 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
+    if constexpr (LOG_LS == 1)
+      if (rows == 512) softmax_backward_slab_kernel<LOG_LS, 512 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
+    if constexpr (LOG_LS < 3)
+      if (rows == 256) softmax_backward_slab_kernel<LOG_LS, 256 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
     if (rows != 128) return launched("softmax_backward_slab_kernel");
   }
   softmax_backward_slab_kernel<LOG_LS, 128 / PR, SW, Id><<<grid, kThreads, 0, stream>>>(a, slabs, shift);
@@ -1658,7 +1699,7 @@ int forward_slabs(const ForwardArgs& a, hipStream_t stream) {
                                                overlap(a.null_alpha, a.null_logit, a.n_nodes * a.channels));
   const int log_ls = slab_lanes_log(a.channels);
   const int64_t slabs = ((a.channels + 3) / 4 + shift + (1 << log_ls) - 1) >> log_ls;
-  const int rows = slab_rows(a.n_edges, a.n_nodes);
+  const int rows = slab_rows(a.n_edges, a.n_nodes, log_ls);
   if (!grid_fits(a.n_nodes * slabs, kBlock)) return fail(DPA4K_EINVAL, "segment softmax: grid too large");
   switch (row_ids(a.order, a.n_edges, a.channels)) {
     case RowIds::kViews: return DPA4K_SLABS(launch_forward_slabs, Views);
@@ -1676,7 +1717,7 @@ int backward_slabs(const BackwardArgs& a, hipStream_t stream) {
                                  overlap(a.grad_null_logit, a.null_alpha, null_elements));
   const int log_ls = slab_lanes_log(a.channels);
   const int64_t slabs = ((a.channels + 3) / 4 + shift + (1 << log_ls) - 1) >> log_ls;
-  const int rows = slab_rows(a.n_edges, a.n_nodes);
+  const int rows = slab_rows(a.n_edges, a.n_nodes, log_ls);
   switch (row_ids(a.order, a.n_edges, a.channels)) {
     case RowIds::kViews: return DPA4K_SLABS(launch_backward_slabs, Views);
     case RowIds::kSharedViews: return launch_backward_slabs<3, SharedViews>(a, rows, slabs, shift, stream);
@@ -1709,12 +1750,22 @@ int softmax_forward(const float* logit, const float* env, const int64_t* offsets
   const bool vec4 = channels % 4 == 0 && aligned16(logit) && aligned16(alpha) &&
                     (null_logit == nullptr || (aligned16(null_logit) && aligned16(null_alpha)));
   const ForwardArgs a{logit, env, offsets, null_logit, order, alpha, null_alpha, n_edges, n_nodes, channels};
-  if (uses_slabs(channels, vec4)) return forward_slabs(a, stream);
+  if (uses_slabs(channels, vec4, n_edges, n_nodes)) return forward_slabs(a, stream);
   // a plan applies only to the geometry it was built for; otherwise run unplanned
-  const bool use_plan = plan != nullptr && plan_capacity == capacity_for(channels, vec4);
+  const bool use_plan = plan != nullptr && plan_capacity == capacity_for(channels, vec4, n_edges, n_nodes);
   const int64_t* words = use_plan ? static_cast<const int64_t*>(plan) : nullptr;
   const int64_t listed = use_plan ? n_long : 0;
-  if (vec4) return channels == 4 ? launch_forward<4, 0>(a, words, listed, stream) : launch_forward<4, 1>(a, words, listed, stream);
+  if (vec4) {
+    switch (lanes_log_for(channels / 4)) {
+      case 0: return launch_forward<4, 0>(a, words, listed, stream);
+      case 1: return launch_forward<4, 1>(a, words, listed, stream);
+      case 2: return launch_forward<4, 2>(a, words, listed, stream);
+      case 3: return launch_forward<4, 3>(a, words, listed, stream);
+      case 4: return launch_forward<4, 4>(a, words, listed, stream);
+      case 5: return launch_forward<4, 5>(a, words, listed, stream);
+      default: return launch_forward<4, 6>(a, words, listed, stream);
+    }
+  }
   if (channels == 1) return launch_forward<1, 0>(a, words, listed, stream);
   if (channels == 2) return launch_forward<1, 1>(a, words, listed, stream);
   return launch_forward<1, 2>(a, words, listed, stream);
@@ -1742,12 +1793,22 @@ int softmax_backward(const float* alpha, const float* grad_alpha, const float* e
                                    aligned16(grad_null_logit)));
   const BackwardArgs a{alpha, grad_alpha, env, offsets, null_alpha, grad_null_alpha, order,
                        grad_logit, grad_null_logit, grad_env, n_edges, n_nodes, channels};
-  if (uses_slabs(channels, vec4)) return backward_slabs(a, stream);
+  if (uses_slabs(channels, vec4, n_edges, n_nodes)) return backward_slabs(a, stream);
   // a plan applies only to the geometry it was built for; otherwise run unplanned
-  const bool use_plan = plan != nullptr && plan_capacity == capacity_for(channels, vec4);
+  const bool use_plan = plan != nullptr && plan_capacity == capacity_for(channels, vec4, n_edges, n_nodes);
   const int64_t* words = use_plan ? static_cast<const int64_t*>(plan) : nullptr;
   const int64_t listed = use_plan ? n_long : 0;
-  if (vec4) return channels == 4 ? launch_backward<4, 0>(a, words, listed, stream) : launch_backward<4, 1>(a, words, listed, stream);
+  if (vec4) {
+    switch (lanes_log_for(channels / 4)) {
+      case 0: return launch_backward<4, 0>(a, words, listed, stream);
+      case 1: return launch_backward<4, 1>(a, words, listed, stream);
+      case 2: return launch_backward<4, 2>(a, words, listed, stream);
+      case 3: return launch_backward<4, 3>(a, words, listed, stream);
+      case 4: return launch_backward<4, 4>(a, words, listed, stream);
+      case 5: return launch_backward<4, 5>(a, words, listed, stream);
+      default: return launch_backward<4, 6>(a, words, listed, stream);
+    }
+  }
   if (channels == 1) return launch_backward<1, 0>(a, words, listed, stream);
   if (channels == 2) return launch_backward<1, 1>(a, words, listed, stream);
   return launch_backward<1, 2>(a, words, listed, stream);
@@ -1796,7 +1857,7 @@ extern "C" int dpa4k_segment_softmax_plan(const int64_t* offsets, int64_t n_edge
   hipStream_t stream = as_stream(stream_handle);
   // The plan is for the 128-bit row kernel when C % 4 == 0 (operands from
   // torch's allocator are 16-byte aligned), for the scalar one otherwise.
-  const int64_t capacity = capacity_for(channels, channels % 4 == 0);
+  const int64_t capacity = capacity_for(channels, channels % 4 == 0, n_edges, n_nodes > 0 ? n_nodes : 1);
   int64_t* words = static_cast<int64_t*>(plan);
   // The slab kernels need no plan: an empty one, and no host synchronisation.
   const int64_t tiles = capacity > 0 ? plan_tiles(n_nodes) : 0;

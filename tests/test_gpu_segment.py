@@ -939,6 +939,49 @@ def test_segment_softmax_config2_full_size_and_determinism():
     assert_close_scaled(total, torch.ones_like(total), what="sum to one")
 
 
+_SOFTMAX_GRAPHS = {  # mean degrees on both sides of what picks the kernel and its rows, with outliers of every length
+    "1": [0, 1, 3, 0, 2] * 40, "10": [0, 9, 31, 1] * 20 + [25], "15": [15, 17, 14, 16] * 20 + [40, 0],
+    "25": [25, 31, 20, 33, 64, 65] * 8, "60": [60, 96, 97, 30, 71, 10] * 8, "100": [100, 128, 129, 70, 150, 48] * 6,
+    "200": [200, 256, 257, 140, 90, 300] * 5, "long": [1500, 0, 2700, 1]}
+
+
+@pytest.mark.parametrize("channels", [4, 5, 8, 12, 13, 16, 20, 32, 33, 60, 64, 128, 200, 256, 260])
+@pytest.mark.parametrize("graph", sorted(_SOFTMAX_GRAPHS))
+@pytest.mark.parametrize("ordered", [False, True])
+def test_segment_softmax_routes(channels, graph, ordered):
+    """Lane groups and slabs of every size, chosen by width and mean degree: results and gradients against the oracle and 64
+    bits, planned; the unplanned calls bit for bit the same."""
+    announce("softmax routes", channels, graph, ordered)
+    dst, offsets = _graph(_SOFTMAX_GRAPHS[graph])
+    order, order_dev = None, torch.empty(0, dtype=torch.int64, device=DEV)
+    if ordered:
+        dst, order, offsets = _shuffled(dst, channels)
+        order_dev = order.to(DEV)
+    edges, nodes, gen = dst.numel(), offsets.numel() - 1, torch.Generator().manual_seed(channels)
+    logit, up = (torch.randn(edges, channels, generator=gen) * 2.0 for _ in range(2))
+    null, up_null = (torch.randn(nodes, channels, generator=gen) for _ in range(2))
+    env = torch.rand(edges, generator=gen) + 0.05
+    env[::17] = 0.0
+    x, e, n = (t.to(DEV).requires_grad_(True) for t in (logit, env, null))
+    alpha, null_alpha = kernels.segment_softmax(x, e, offsets.to(DEV), n, order=None if order is None else order_dev)
+    e_alpha, e_null = ref.segment_softmax_reference(logit, env, dst, offsets, null)
+    assert_close_scaled(alpha, e_alpha, what="alpha")
+    assert_close_scaled(null_alpha, e_null, what="null_alpha")
+    grads = torch.autograd.grad((alpha, null_alpha), (x, e, n), (up.to(DEV), up_null.to(DEV)))
+    oracle = ref.segment_softmax_backward_reference(up, logit, env, dst, offsets, null, up_null)
+    truth = segment_softmax_backward_f64(up, logit, env, dst, nodes, null, up_null)
+    for got, wanted, exact, label in zip(grads, oracle, truth, ("logit", "env", "null")):
+        assert_gradient(got, wanted, exact, f"grad_{label}")
+    library, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    plain, plain_null = torch.empty_like(alpha), torch.empty_like(null_alpha)
+    ed, od, order_ptr = e.detach(), offsets.to(DEV), order_dev.data_ptr() if ordered else None
+    _lib.check(library.dpa4k_segment_softmax_forward(
+        x.data_ptr(), ed.data_ptr(), od.data_ptr(), n.data_ptr(), order_ptr, plain.data_ptr(), plain_null.data_ptr(),
+        edges, nodes, channels, stream))
+    assert_bitwise(plain, alpha.detach(), "unplanned alpha")
+    assert_bitwise(plain_null, null_alpha.detach(), "unplanned null_alpha")
+
+
 @pytest.mark.parametrize("channels", [3, 8, 13, 33, 66, 257, 290])
 @pytest.mark.parametrize("ordered", [False, True])
 def test_segment_softmax_in_place(channels, ordered):
