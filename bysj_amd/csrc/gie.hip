@@ -26,6 +26,8 @@
 // reading one slot, e.g. one radial channel per degree l) go through a
 // one-wave kernel that stages the per-row products in LDS and sums them per
 // slot in ascending row order.
+#include <type_traits>
+
 #include "common.h"
 
 namespace dpa4k {
@@ -760,13 +762,6 @@ dim3 node_grid(int64_t n_nodes, bool split) {
   return launch_grid(split ? n_nodes : (n_nodes + kWaves - 1) / kWaves, kBlock);
 }
 
-template <bool kFirst, typename A, typename B>
-struct conditional { using type = A; };
-template <typename A, typename B>
-struct conditional<false, A, B> { using type = B; };
-template <bool kFirst, typename A, typename B>
-using conditional_t = typename conditional<kFirst, A, B>::type;
-
 // The waves' partial sums of a node, in wave order.
 template <int N, typename T>
 __device__ __forceinline__ T node_total(const T (&partial)[N]) {
@@ -787,7 +782,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
     float* __restrict__ grad_inv, int64_t n_edges, int64_t n_nodes, int64_t n_rows,
     int64_t n_radial, int64_t channels) {
   // the row before inv, the wave's edges: split over waves in 64 bits, so that the split costs no accuracy
-  using Sum = conditional_t<(NW > 1), double, float>;
+  using Sum = std::conditional_t<(NW > 1), double, float>;
   __shared__ Sum inv_sum[NW];
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int member = NW > 1 ? wave : 0;
