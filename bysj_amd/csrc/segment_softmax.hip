@@ -12,13 +12,15 @@
 //
 // Work decomposition.  Rows of more than two 16-byte chunks are cut into slabs
 // of up to 8 chunks, one wave per (segment, slab): see the slab kernels.  Rows
-// of one or two aligned chunks (C = 4, 8) and of C <= 3 run lane groups:
+// of one or two aligned chunks (C = 4, 8), of C <= 3, and aligned rows of up to
+// 64 chunks at the mean degrees that slabs do not suit (uses_slabs) run lane
+// groups:
 //   * LC lanes cover one edge row (LC = next power of two >= C / V).
-//   * Short segments (degree <= CAP) belong to 32-lane groups: the group
-//     issues all of its segment's loads at once into RMAX register tiles of
-//     PG = 32 / LC rows, so one memory round trip brings the whole segment in;
-//     max, sum and normalisation run on the registers and alpha is written
-//     once.
+//   * Short segments (degree <= CAP) belong to G-lane groups (G = 32, or 64
+//     when LC = 64): the group issues all of its segment's loads at once into
+//     RMAX register tiles of PG = G / LC rows, so one memory round trip brings
+//     the whole segment in; max, sum and normalisation run on the registers
+//     and alpha is written once.
 //   * Long segments (degree > CAP) belong to a whole 256-thread workgroup:
 //     up to RMAXB tiles of PB = 256 / LC rows are staged in registers (one
 //     read); longer segments stream twice (an online max/sum pass, then the
@@ -1001,7 +1003,8 @@ constexpr int kSlabWaves = 8;  // most slabs of one segment side by side in a ba
 // How a wave finds its rows: natural order through buffer views, or edge ids
 // (from `order`, or the slot itself) and 64-bit addresses, the ids kept in 32
 // bits where they fit.  Rows are read and written once and go non-temporally,
-// except (SharedViews) where slabs of 128 bytes do not fall on cache lines, so
+// except the first reading of a segment that is streamed (kKeep; C = 32, segments of
+// 90 rows among twice as many empty ones: 56 -> 46 us), and (SharedViews) where slabs of 128 bytes do not fall on cache lines, so
 // that two waves share most lines: there the default policy keeps a line until
 // its other half comes (C = 191, 991k edges: 1,364 -> 961 us; C = 256 the
 // other way round: 659 against 726 us).

@@ -327,7 +327,8 @@ class SoftmaxPlan:
 
 
 def segment_softmax_plan(offsets, n_edges: int, channels: int) -> SoftmaxPlan:
-    """Build the degree plan of ``offsets`` on its device (synchronises once; empty, and without, past 8 channels)."""
+    """Build the degree plan of ``offsets`` on its device (synchronises once, or not
+    where the kernels of these channels and this mean degree take none: the plan is then empty)."""
     nodes = _offsets(offsets, "segment softmax offsets")
     _check(int(channels) > 0, "segment softmax requires at least one channel")
     nbytes = _LIB.dpa4k_segment_softmax_plan_size(nodes)

@@ -407,7 +407,8 @@ def segment_softmax(logit, env, offsets, null_logit=None, *, order=None, check_g
     non-positive envelope carry no mass.  ``check_grouping`` is accepted for
     signature compatibility; the softmax has no ``dst`` to check against.
     The first call on an ``offsets`` tensor builds its degree plan (one host
-    synchronisation); reuse the tensor across calls.
+    synchronisation, where the kernels that the width and the mean degree
+    select use one); reuse the tensor across calls.
     """
     _validate_segment_softmax(logit, env, offsets, null_logit, order)
     require_dcu(logit, env, offsets, null_logit, order)

@@ -186,9 +186,11 @@ int dpa4k_segment_softmax_backward(const float* alpha, const float* grad_alpha,
  * channel count.  plan >= dpa4k_segment_softmax_plan_size(N) bytes of device
  * memory (8-byte aligned); *n_long and *plan_capacity (host) receive the
  * number of listed segments and the degree threshold the list was built for.
- * Synchronises (to read them back).  Only rows of 4 or 8 channels (and of
- * fewer than 4) have a plan: for any other count it is empty, both numbers are
- * 0, nothing synchronises, and the planned entry points run as the others. */
+ * Synchronises (to read them back), except where the kernels that run these
+ * channels at this mean degree (n_edges / n_nodes) take no plan: it is then
+ * empty, both numbers are 0, and the planned entry points run as the others.
+ * Rows of up to 4 and of 8 channels always have one, rows that are not a
+ * multiple of 4 or are wider than 256 never. */
 size_t dpa4k_segment_softmax_plan_size(int64_t n_nodes);
 int dpa4k_segment_softmax_plan(const int64_t* offsets, int64_t n_edges,
                                int64_t n_nodes, int64_t channels, void* plan,
