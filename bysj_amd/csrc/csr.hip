@@ -50,7 +50,6 @@
 // unique).
 #include <algorithm>
 #include <atomic>
-#include <mutex>
 
 #include "common.h"
 
@@ -1912,31 +1911,36 @@ __global__ void publish_word_kernel(const int32_t* __restrict__ word, int32_t* _
   if (threadIdx.x == 0) *host = *word;
 }
 
-// Pinned host words through which the synchronous builds read their flags.  A
-// copy into pageable memory went through the runtime's staging buffer and a
-// blit kernel: 5.9M keys 70 -> 63 us a call, 18,150 keys 42 -> 33.  One page for the process,
-// allocated by the first call and kept (its 64 words serve every device,
-// stream and thread; a call holds one from its launch to its synchronisation).
+// Pinned host words through which the synchronous builds read their flags, each
+// written by a one-word kernel.  A copy into pageable memory takes a kernel of
+// the runtime as well, and its staging buffer, which is what costs: 5.9M keys 68 ->
+// 61 us a call, 20,000 keys 39 -> 29.  One page for the process, allocated by the
+// first call and kept (its 64 words serve every device, stream and thread; a call
+// holds one from its launch to its synchronisation).
+constexpr int kHostWords = 64;
+std::atomic<uint64_t> g_host_words{~uint64_t(0)};  // those in use; only dpa4k_set_host_words changes it
+
 class HostWords {
  public:
-  // a word nobody else holds, or nullptr (no page, or more than 64 calls at once)
+  HostWords() {
+    // another thread's stream capture must not mind the allocation
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    void* page = nullptr;
+    if (hipHostMalloc(&page, kHostWords * kStride * sizeof(int32_t), hipHostMallocPortable) == hipSuccess)
+      page_ = static_cast<int32_t*>(page);
+    else
+      (void)hipGetLastError();
+    if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  // a word nobody else holds, or nullptr (no page, or more calls at once than words)
   int32_t* take() {
-    std::call_once(once_, [this] {
-      // another thread's stream capture must not mind the allocation
-      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-      const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-      void* page = nullptr;
-      if (hipHostMalloc(&page, kWords * kStride * sizeof(int32_t), hipHostMallocPortable) == hipSuccess)
-        page_ = static_cast<int32_t*>(page);
-      else
-        (void)hipGetLastError();
-      if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    });
     if (page_ == nullptr) return nullptr;
+    const uint64_t used = g_host_words.load(std::memory_order_relaxed);
     uint64_t free = free_.load(std::memory_order_relaxed);
-    while (free != 0u) {
-      const int at = __builtin_ctzll(free);
-      if (free_.compare_exchange_weak(free, free & (free - 1u), std::memory_order_acquire))
+    while ((free & used) != 0u) {
+      const int at = __builtin_ctzll(free & used);
+      if (free_.compare_exchange_weak(free, free & ~(uint64_t(1) << at), std::memory_order_acquire))
         return page_ + at * kStride;
     }
     return nullptr;
@@ -1946,20 +1950,24 @@ class HostWords {
   }
 
  private:
-  static constexpr int kWords = 64;
   static constexpr int kStride = 16;  // a cache line per word
-  std::once_flag once_;
   int32_t* page_ = nullptr;
   std::atomic<uint64_t> free_{~uint64_t(0)};
 };
 
-// Brings the flags word to the host once the stream has drained.
+// Brings the flags word to the host once the stream has drained.  A capturing
+// stream cannot be waited for: the copy refuses it, and no word is taken.
 int read_flags(const int32_t* flags, int32_t& host, hipStream_t stream) {
   static HostWords words;
-  if (int32_t* word = words.take()) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  const bool capturing = hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone;
+  if (int32_t* word = capturing ? nullptr : words.take()) {
     publish_word_kernel<<<1, 64, 0, stream>>>(flags, word);
+    if (int s = launched("publish_word_kernel")) {
+      words.give_back(word);
+      return s;
+    }
     // (a word whose kernel may still run is not given back)
-    if (int s = launched("publish_word_kernel")) return s;
     if (int s = hip_status(hipStreamSynchronize(stream), "hipStreamSynchronize")) return s;
     host = *static_cast<volatile int32_t*>(word);
     words.give_back(word);
@@ -2017,6 +2025,13 @@ int group_by_key_impl(const int64_t* keys, int64_t n_edges, int64_t n_nodes, int
 }  // namespace dpa4k
 
 using namespace dpa4k;
+
+extern "C" int dpa4k_set_host_words(int64_t words) {
+  clear_error();
+  if (words < 0 || words > kHostWords) return fail(DPA4K_EINVAL, "host words must be 0 to %d", kHostWords);
+  g_host_words.store(words == kHostWords ? ~uint64_t(0) : (uint64_t(1) << words) - 1u, std::memory_order_relaxed);
+  return DPA4K_OK;
+}
 
 extern "C" size_t dpa4k_segment_offsets_workspace_size(int64_t n_edges, int64_t n_nodes) {
   return n_nodes > 0 && n_edges >= 0 ? scratch_bytes(Plan(n_edges, n_nodes)) : 0;

@@ -91,6 +91,7 @@ PROTOTYPES: dict[str, tuple[object, list[object]]] = {
                _I64, _I64, _I64, _P]),
     "dpa4k_stream_calibrate": (_INT, [_P, _I64, _P, _I64, _P]),
     "dpa4k_set_launch_row_limit": (_INT, [_I64]),
+    "dpa4k_set_host_words": (_INT, [_I64]),
 }
 
 _LOCK = threading.Lock()

@@ -549,6 +549,12 @@ int dpa4k_stream_calibrate(const float* src, int64_t read_floats, float* dst,
  * do not depend on it.  Not meant to be changed while other threads launch. */
 int dpa4k_set_launch_row_limit(int64_t blocks);
 
+/* The synchronous CSR builds read their flags through one of 64 pinned host
+ * words; a call that finds none free copies them instead.  This lowers the
+ * words in use to `words` (0 to 64, 64 restores all) for every later call in
+ * the process, so that tests reach the copy.  Results do not depend on it. */
+int dpa4k_set_host_words(int64_t words);
+
 #ifdef __cplusplus
 }
 #endif

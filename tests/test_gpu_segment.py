@@ -142,35 +142,46 @@ def test_counting_sort_past_the_grouped_limits(edges, nodes):
     _check_grouping_against_numpy(keys, nodes, f"four-launch E={edges} N={nodes}")
 
 
-def test_grouping_flags_of_concurrent_calls():
-    """Each call reads its own flags: threads on their own streams, half of them with a key out of range."""
+@pytest.mark.parametrize("words", [64, 2, 0])
+def test_grouping_flags_of_concurrent_calls(words):
+    """Each call reads its own flags: threads on their own streams, half of them with a key out of range; with a pinned
+    word for every call, with fewer words than calls at once, and with the copy alone."""
     import threading
 
-    announce("counting sort: concurrent flags")
+    announce("counting sort: concurrent flags", words)
     good = torch.from_numpy(workloads.rng(6).integers(0, 500, size=20_000).astype(np.int64)).to(DEV)
     bad = good.clone()
     bad[777] = 500
     expected = torch.sort(good, stable=True).indices
     torch.cuda.synchronize()
-    wrong = []
+    wrong, done = [], []
 
     def calls(keys, in_range):
-        with torch.cuda.stream(torch.cuda.Stream()):
-            for _ in range(40):
-                try:
-                    order, _ = kernels.group_by_source(keys, 500)
-                    if not in_range or not torch.equal(order, expected):
-                        wrong.append(in_range)
-                except ValueError:
-                    if in_range:
-                        wrong.append(in_range)
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(40):
+                    try:
+                        order, _ = kernels.group_by_source(keys, 500)
+                        if not in_range or not torch.equal(order, expected):
+                            wrong.append(in_range)
+                    except ValueError:
+                        if in_range:
+                            wrong.append(in_range)
+                    done.append(in_range)
+        except BaseException as error:  # a thread that ends early fails the test
+            wrong.append(error)
 
-    threads = [threading.Thread(target=calls, args=((good, True) if k % 2 else (bad, False))) for k in range(8)]
-    for thread in threads:
-        thread.start()
-    for thread in threads:
-        thread.join()
-    assert not wrong
+    _lib.check(_lib.load().dpa4k_set_host_words(words))
+    try:
+        threads = [threading.Thread(target=calls, args=((good, True) if k % 2 else (bad, False))) for k in range(8)]
+        for thread in threads:
+            thread.start()
+        for thread in threads:
+            thread.join()
+    finally:
+        _lib.check(_lib.load().dpa4k_set_host_words(64))
+    assert not wrong and done.count(True) == done.count(False) == 160
+    assert _lib.load().dpa4k_set_host_words(65) == _lib.EINVAL and _lib.load().dpa4k_set_host_words(-1) == _lib.EINVAL
 
 
 def test_group_by_key_async_status_and_capture():
@@ -980,6 +991,30 @@ def test_segment_softmax_routes(channels, graph, ordered):
         edges, nodes, channels, stream))
     assert_bitwise(plain, alpha.detach(), "unplanned alpha")
     assert_bitwise(plain_null, null_alpha.detach(), "unplanned null_alpha")
+
+
+@pytest.mark.parametrize("ordered", [False, True])
+def test_segment_softmax_of_very_wide_rows(ordered):
+    """Rows past 2^20 columns address their edges with 64 bits."""
+    channels = 2**20 + 1
+    announce("softmax very wide", channels, ordered)
+    dst, offsets = _graph([3, 0, 1])
+    order = None
+    if ordered:
+        dst = torch.tensor([2, 0, 0, 0])
+        order, offsets = ref.group_by_source(dst, 3)
+    gen = torch.Generator().manual_seed(1)
+    logit, up = (torch.randn(4, channels, generator=gen) for _ in range(2))
+    env = torch.rand(4, generator=gen) + 0.1
+    x, e = logit.to(DEV).requires_grad_(True), env.to(DEV).requires_grad_(True)
+    alpha = kernels.segment_softmax(x, e, offsets.to(DEV), order=None if order is None else order.to(DEV))
+    assert_close_scaled(alpha, ref.segment_softmax_reference(logit, env, dst, offsets, None)[0], what="alpha")
+    grads = torch.autograd.grad(alpha, (x, e), up.to(DEV))
+    t_logit, t_env, _ = segment_softmax_backward_f64(up, logit, env, dst, 3)
+    assert_close_scaled(grads[0], t_logit, what="grad_logit")
+    # grad_env adds 2^20 terms in single precision: a tree over lanes and slabs, then rounds of 8 slabs one after another
+    terms = (t_logit.abs().sum(1) * 2.0 / env.double())
+    assert bool(((grads[1].cpu().double() - t_env).abs() <= 4200 * 2.0**-24 * terms).all()), "grad_env"
 
 
 @pytest.mark.parametrize("channels", [3, 8, 13, 33, 66, 257, 290])
