@@ -546,7 +546,8 @@ int scratch_for_stream(hipStream_t stream, float*& out) {
 }
 
 size_t backward_workspace_bytes(int64_t rows, int64_t width) {
-  if (rows <= 0 || width <= 0 || !fits_registers(width)) return 0;
+  if (rows <= 0 || width <= 0) return 0;
+  if (!fits_registers(width)) return round_up_256(static_cast<size_t>(width) * 4);  // not used: a size grows with the input
   return round_up_256(static_cast<size_t>(partial_blocks(rows, width)) * static_cast<size_t>(width) * 4);
 }
 
@@ -571,10 +572,10 @@ int rmsnorm_backward(const float* grad, const float* x, const float* scale, cons
     return fail(DPA4K_EINVAL, "RMSNorm backward: null pointer");
   // Rows of more than 1,024 floats, unless whole aligned chunks, have always been
   // accepted without a workspace (the header asks for one): the columns kernel takes these.
-  const size_t needed = backward_workspace_bytes(rows, width);
+  const bool wide = !fits_registers(width);
+  const size_t needed = wide ? 0 : backward_workspace_bytes(rows, width);
   const bool chunked = width % 4 == 0 && aligned16(grad) && aligned16(x) && aligned16(grad_x) && aligned16(scale);
   const bool short_workspace = !static_scratch && (workspace == nullptr || workspace_bytes < needed);
-  const bool wide = !fits_registers(width);
   const bool columns = grad_scale != nullptr && (wide || (short_workspace && width > 1024 && !chunked));
   if (columns) {  // first: grad_x may be grad or x
     rmsnorm_scale_columns_kernel<<<launch_grid((width + 31) / 32, kColumnWaves * 64), kColumnWaves * 64, 0, stream>>>(

@@ -493,8 +493,8 @@ int dpa4k_rmsnorm_forward(const float* x, const float* scale, float* y,
  *   grad_scale[w] = sum_rows grad * x * inv      (if grad_scale != NULL)
  * grad_x may be the grad or the x array.
  * grad_scale is reduced over rows in a fixed two-stage order (no atomics);
- * it needs workspace >= dpa4k_rmsnorm_backward_workspace_size(rows, W), which
- * is 0 for W > 4096.  A missing or short workspace is DPA4K_EWORKSPACE, except
+ * it needs workspace >= dpa4k_rmsnorm_backward_workspace_size(rows, W), except
+ * for W > 4096, which uses none.  A missing or short workspace is DPA4K_EWORKSPACE, except
  * for rows of more than 1024 floats that are not whole 16-byte chunks (W % 4
  * != 0, or a base off 16 bytes): grad_scale is then summed by another kernel,
  * which reads grad and x once more and rounds differently. */

@@ -92,12 +92,18 @@ def test_streamed_rows_share_no_memory(rows, width):
     workspace or none, and calls of the no-allocation form that overlap on two streams do not disturb each other."""
     library = _lib.load()
     announce("rmsnorm backward, streamed rows, two streams", rows, width)
-    assert library.dpa4k_rmsnorm_backward_workspace_size(rows, width) == 0
     cases = [_inputs(rows, width, seed=s) for s in (1, 2)]
     want = [_with_workspace(library, *case) for case in cases]
     for (grad, x, scale, _), (_, got) in zip(cases, want):
         _, truth = rmsnorm_backward_f64(grad, x, scale, 1e-6)
         assert_close_scaled(got, truth, what="grad_scale vs fp64 closed form")
+    grad, x, scale, inverse_rms = cases[0]
+    bare_x, bare_scale = torch.empty_like(x), torch.empty_like(scale)
+    _lib.check(library.dpa4k_rmsnorm_backward(grad.data_ptr(), x.data_ptr(), scale.data_ptr(), inverse_rms.data_ptr(),
+                                              bare_x.data_ptr(), bare_scale.data_ptr(), rows, width, None, 0,
+                                              torch.cuda.current_stream().cuda_stream))
+    assert_bitwise(bare_x, want[0][0], "grad_x without a workspace")
+    assert_bitwise(bare_scale, want[0][1], "grad_scale without a workspace")
     streams = [torch.cuda.Stream(DEV) for _ in cases]
     torch.cuda.synchronize()
     got = [(torch.empty_like(x), torch.empty_like(scale)) for _, x, scale, _ in cases]
