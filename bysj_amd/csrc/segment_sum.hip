@@ -358,7 +358,7 @@ __global__ __launch_bounds__(kBlock) void segment_sum_backward_wide_kernel(
   constexpr int SG = kBlock / G;
   __shared__ float partial[SG];
   const int64_t unit = block_index();
-  const int64_t segment = uniform_i64(shares == 1 ? unit : unit / shares);
+  const int64_t segment = shares == 1 ? unit : unit / shares;
   if (segment >= n_nodes) return;
   const int share = static_cast<int>(unit - segment * shares);
   const int lane = threadIdx.x % G;
@@ -484,7 +484,6 @@ int launch_staged_forward(const float* src, const int64_t* offsets, const float*
 // 68; 90 or 60 rows of 256 floats in two shares 374 -> 344; rows gathered through
 // an order 463 -> 452.  The sum of grad_node_scale keeps one workgroup.
 constexpr int64_t kShareBytes = 32768;
-constexpr int64_t kStreamedFloats = int64_t(1) << 24;
 int backward_shares(int64_t n_edges, int64_t n_nodes, int64_t channels, bool want_node) {
   if (want_node) return 1;
   const double bytes = static_cast<double>(n_edges) / static_cast<double>(n_nodes) * static_cast<double>(channels) * 4.0;
@@ -500,12 +499,14 @@ int launch_wide_backward_g(const float* grad_out, const float* src, const int64_
   constexpr int U = CPL >= 8 ? 1 : 8 / CPL;  // 8 chunks of a row set in flight per lane
   const int shares = backward_shares(n_edges, n_nodes, channels, grad_node_scale != nullptr);
   const dim3 grid = launch_grid(n_nodes * shares, kBlock);
-  // Gradient rows are stored non-temporally, and on small grids of little data the rows loaded so (config 1: 11.4 ->
-  // 10.6-10.9 us; on large ones it does not pay, config 1R: 1,846 -> 1,886-1,903 us, nor on few segments of
-  // much data, 2,604 gathered segments of 30 rows of 512: 69 against 61 us), except rows of several
+  // Gradient rows are stored non-temporally, and on small grids the rows loaded so (config 1: 11.4 -> 10.6-10.9 us;
+  // on large ones it does not pay, config 1R: 1,846 -> 1,886-1,903 us) unless they are 64 to 256 MB, which the
+  // memory-side cache may still hold (160 MB, 2,604 gathered segments of 30 rows of 512: 69 against 55 us; 1.1 GB, 3,000
+  // of 90 rows of 1,024: 416 against 432), except rows of several
   // chunks per lane that do not end on cache lines (C = 331: 419 -> 390 us forward and backward; C = 77, one
   // chunk per lane, the other way round: 402 against 424 us).
-  const bool stream_rows = n_nodes < 4096 && n_edges * channels < kStreamedFloats;  // (64 MB)
+  const double megabytes = static_cast<double>(n_edges) * static_cast<double>(channels) * 4e-6;
+  const bool stream_rows = n_nodes < 4096 && (megabytes < 64.0 || megabytes > 256.0);
   const bool shared_lines = CPL > 1 && channels % 32 != 0;
 #define DPA4K_SUM_BWD_WIDE_T(ORD, NT, NTG, TAIL)                                                         \
   segment_sum_backward_wide_kernel<G, CPL, U, ORD, NT, NTG, TAIL><<<grid, kBlock, 0, stream>>>(          \
