@@ -6,13 +6,20 @@
 //
 // The reference scatters every (edge, row, channel) product with a float
 // atomic into a zero-filled output and rescales it in a second pass.  Here
-// the edges are grouped by destination first (csr.hip) and one wave owns one
-// node: lane l owns the output chunks q = l, l + 64, ... of rows 1..R
-// (chunk = 4 channels), walks the node's edges in CSR order and accumulates
-// each element sequentially (product rounded, then added), normalising once
-// after the sum.  The node's [R, C] accumulator never leaves registers, the
-// output is written once, and the result equals the sequential fp32 chain
-// `gather -> mul -> index_add_ -> mul` bit for bit.  The forward kernels load
+// the edges are grouped by destination first (csr.hip) and one wave (or half
+// of one) owns one node, walks its edges in CSR order and accumulates each
+// element sequentially (product rounded, then added), normalising once after
+// the sum.  The node's [R, C] accumulator never leaves registers, the output
+// is written once, and the result equals the sequential fp32 chain
+// `gather -> mul -> index_add_ -> mul` bit for bit.  By the radial map
+// (slot_info):
+//   * one slot per degree, lmax <= 4, C = 32, 64 or 128 (DeepMD's):
+//     gie_forward_degrees_kernel, every row of a channel in one lane;
+//   * other maps with two to eight rows on a slot, and that map at other
+//     widths: gie_forward_shared_kernel, rows dealt to lane groups;
+//   * distinct slots, unknown maps and the rest: gie_forward_kernel, lane l on
+//     the output chunks q = l, l + 64, ... of rows 1..R (chunk = 4 channels).
+// The forward kernels load
 // the radial rows non-temporally: each is read once, and keeping them out of
 // the caches' normal replacement made the [E, 16, 64] forward 5% (fused with
 // RMSNorm 8%) faster; the backward kernels keep ordinary loads, which were
@@ -20,12 +27,16 @@
 //
 // Backward is node-parallel as well.  It recomputes the unnormalised sum for
 // the inverse-degree gradient in the same pass that reads radial/zonal for
-// the zonal/radial gradients, so each edge row is read once.  With distinct
-// radial slots (each slot feeds at most one row) lanes own (slot, chunk)
-// pairs and everything stays in registers; shared slots (several rows
-// reading one slot, e.g. one radial channel per degree l) go through a
-// one-wave kernel that stages the per-row products in LDS and sums them per
-// slot in ascending row order.
+// the zonal/radial gradients, so each edge row is read once:
+//   * distinct slots (each slot feeds at most one row):
+//     gie_backward_distinct_kernel, lanes on (slot, chunk) pairs, a node per
+//     workgroup or per wave;
+//   * one to four slots, C = 32, 64 or 128 (DeepMD's map among them):
+//     gie_backward_edge_lanes_kernel, likewise;
+//   * other maps with two to eight rows on a slot: gie_backward_shared_kernel,
+//     a wave per node, registers only;
+//   * the rest: gie_backward_general_kernel, one wave that stages the per-row
+//     products in LDS and sums them per slot in ascending row order.
 #include <type_traits>
 
 #include "common.h"
@@ -140,8 +151,9 @@ __global__ __launch_bounds__(kBlock) void gie_forward_kernel(
 // own (a slot with k rows takes ceil(k / G) groups); lane pair p = lane + 64 j
 // serves chunk p % row_chunks of group p / row_chunks.  Every radial element
 // is then loaded by one lane per group of its slot instead of once per row,
-// and the lanes' row counts stay within G of each other (DeepMD's 3 / 5 / 7
-// rows at C = 64 become 4 groups of at most 5).  Lane r < R loads zonal[e, r]
+// and the lanes' row counts stay within G of each other (3 / 5 / 7 rows on
+// three slots at C = 64 become 4 groups of at most 5; with the slots in degree
+// order that map runs gie_forward_degrees_kernel).  Lane r < R loads zonal[e, r]
 // and the lanes fetch the values of their rows with ds_bpermute.  Per output
 // element the arithmetic is gie_forward_kernel's (edges in CSR order, product
 // rounded, then added, normalised after the sum): the same output bit for
@@ -893,7 +905,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
 // Each radial element is read and each gradient written once.  Every
 // iteration loads UU wave steps' radial and zonal values before any of
 // their arithmetic, which keeps enough bytes in flight per wave.  (Measured
-// on the DeepMD map at C = 64: 8 channels per lane beat 4 (more butterfly
+// on the DeepMD map at C = 64, which runs gie_backward_edge_lanes_kernel now: 8 channels per lane beat 4 (more butterfly
 // steps) and 16 (register-bound occupancy), and the plain loop beat
 // software-pipelined forms, whose loads waited for the previous step's
 // stores: gfx9's vmcnt counts both.)  Fused multiply-adds in a fixed order:
@@ -1413,7 +1425,7 @@ int launch_general(int cpl, size_t lds_bytes, const float* grad_output, const fl
   return launched("gie_backward_general_kernel");
 }
 
-// Bits of dpa4k_gie_group's host_info that pick a kernel: bit 2 = every slot
+// Values in dpa4k_gie_group's host_info that pick a kernel: 2 = every slot
 // feeds at most one row, bits 16..23 = the most rows that read one slot.
 constexpr int32_t kSlotsDistinct = 2;
 int slot_rows(int32_t slot_info) { return (slot_info >> 16) & 0xff; }

@@ -558,8 +558,8 @@ def _gie_checks(zonal, radial, dst, radial_slot, inv_sqrt_deg):
 def gie_group(dst, radial_slot, n_nodes: int, n_radial: int):
     """Destination CSR of an unsorted ``dst``: ``(offsets, order or None, info)``.
 
-    ``order`` is None when ``dst`` is already non-decreasing; ``info`` bit 2
-    says every radial slot feeds at most one row, bit 4 that each degree l has
+    ``order`` is None when ``dst`` is already non-decreasing; ``info & 2``
+    says every radial slot feeds at most one row, ``info & 4`` that each degree l has
     one slot (l - 1) for its 2 l + 1 rows, and bits 16..23 hold the most rows
     that read one slot.  The GIE kernels below take ``info`` as
     ``slot_info`` to pick their layout.  ValueError on out-of-range ``dst`` or
