@@ -793,9 +793,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
     const float* __restrict__ inv, float* __restrict__ grad_zonal, float* __restrict__ grad_radial,
     float* __restrict__ grad_inv, int64_t n_edges, int64_t n_nodes, int64_t n_rows,
     int64_t n_radial, int64_t channels) {
-  // the row before inv, the wave's edges: split over waves in 64 bits, so that the split costs no accuracy
-  using Sum = std::conditional_t<(NW > 1), double, float>;
-  __shared__ Sum inv_sum[NW];
+  __shared__ double inv_sum[NW];
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int member = NW > 1 ? wave : 0;
   const int64_t node = NW > 1 ? block_index() : block_index() * kWaves + wave;
@@ -810,7 +808,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
   // addresses in registers.
   uint32_t col_at[CPL], zon_at[CPL], out_at[CPL], gz_at[CPL];
   fvec<V> g[CPL];
-  Sum pre[CPL][V];
+  double pre[CPL][V];  // the row before inv, the wave's edges: in 64 bits, so that no split of them costs accuracy
 #pragma unroll
   for (int j = 0; j < CPL; ++j) {
     const int64_t q = lane + 64 * j;
@@ -833,7 +831,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
       for (int i = 0; i < V; ++i) g[j].v[i] = 0.0f;
     }
 #pragma unroll
-    for (int i = 0; i < V; ++i) pre[j][i] = 0;
+    for (int i = 0; i < V; ++i) pre[j][i] = 0.0;
   }
   const int64_t radial_bytes = edge_stride * 4, zonal_bytes = n_rows * 4;
 
@@ -863,8 +861,7 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
       fvec<V> out;
 #pragma unroll
       for (int i = 0; i < V; ++i) {
-        if constexpr (NW > 1) pre[j][i] = __builtin_fma(static_cast<double>(z[j]), static_cast<double>(x[j].v[i]), pre[j][i]);
-        else pre[j][i] = pre[j][i] + z[j] * x[j].v[i];
+        pre[j][i] = __builtin_fma(static_cast<double>(z[j]), static_cast<double>(x[j].v[i]), pre[j][i]);
         const float h = g[j].v[i] * sc;
         dot = dot + h * x[j].v[i];
         out.v[i] = h * z[j];
@@ -875,21 +872,18 @@ __global__ __launch_bounds__(kBlock) void gie_backward_distinct_kernel(
     }
   }
   if (grad_inv != nullptr) {
-    Sum total = 0;
+    double total = 0.0;
 #pragma unroll
     for (int j = 0; j < CPL; ++j)
 #pragma unroll
-      for (int i = 0; i < V; ++i) {
-        if constexpr (NW > 1) total = __builtin_fma(static_cast<double>(g[j].v[i]), pre[j][i], total);
-        else total = total + g[j].v[i] * pre[j][i];
-      }
+      for (int i = 0; i < V; ++i) total = __builtin_fma(static_cast<double>(g[j].v[i]), pre[j][i], total);
     total = group_sum<64>(total);
     if constexpr (NW > 1) {
       if (lane == 0) inv_sum[wave] = total;
       __syncthreads();
       if (threadIdx.x == 0) grad_inv[node] = static_cast<float>(node_total(inv_sum));
     } else {
-      if (lane == 0) grad_inv[node] = total;
+      if (lane == 0) grad_inv[node] = static_cast<float>(total);
     }
   }
 }

@@ -563,3 +563,24 @@ def test_gie_wave_per_node(slots, n_radial, channels, shuffle):
     truth = zonal_scatter_backward_f64(up, *inputs)
     for label, actual, wanted, exact in zip(("zonal", "radial", "inverse"), grads, oracle, truth):
         assert_gradient(actual, wanted, exact, f"grad {label}")
+
+
+@pytest.mark.parametrize("degree", [2, 14])
+def test_gie_distinct_inverse_gradient_in_64_bits(degree):
+    """Distinct slots sum the gradient of `inverse` in 64 bits, with a wave or a workgroup per node: the float32 result is
+    within half a unit of its last place, and what rounding n terms in 64 bits adds, of the exact sum."""
+    n_rows, channels, nodes = 8, 32, 5000
+    announce("gie distinct inverse gradient", degree)
+    generator = torch.Generator().manual_seed(degree)
+    dst = torch.repeat_interleave(torch.arange(nodes), degree)
+    zonal = torch.randn((dst.numel(), n_rows), generator=generator)
+    radial = torch.randn((dst.numel(), n_rows, channels), generator=generator)
+    inverse = torch.rand(nodes, generator=generator) + 0.5
+    up = torch.randn((nodes, n_rows + 1, channels), generator=generator)
+    z, r, d, k, inv = _to((zonal, radial, dst, torch.arange(n_rows), inverse))
+    inv.requires_grad_(True)
+    actual = torch.autograd.grad(kernels.zonal_scatter(z, r, d, k, inv), inv, up.to(DEV))[0].cpu().double()
+    terms = zonal.double()[:, :, None] * radial.double() * up.double()[dst, 1:]
+    exact, magnitude = (t.reshape(nodes, -1).sum(1) for t in (terms, terms.abs()))
+    bound = 2.0**-24 * exact.abs() + (degree * n_rows * channels) * 2.0**-52 * magnitude
+    assert bool(((actual - exact).abs() <= bound).all())
