@@ -764,7 +764,7 @@ static_assert(kNodeWaves == kWaves, "a workgroup holds one node or a wave per no
 // nodes are too few to fill the chip with a wave each.  Below, most of the waves only stage rows and wait at the
 // barrier behind grad_inv.  DeepMD's map at lmax 3, 600k edges, a workgroup and a wave per node, us: C = 64 degree 8 559 /
 // 307, 16 313 / 223, 24 235 / 221, 48 192 / 232, without grad_inv 24 203 / 221; C = 32 16 283 / 130, 24 209 / 117, 48 111 /
-// 118; C = 128 8 720 / 574, 24 380 / 443.  Distinct slots, C = 64, 200k edges: 2 687 / 376, 16 296 / 333.  1,000 nodes of 20
+// 118; C = 128 8 720 / 574, 24 380 / 443.  Distinct slots, C = 64, 200k edges: 2 687 / 355, 16 296 / 333.  1,000 nodes of 20
 // edges, C = 64: 10 / 16.
 bool split_nodes(int64_t n_edges, int64_t n_nodes, double enough, double some) {
   const double degree = static_cast<double>(n_edges) / static_cast<double>(n_nodes);
@@ -1355,7 +1355,11 @@ int launch_distinct(int cpl, const float* grad_output, const float* zonal, const
                     const float* inv, float* grad_zonal, float* grad_radial, float* grad_inv,
                     int64_t n_edges, int64_t n_nodes, int64_t n_rows, int64_t n_radial,
                     int64_t channels, hipStream_t stream) {
-  const bool split = split_nodes(n_edges, n_nodes, 12.0, 4.0);
+  // The line moves with the chunks a lane holds, which every wave of a node loads of its upstream and keeps sums of.  A
+  // workgroup and a wave per node, 200k edges, us: cpl 1 (lmax 1, C = 64) degree 6 54 / 55, 10 49 / 53; cpl 2 (lmax 3,
+  // C = 32) degree 2 261 / 187, 4 158 / 169, 5 145 / 169; cpl 4 (lmax 3, C = 64) degree 6 328 / 333, 10 292 / 332,
+  // (lmax 4, C = 32) degree 6 323 / 269, 8 279 / 271, 10 255 / 269; cpl 8 (lmax 3, C = 128) degree 8 739 / 648, 10 665 / 654.
+  const bool split = split_nodes(n_edges, n_nodes, cpl == 1 ? 6.0 : cpl == 2 ? 4.0 : cpl == 4 ? 8.0 : 10.0, 4.0);
   const dim3 grid = node_grid(n_nodes, split);
 #define DPA4K_GIE_DIST_NW(C, NW)                                                              \
   gie_backward_distinct_kernel<V, C, RC, NW, kOrdered><<<grid, kBlock, 0, stream>>>(          \
